@@ -106,79 +106,183 @@ __global__ void __launch_bounds__(kConvThreads)
     }
 }
 
-// LDS-tiled form for z-columns of at most 64 cells (nz a multiple of 16): a
-// block of four waves computes a 2 x 2 group of whole z-columns, one per
-// wave.  The 4 x 4 input columns around them (with one cell of z halo) are
-// staged in LDS once, 16 bytes (8 channels) per slot with the slot index
-// swizzled by the cell's low bits so that the 16 lanes of an operand read
-// spread over the banks; every tap's A operands then come from LDS.
-constexpr int kColumnTile = 2, kStageCols = (kColumnTile + 2) * (kColumnTile + 2), kMaxColumn = 64;
-template <int Epi>
-__global__ void __launch_bounds__(kConvThreads)
-    k_conv3d_columns(int nx, int ny, int nz, const uint16_t* __restrict__ in, const uint16_t* __restrict__ w,
-                     const float* __restrict__ bias, const uint16_t* __restrict__ mask, uint16_t* __restrict__ out,
-                     float* __restrict__ out_f32) {
-  __shared__ uint4 xs[kStageCols][kMaxColumn + 2][4];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int row = lane & 15, group = lane >> 4;
-  const int tiles_j = (ny + kColumnTile - 1) / kColumnTile;
-  const int i0 = (int)(blockIdx.x / tiles_j) * kColumnTile, j0 = (int)(blockIdx.x % tiles_j) * kColumnTile;
-  const int depth = nz + 2, per_col = depth * 4;
-  for (int e = threadIdx.x; e < kStageCols * per_col; e += blockDim.x) {
-    const int col = e / per_col, rem = e - col * per_col, cell = rem >> 2, chunk = rem & 3;
-    const int i = i0 - 1 + col / 4, j = j0 - 1 + col % 4, k = cell - 1;
-    uint4 v = make_uint4(0u, 0u, 0u, 0u);
-    if (i >= 0 && i < nx && j >= 0 && j < ny && k >= 0 && k < nz)
-      v = *reinterpret_cast<const uint4*>(in + (((long)i * ny + j) * nz + k) * kC + chunk * 8);
-    xs[col][cell][chunk ^ (cell & 3)] = v;
+// The form for z-columns of 16, 32, 48 or 64 cells.  A product of 16 cells x
+// 16 output channels over one tap's 32 input channels is one
+// v_mfma_f32_16x16x32_bf16, 16 cycles of a SIMD's matrix core, and needs 1 KB
+// an operand: with both operands read from LDS four SIMDs ask for four times
+// what it delivers.  So a wave keeps its 16 channels' weights of all 27 taps
+// in registers (108), and the block sweeps along x with three output slabs in
+// accumulators: a cell operand read once from LDS (own slab s, shift dj, dk)
+// feeds the outputs of slabs s - 1, s and s + 1.  The next slab travels from
+// memory to registers meanwhile and into the second LDS buffer after; one
+// barrier a slab.
+//   - The weights are operand A (rows: output channels) and the cells operand
+//     B, so a lane ends up with 4 consecutive channels of one cell (8 bytes).
+//   - Eight waves: two halves of the channels times four groups of T tiles of
+//     16 cells, over kSweepCols columns of y and `per` slabs of x.
+//   - LDS holds 16-byte pieces (8 channels); piece c of cell m sits at
+//     c ^ (m / 4 % 4), so that 16 consecutive cells' pieces cover all banks.
+// A wave with all 32 channels (v_mfma_f32_32x32x16, 216 weight registers, one
+// wave a SIMD) left the compiler no registers to read ahead: 67 us at
+// 128x64x64 against 35 us here, and 79 us for 2 x 2 staged columns a block
+// with the weights read from memory for every tap (masked form: 101 to 40 us).
+//
+// Two floats as packed BF16, rounded to nearest even.
+__device__ __forceinline__ uint32_t pack2(float lo, float hi) {
+  typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+  return __builtin_bit_cast(uint32_t, bf16x2{(__bf16)lo, (__bf16)hi});
+}
+// `value` where the packed BF16 pair `m` is positive, else zero.
+__device__ __forceinline__ uint32_t keep_positive(uint32_t value, uint32_t m) {
+  const uint32_t lo = ((m & 0xffffu) - 1u) < 0x7f80u ? 0xffffu : 0u;
+  const uint32_t hi = ((m >> 16) - 1u) < 0x7f80u ? 0xffff0000u : 0u;
+  return value & (lo | hi);
+}
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+
+constexpr int kMaxColumn = 64;
+constexpr int kSweepThreads = 512, kSweepCols = 4;
+constexpr int kSweepColumn = (kMaxColumn + 2) * 4, kSweepSlab = (kSweepCols + 2) * kSweepColumn;
+template <int Epi, int T>
+__global__ void __launch_bounds__(kSweepThreads, 2)
+    k_conv3d_sweep(int nx, int ny, int per, const uint16_t* __restrict__ in, const uint16_t* __restrict__ w,
+                   const float* __restrict__ bias, const uint16_t* __restrict__ mask, uint16_t* __restrict__ out,
+                   float* __restrict__ out_f32) {
+  constexpr int nz = 16 * T;  // four columns of nz cells are 4 T tiles, T a wave
+  constexpr int kPieces = (kSweepCols + 2) * nz * 4;
+  constexpr int kFetch = (kPieces + kSweepThreads - 1) / kSweepThreads;  // 16-byte pieces a thread stages
+  __shared__ u32x4 xs[2][kSweepSlab];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, row = lane & 15, group = lane >> 4;
+  const int channels = (wave & 1) * 16, tile0 = (wave >> 1) * T;
+  const int tiles_j = (ny + kSweepCols - 1) / kSweepCols;
+  const int j0 = (int)(blockIdx.x % tiles_j) * kSweepCols, x0 = (int)(blockIdx.x / tiles_j) * per;
+  const int x1 = min(nx, x0 + per);
+  for (int e = threadIdx.x; e < 2 * kSweepSlab; e += kSweepThreads) (&xs[0][0])[e] = u32x4{0u, 0u, 0u, 0u};
+  bf16x8 wr[kTaps];
+#pragma unroll
+  for (int t = 0; t < kTaps; ++t)
+    wr[t] = *reinterpret_cast<const bf16x8*>(w + ((long)t * kC + channels + row) * kC + 8 * group);
+  float bias_r[4];
+#pragma unroll
+  for (int r = 0; r < 4; ++r) bias_r[r] = Epi == ICYC_RELU_BF16 ? bias[channels + 4 * group + r] : 0.0f;
+  // Staging: piece e % 4 of cell e / 4 of the slab's columns; a thread
+  // without a piece reads the slab's first and stores none.
+  int src[kFetch], dst[kFetch];
+#pragma unroll
+  for (int f = 0; f < kFetch; ++f) {
+    const int e = threadIdx.x + f * kSweepThreads, col = e / (nz * 4), k = e / 4 % nz, c = e % 4, j = j0 - 1 + col;
+    const bool mine = e < kPieces && j >= 0 && j < ny;
+    src[f] = mine ? (j * nz + k) * 4 + c : 0;
+    dst[f] = mine ? col * kSweepColumn + (k + 1) * 4 + (c ^ (((k + 1) >> 2) & 3)) : -1;
   }
-  __syncthreads();
-  const int wi = wave >> 1, wj = wave & 1, i = i0 + wi, j = j0 + wj;
-  if (i >= nx || j >= ny) return;
-  const int mtiles = nz / 16;
-  constexpr int kTiles = Epi == ICYC_LINEAR_F32 ? 1 : 2;  // one output: only channels 0..15 are formed
-  floatx4 acc[4][2];
+  u32x4 fetched[kFetch];
+  auto fetch = [&](int s) __attribute__((always_inline)) {
+    const u32x4* slab = reinterpret_cast<const u32x4*>(in) + (long)s * ny * nz * 4;
 #pragma unroll
-  for (int mt = 0; mt < 4; ++mt) acc[mt][0] = acc[mt][1] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
-  for (int t = 0; t < kTaps; ++t) {
-    const int di = t / 9 - 1, dj = (t / 3) % 3 - 1, dk = t % 3 - 1;
-    const uint4* wt = reinterpret_cast<const uint4*>(w + (long)t * kC * kC);
-    const bf16x8 b0 = as_bf16x8(wt[row * 4 + group]);
-    const bf16x8 b1 = kTiles == 2 ? as_bf16x8(wt[(16 + row) * 4 + group]) : b0;
-    const int col = (wi + 1 + di) * 4 + (wj + 1 + dj);
+    for (int f = 0; f < kFetch; ++f) fetched[f] = slab[src[f]];
+  };
+  auto stage = [&](u32x4* buffer) __attribute__((always_inline)) {
 #pragma unroll
-    for (int mt = 0; mt < 4; ++mt) {
-      if (mt < mtiles) {
-        const int cell = mt * 16 + row + 1 + dk;
-        const bf16x8 a = as_bf16x8(xs[col][cell][group ^ (cell & 3)]);
-        acc[mt][0] = mfma(a, b0, acc[mt][0]);
-        if (kTiles == 2) acc[mt][1] = mfma(a, b1, acc[mt][1]);
-      }
+    for (int f = 0; f < kFetch; ++f)
+      if (dst[f] >= 0) buffer[dst[f]] = fetched[f];
+  };
+  // This lane's cell of each tile, and where its operand pieces start.
+  int at[T][3], cell_j[T], cell_k[T];
+#pragma unroll
+  for (int tl = 0; tl < T; ++tl) {
+    const int m = tile0 + tl;
+    cell_j[tl] = m / T;
+    cell_k[tl] = m % T * 16 + row;
+#pragma unroll
+    for (int dk = 0; dk < 3; ++dk) {
+      const int cell = cell_k[tl] + dk;
+      at[tl][dk] = cell_j[tl] * kSweepColumn + cell * 4 + (group ^ ((cell >> 2) & 3));
     }
   }
-  const long base = ((long)i * ny + j) * nz;
+  __syncthreads();
+  if (x0 > 0) {
+    fetch(x0 - 1);
+    stage(xs[0]);
+  }
+  int current = 0;
+  floatx4 acc[3][T];
+  // Slab s into the outputs of slabs s - 1 (accumulators P), s (C) and s + 1
+  // (N, cleared here); then the finished outputs of slab s - 1.
+  auto step = [&](int s, floatx4(&P)[T], floatx4(&C)[T], floatx4(&N)[T]) __attribute__((always_inline)) {
+    __syncthreads();
+    const bool more = s + 1 <= x1 && s + 1 < nx;
+    if (more) fetch(s + 1);
 #pragma unroll
-  for (int mt = 0; mt < 4; ++mt) {
-    if (mt >= mtiles) continue;
+    for (int tl = 0; tl < T; ++tl) N[tl] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+    const bool do_p = s - 1 >= x0, do_c = s >= x0 && s < x1, do_n = s + 1 < x1;
+    if (s >= 0 && s < nx) {
+      const u32x4* buffer = xs[current];
+      if (do_p && do_c && do_n) {
 #pragma unroll
-    for (int nt = 0; nt < kTiles; ++nt) {
-      const int co = nt * 16 + row;
+        for (int dj = 0; dj < 3; ++dj)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const long cell = base + mt * 16 + group * 4 + r;
-        const float x = acc[mt][nt][r];
-        if (Epi == ICYC_RELU_BF16) {
-          out[cell * kC + co] = f2bf(fmaxf(0.0f, x + bias[co]));
-        } else if (Epi == ICYC_LINEAR_F32) {
-          if (co == 0) out_f32[cell] = x + bias[0];
+          for (int dk = 0; dk < 3; ++dk) {
+            bf16x8 b[T];
+#pragma unroll
+            for (int tl = 0; tl < T; ++tl)
+              b[tl] = __builtin_bit_cast(bf16x8, buffer[at[tl][dk] + dj * kSweepColumn]);
+#pragma unroll
+            for (int tl = 0; tl < T; ++tl) {
+              P[tl] = mfma(wr[18 + 3 * dj + dk], b[tl], P[tl]);
+              C[tl] = mfma(wr[9 + 3 * dj + dk], b[tl], C[tl]);
+              N[tl] = mfma(wr[3 * dj + dk], b[tl], N[tl]);
+            }
+          }
+      } else {  // the first and last slabs: one or two of the three
+        auto plane = [&](int first, floatx4(&A)[T]) __attribute__((always_inline)) {
+#pragma unroll
+          for (int e = 0; e < 9; ++e)
+#pragma unroll
+            for (int tl = 0; tl < T; ++tl)
+              A[tl] = mfma(wr[first + e],
+                           __builtin_bit_cast(bf16x8, buffer[at[tl][e % 3] + e / 3 * kSweepColumn]), A[tl]);
+        };
+        if (do_p) plane(18, P);
+        if (do_c) plane(9, C);
+        if (do_n) plane(0, N);
+      }
+    }
+    if (do_p) {
+#pragma unroll
+      for (int tl = 0; tl < T; ++tl) {
+        const int j = j0 + cell_j[tl];
+        if (j >= ny) continue;
+        const long cell = ((long)(s - 1) * ny + j) * nz + cell_k[tl];
+        if (Epi == ICYC_LINEAR_F32) {
+          if (channels + group == 0) out_f32[cell] = P[tl][0] + bias[0];
         } else {
-          out[cell * kC + co] = bf2f(mask[cell * kC + co]) > 0.0f ? f2bf(x) : (uint16_t)0;
+          float v[4];
+#pragma unroll
+          for (int r = 0; r < 4; ++r) v[r] = Epi == ICYC_RELU_BF16 ? fmaxf(0.0f, P[tl][r] + bias_r[r]) : P[tl][r];
+          uint2 packed = make_uint2(pack2(v[0], v[1]), pack2(v[2], v[3]));
+          const long at_c = cell * kC + channels + 4 * group;
+          if (Epi == ICYC_MASKED_BF16) {
+            const uint2 m = *reinterpret_cast<const uint2*>(mask + at_c);
+            packed = make_uint2(keep_positive(packed.x, m.x), keep_positive(packed.y, m.y));
+          }
+          *reinterpret_cast<uint2*>(out + at_c) = packed;
         }
       }
     }
+    current ^= 1;
+    if (more) stage(xs[current]);
+  };
+  for (int s = x0 - 1;;) {
+    step(s, acc[0], acc[1], acc[2]);
+    if (++s > x1) break;
+    step(s, acc[1], acc[2], acc[0]);
+    if (++s > x1) break;
+    step(s, acc[2], acc[0], acc[1]);
+    if (++s > x1) break;
   }
 }
 
+constexpr int kColumnTile = 2, kStageCols = (kColumnTile + 2) * (kColumnTile + 2);
 // The first layer's form: its input has 8 real channels (the features), so
 // one MFMA takes four taps' 8 channels as its 32-deep K (lane group g: tap
 // 4m + g), 7 MFMAs per output tile instead of 27 over zero-padded channels;
@@ -490,6 +594,23 @@ int status() {
 }
 bool valid_grid(int nx, int ny, int nz) { return nx > 0 && ny > 0 && nz > 0 && (long)nx * ny * nz < (1L << 31); }
 unsigned blocks_of(long count, int threads) { return (unsigned)((count + threads - 1) / threads); }
+// Slabs a sweep block owns: as many as leave one block for each of the 256
+// CUs (a block fills a CU: its waves hold 512 registers), at least one.
+int sweep_slabs(int nx, int tiles_j) {
+  const int chunks = tiles_j >= 256 ? 1 : 256 / tiles_j;
+  return (nx + chunks - 1) / chunks;
+}
+template <int Epi>
+void launch_sweep(int nx, int ny, int nz, const uint16_t* in, const uint16_t* w, const float* bias,
+                  const uint16_t* mask, uint16_t* out, float* out_f32, hipStream_t s) {
+  const int tiles_j = (ny + kSweepCols - 1) / kSweepCols, per = sweep_slabs(nx, tiles_j);
+  const unsigned blocks = (unsigned)(tiles_j * ((nx + per - 1) / per));
+  auto kernel = nz == 16   ? k_conv3d_sweep<Epi, 1>
+                : nz == 32 ? k_conv3d_sweep<Epi, 2>
+                : nz == 48 ? k_conv3d_sweep<Epi, 3>
+                           : k_conv3d_sweep<Epi, 4>;
+  kernel<<<blocks, kSweepThreads, 0, s>>>(nx, ny, per, in, w, bias, mask, out, out_f32);
+}
 int wgrad_blocks(int nx, int ny) { return nx * ny < kMaxGradBlocks ? nx * ny : kMaxGradBlocks; }
 
 }  // namespace icyc
@@ -503,22 +624,18 @@ int icyc_conv3d(int32_t nx, int32_t ny, int32_t nz, const uint16_t* in, const ui
   if (!valid_grid(nx, ny, nz) || !in || !weights) return ICYC_ERR_ARGUMENT;
   hipStream_t s = (hipStream_t)stream;
   if (nz % 16 == 0 && nz <= kMaxColumn) {
-    const unsigned tiles = (unsigned)(((nx + kColumnTile - 1) / kColumnTile) * ((ny + kColumnTile - 1) / kColumnTile));
     switch (epilogue) {
       case ICYC_RELU_BF16:
         if (!bias || !out_bf16) return ICYC_ERR_ARGUMENT;
-        k_conv3d_columns<ICYC_RELU_BF16><<<tiles, kConvThreads, 0, s>>>(nx, ny, nz, in, weights, bias, nullptr,
-                                                                       out_bf16, nullptr);
+        launch_sweep<ICYC_RELU_BF16>(nx, ny, nz, in, weights, bias, nullptr, out_bf16, nullptr, s);
         break;
       case ICYC_LINEAR_F32:
         if (!bias || !out_f32) return ICYC_ERR_ARGUMENT;
-        k_conv3d_columns<ICYC_LINEAR_F32><<<tiles, kConvThreads, 0, s>>>(nx, ny, nz, in, weights, bias, nullptr,
-                                                                        nullptr, out_f32);
+        launch_sweep<ICYC_LINEAR_F32>(nx, ny, nz, in, weights, bias, nullptr, nullptr, out_f32, s);
         break;
       case ICYC_MASKED_BF16:
         if (!mask_act || !out_bf16) return ICYC_ERR_ARGUMENT;
-        k_conv3d_columns<ICYC_MASKED_BF16><<<tiles, kConvThreads, 0, s>>>(nx, ny, nz, in, weights, nullptr,
-                                                                         mask_act, out_bf16, nullptr);
+        launch_sweep<ICYC_MASKED_BF16>(nx, ny, nz, in, weights, nullptr, mask_act, out_bf16, nullptr, s);
         break;
       default:
         return ICYC_ERR_ARGUMENT;

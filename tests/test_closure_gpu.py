@@ -285,3 +285,14 @@ def test_weight_gradient_at_closure_grid():
     scale = np.abs(dw).max()
     assert np.abs(got[:co.TAPS * co.C * co.C] - dw.ravel()).max() <= 1e-5 * scale
     assert np.abs(got[co.TAPS * co.C * co.C:] - db).max() <= 1e-5 * max(np.abs(db).max(), 1.0)
+
+
+# Column depths and widths where the x sweep's tiles and chunks end unevenly:
+# every depth, y extents that are no multiple of its 4 columns, one slab, and
+# more slabs than one a block (with a shorter last chunk).
+SWEEP_SHAPES = [(1, 1, 16), (1, 5, 48), (4, 7, 48), (3, 9, 64), (70, 17, 16), (37, 30, 32)]
+
+
+@pytest.mark.parametrize("shape", SWEEP_SHAPES)
+def test_conv_sweep_edges(shape):
+    test_conv_forward_epilogues(shape)
