@@ -354,105 +354,211 @@ __global__ void __launch_bounds__(kConvThreads)
 }
 
 // ----------------------------------------------------------- weight grad
-// One block per group of z-columns (i, j): the input's 3x3 neighbour
-// columns (transposed to [channel][k]) and three k-shifted copies of the
-// output gradient ([channel][k]) are staged in LDS, so both MFMA operands are
-// 16-byte LDS reads: D[co][ci] += sum_k dout[k - dk][co] * in_col(di, dj)[k][ci].
-// Wave w accumulates taps w, w + 4, ... (at most 7 taps x 32 x 32 in registers).
-constexpr int kGradThreads = 256;
-constexpr int kColumn = 64;          // cells of a staged z-column (nz <= 64)
-constexpr int kPitch = kColumn + 8;  // padded LDS row (breaks 128-byte bank strides)
-constexpr int kTapsPerWave = 7;
-constexpr int kMaxGradBlocks = 512;
+// dW[t][co][ci] = sum over cells of dout[x][co] in[x + off(t)][ci]: 27
+// products with the cells as the reduction, so both operands need 8
+// consecutive cells of one channel in a lane.  ds_read_b64_tr_b16 reads them
+// so from channels-last rows: in a group of 16 lanes lane l points at row
+// l / 4, channels 4 (l % 4), and gets 4 rows of channel l.  Nothing is
+// transposed or shifted on the way into LDS.
+//   - A block sweeps along x over two columns of y (one for each half of its
+//     eight waves).  An input operand (slab s, shift dj, dk) is read once and
+//     multiplied with the output gradient's rows s - 1, s and s + 1, whose
+//     operands stay in registers from slab to slab: 13 KB read from LDS for
+//     27 products of 32 cycles (v_mfma_f32_32x32x16_bf16), where one read a
+//     product and operand would ask for twice what LDS delivers.
+//   - A wave holds the sums of the 9 taps of three (dj, dk) pairs (144
+//     registers).  Nine pairs over four waves: two each, and the ninth pair's
+//     16-cell chunks spread over the waves.
+//   - At the end the two halves add up through LDS, so 256 blocks write one
+//     partial each (28 MB at 128x64x64, half of one a column group).
+// A block that staged each column's nine neighbours transposed, element by
+// element, took 109 us a layer at 128x64x64; 40 us now, and the fold of half as
+// many partials 7 us instead of 12.
+typedef float floatx16 __attribute__((ext_vector_type(16)));
+__device__ __forceinline__ floatx16 mfma32(bf16x8 a, bf16x8 b, floatx16 c) {
+  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
+}
+typedef short shortx4 __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) shortx4* lds_shortx4;
+// 16 rows (cells) of 32 channels from `rows`, as the operand of one product:
+// lane l gets channel l % 32 of rows 8 (l / 32) + 0..7.
+__device__ __forceinline__ bf16x8 column_operand(const char* rows, int lane_offset) {
+  typedef short shortx8 __attribute__((ext_vector_type(8)));
+  char* at = const_cast<char*>(rows) + lane_offset;
+  const shortx4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_shortx4)at);
+  const shortx4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_shortx4)(at + 4 * kC * 2));
+  return __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+}
+constexpr int kGradThreads = 512, kGradCols = 2;
+constexpr int kGradRow = kC * 2, kGradColumn = (kMaxColumn + 2) * kGradRow;  // bytes; one cell of halo at each end
+constexpr int kGradBuffer = (kGradCols + 2 + kGradCols) * kGradColumn;       // input columns, then gradient columns
+constexpr int kGradTaps = 24;  // taps of the eight pairs that one wave of each half holds alone
+constexpr int kGradShared = kGradTaps * kC * kC * 4;
+static_assert(2 * kGradBuffer <= kGradShared && 8 * 3 * kC * kC * 4 <= kGradShared, "shared buffer too small");
 
-__global__ void __launch_bounds__(kGradThreads)
-    k_conv3d_wgrad(int nx, int ny, int nz, const uint16_t* __restrict__ in, const uint16_t* __restrict__ dout,
+template <int T>
+__global__ void __launch_bounds__(kGradThreads, 2)
+    k_conv3d_wgrad(int nx, int ny, int per, const uint16_t* __restrict__ in, const uint16_t* __restrict__ dout,
                    float* __restrict__ partials) {
-  __shared__ __attribute__((aligned(16))) uint16_t xs[9][kC][kPitch];
-  __shared__ __attribute__((aligned(16))) uint16_t ds[3][kC][kPitch];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int row = lane & 15, group = lane >> 4;
-  const int chunks = (nz + 31) / 32;
-  floatx4 acc[kTapsPerWave][2][2];
+  constexpr int nz = 16 * T;
+  constexpr int kIn = (kGradCols + 2) * nz * 4, kOut = kGradCols * nz * 4;  // 16-byte pieces of a slab and of a row
+  constexpr int kFetch = (kIn + kGradThreads - 1) / kGradThreads;
+  static_assert(kOut <= kGradThreads, "one gradient piece a thread");
+  __shared__ __attribute__((aligned(16))) char shared[kGradShared];
+  __shared__ float bias_part[kGradThreads / 64][kC];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, half = wave >> 2, part = wave & 3;
+  const int tiles_j = (ny + kGradCols - 1) / kGradCols;
+  const int j0 = (int)(blockIdx.x % tiles_j) * kGradCols, x0 = (int)(blockIdx.x / tiles_j) * per;
+  const int x1 = min(nx, x0 + per);
+  for (int e = tid; e < 2 * kGradBuffer / 16; e += kGradThreads)
+    reinterpret_cast<u32x4*>(shared)[e] = u32x4{0u, 0u, 0u, 0u};
+  // Staging: pieces as in the sweep (a thread without one reads the first
+  // piece of the slab and stores none).
+  int src[kFetch], dst[kFetch];
 #pragma unroll
-  for (int tl = 0; tl < kTapsPerWave; ++tl)
-#pragma unroll
-    for (int a = 0; a < 2; ++a) acc[tl][a][0] = acc[tl][a][1] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
-  float bias_acc = 0.0f;
-  const int cell = tid >> 2, quarter = tid & 3;  // staging: one cell's 8 channels per thread
-  for (int column = blockIdx.x; column < nx * ny; column += gridDim.x) {
-    const int i = column / ny, j = column - i * ny;
-    // the shifted gradient copies start from zero (k - dk outside the column)
-    for (int e = tid; e < 3 * kC * kPitch / 8; e += kGradThreads)
-      reinterpret_cast<uint4*>(&ds[0][0][0])[e] = make_uint4(0u, 0u, 0u, 0u);
-    __syncthreads();
-#pragma unroll 1
-    for (int rr = 0; rr < 9; ++rr) {
-      const int ii = i + rr / 3 - 1, jj = j + rr % 3 - 1;
-      uint4 v = make_uint4(0u, 0u, 0u, 0u);
-      if (cell < nz && ii >= 0 && ii < nx && jj >= 0 && jj < ny)
-        v = *reinterpret_cast<const uint4*>(in + (((long)ii * ny + jj) * nz + cell) * kC + quarter * 8);
-      const uint16_t* h = reinterpret_cast<const uint16_t*>(&v);
-#pragma unroll
-      for (int e = 0; e < 8; ++e) xs[rr][quarter * 8 + e][cell] = h[e];
-    }
-    {
-      uint4 v = make_uint4(0u, 0u, 0u, 0u);
-      if (cell < nz) v = *reinterpret_cast<const uint4*>(dout + ((long)column * nz + cell) * kC + quarter * 8);
-      const uint16_t* h = reinterpret_cast<const uint16_t*>(&v);
-#pragma unroll
-      for (int s = 0; s < 3; ++s) {
-        const int k = cell + s - 1;  // ds[s][.][k] = dout[k - (s - 1)]
-        if (cell < nz && k >= 0 && k < kColumn)
-#pragma unroll
-          for (int e = 0; e < 8; ++e) ds[s][quarter * 8 + e][k] = h[e];
-      }
-    }
-    __syncthreads();
-    if (tid < kC)
-      for (int k = 0; k < nz; ++k) bias_acc += bf2f(ds[1][tid][k]);
-#pragma unroll
-    for (int tl = 0; tl < kTapsPerWave; ++tl) {
-      const int t = wave + 4 * tl;
-      if (t >= kTaps) continue;
-      const int rr = (t / 9) * 3 + (t / 3) % 3, s = t % 3;
-      for (int c = 0; c < chunks; ++c) {
-        const int k0 = c * 32 + group * 8;
-        const bf16x8 a0 = as_bf16x8(*reinterpret_cast<const uint4*>(&ds[s][row][k0]));
-        const bf16x8 a1 = as_bf16x8(*reinterpret_cast<const uint4*>(&ds[s][16 + row][k0]));
-        const bf16x8 b0 = as_bf16x8(*reinterpret_cast<const uint4*>(&xs[rr][row][k0]));
-        const bf16x8 b1 = as_bf16x8(*reinterpret_cast<const uint4*>(&xs[rr][16 + row][k0]));
-        acc[tl][0][0] = mfma(a0, b0, acc[tl][0][0]);
-        acc[tl][0][1] = mfma(a0, b1, acc[tl][0][1]);
-        acc[tl][1][0] = mfma(a1, b0, acc[tl][1][0]);
-        acc[tl][1][1] = mfma(a1, b1, acc[tl][1][1]);
-      }
-    }
-    __syncthreads();
+  for (int f = 0; f < kFetch; ++f) {
+    const int e = tid + f * kGradThreads, col = e / (nz * 4), k = e / 4 % nz, c = e % 4, j = j0 - 1 + col;
+    const bool mine = e < kIn && j >= 0 && j < ny;
+    src[f] = mine ? (j * nz + k) * 4 + c : 0;
+    dst[f] = mine ? col * kGradColumn + (k + 1) * kGradRow + c * 16 : -1;
   }
-  float* part = partials + (long)blockIdx.x * kLayer;
+  int out_src = 0, out_dst = -1;
+  {
+    const int col = tid / (nz * 4), k = tid / 4 % nz, c = tid % 4, j = j0 + col;
+    if (tid < kOut && j < ny) {
+      out_src = (j * nz + k) * 4 + c;
+      out_dst = (kGradCols + 2 + col) * kGradColumn + (k + 1) * kGradRow + c * 16;
+    }
+  }
+  u32x4 fetched[kFetch], fetched_out;
+  // Slab s of the input and row s + 1 of the output gradient.
+  auto fetch = [&](int s) __attribute__((always_inline)) {
+    if (s >= 0 && s < nx) {
+      const u32x4* slab = reinterpret_cast<const u32x4*>(in) + (long)s * ny * nz * 4;
 #pragma unroll
-  for (int tl = 0; tl < kTapsPerWave; ++tl) {
-    const int t = wave + 4 * tl;
-    if (t >= kTaps) continue;
+      for (int f = 0; f < kFetch; ++f) fetched[f] = slab[src[f]];
+    }
+    if (s + 1 < x1) fetched_out = (reinterpret_cast<const u32x4*>(dout) + (long)(s + 1) * ny * nz * 4)[out_src];
+  };
+  float bias_acc[8] = {};
+  auto stage = [&](int s, char* buffer) __attribute__((always_inline)) {
+    if (s >= 0 && s < nx) {
 #pragma unroll
-    for (int mt = 0; mt < 2; ++mt)
+      for (int f = 0; f < kFetch; ++f)
+        if (dst[f] >= 0) *reinterpret_cast<u32x4*>(buffer + dst[f]) = fetched[f];
+    }
+    if (s + 1 < x1 && out_dst >= 0) {
+      *reinterpret_cast<u32x4*>(buffer + out_dst) = fetched_out;
 #pragma unroll
-      for (int nt = 0; nt < 2; ++nt)
+      for (int e = 0; e < 4; ++e) {
+        bias_acc[2 * e] += __uint_as_float(fetched_out[e] << 16);
+        bias_acc[2 * e + 1] += __uint_as_float(fetched_out[e] & 0xffff0000u);
+      }
+    }
+  };
+  const int lane_offset = (8 * (lane >> 5) + ((lane & 15) >> 2)) * kGradRow + ((lane >> 4) & 1) * 32 + (lane & 3) * 8;
+  const int out_column = (kGradCols + 2 + half) * kGradColumn + kGradRow;
+  int pair_at[3], pair[3] = {2 * part, 2 * part + 1, 8};
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int co = mt * 16 + group * 4 + r, ci = nt * 16 + row;
-          part[(t * kC + co) * kC + ci] = acc[tl][mt][nt][r];
+  for (int q = 0; q < 3; ++q) pair_at[q] = (half + pair[q] / 3) * kGradColumn + pair[q] % 3 * kGradRow;
+  floatx16 acc[3][3];  // [pair][di]
+#pragma unroll
+  for (int q = 0; q < 3; ++q)
+#pragma unroll
+    for (int d = 0; d < 3; ++d)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[q][d][r] = 0.0f;
+  __syncthreads();
+  fetch(x0 - 1);
+  stage(x0 - 1, shared);
+  int current = 0;
+  bf16x8 rows[3][T];
+  // Input slab s with the gradient's rows s - 1 (A), s (B) and s + 1 (C, read here).
+  auto step = [&](int s, bf16x8(&A)[T], bf16x8(&B)[T], bf16x8(&C)[T]) __attribute__((always_inline)) {
+    __syncthreads();
+    const char* buffer = shared + current * kGradBuffer;
+    if (s < x1) fetch(s + 1);
+    const bool has_a = s - 1 >= x0, has_b = s >= x0 && s < x1, has_c = s + 1 < x1;
+    if (has_c) {
+#pragma unroll
+      for (int c = 0; c < T; ++c) C[c] = column_operand(buffer + out_column + c * 16 * kGradRow, lane_offset);
+    }
+    if (s >= 0 && s < nx) {
+#pragma unroll
+      for (int c = 0; c < T; ++c)
+#pragma unroll
+        for (int q = 0; q < 3; ++q) {
+          if (q == 2 && c != part) continue;
+          const bf16x8 x = column_operand(buffer + pair_at[q] + c * 16 * kGradRow, lane_offset);
+          if (has_c) acc[q][0] = mfma32(C[c], x, acc[q][0]);
+          if (has_b) acc[q][1] = mfma32(B[c], x, acc[q][1]);
+          if (has_a) acc[q][2] = mfma32(A[c], x, acc[q][2]);
         }
+    }
+    current ^= 1;
+    if (s < x1) stage(s + 1, shared + current * kGradBuffer);
+  };
+  for (int s = x0 - 1;;) {
+    step(s, rows[0], rows[1], rows[2]);
+    if (++s > x1) break;
+    step(s, rows[1], rows[2], rows[0]);
+    if (++s > x1) break;
+    step(s, rows[2], rows[0], rows[1]);
+    if (++s > x1) break;
   }
-  if (tid < kC) part[kWeights + tid] = bias_acc;
+  float* result = partials + (long)blockIdx.x * kLayer;
+  float* red = reinterpret_cast<float*>(shared);
+  // Lane l's sums: input channel l % 32, output channels 8 (r / 4) + 4 (l / 32) + r % 4.
+  auto element = [&](int r) { return (8 * (r / 4) + 4 * (lane >> 5) + r % 4) * kC + (lane & 31); };
+  __syncthreads();
+  if (half == 1)
+#pragma unroll
+    for (int q = 0; q < 2; ++q)
+#pragma unroll
+      for (int d = 0; d < 3; ++d)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) red[(d * 8 + pair[q]) * kC * kC + element(r)] = acc[q][d][r];
+  __syncthreads();
+  if (half == 0)
+#pragma unroll
+    for (int q = 0; q < 2; ++q)
+#pragma unroll
+      for (int d = 0; d < 3; ++d)
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+          result[(d * 9 + pair[q]) * kC * kC + element(r)] =
+              acc[q][d][r] + red[(d * 8 + pair[q]) * kC * kC + element(r)];
+  __syncthreads();
+#pragma unroll
+  for (int d = 0; d < 3; ++d)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) red[(wave * 3 + d) * kC * kC + element(r)] = acc[2][d][r];
+  // Bias: lanes of equal l % 4 hold the same 8 channels.
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    for (int off = 4; off < 64; off <<= 1) bias_acc[e] += __shfl_xor(bias_acc[e], off);
+    if (lane < 4) bias_part[wave][lane * 8 + e] = bias_acc[e];
+  }
+  __syncthreads();
+  for (int e = tid; e < 3 * kC * kC; e += kGradThreads) {
+    float sum = 0.0f;
+#pragma unroll
+    for (int v = 0; v < 8; ++v) sum += red[v * 3 * kC * kC + e];
+    result[(e / (kC * kC) * 9 + 8) * kC * kC + e % (kC * kC)] = sum;
+  }
+  if (tid < kC) {
+    float sum = 0.0f;
+#pragma unroll
+    for (int v = 0; v < 8; ++v) sum += bias_part[v][tid];
+    result[kWeights + tid] = sum;
+  }
 }
 
 // grad[p] = sum over blocks of partials[b][p], in block order.  Bound by
-// reading the partials (57 MB for 512 blocks): one thread a parameter, the
+// reading the partials (28 MB for 256 blocks): one thread a parameter, the
 // adds in order, but kFoldBatch loads in flight and 64-thread blocks so that
 // every CU has some.  One load at a time in 256-thread blocks left 108 blocks
-// waiting on memory: 144 us a layer at 128x64x64, 12 us now.
+// waiting on memory: 144 us for 512 rows at 128x64x64, 12 us this way.
 constexpr int kFoldThreads = 64, kFoldBatch = 32;
 __global__ void __launch_bounds__(kFoldThreads)
     k_fold(const float* __restrict__ partials, int blocks, int count, float* __restrict__ out) {
@@ -611,7 +717,17 @@ void launch_sweep(int nx, int ny, int nz, const uint16_t* in, const uint16_t* w,
                            : k_conv3d_sweep<Epi, 4>;
   kernel<<<blocks, kSweepThreads, 0, s>>>(nx, ny, per, in, w, bias, mask, out, out_f32);
 }
-int wgrad_blocks(int nx, int ny) { return nx * ny < kMaxGradBlocks ? nx * ny : kMaxGradBlocks; }
+// Weight-gradient blocks: pairs of columns times chunks of slabs, one block
+// for each of the 256 CUs where the grid has as many, but four slabs a chunk
+// at least: a chunk reads two slabs more than it owns and writes 110 KB of
+// sums that the fold reads again.
+struct GradPlan {
+  int per, blocks;
+};
+GradPlan wgrad_plan(int nx, int ny) {
+  const int tiles_j = (ny + kGradCols - 1) / kGradCols, slabs = sweep_slabs(nx, tiles_j), per = slabs < 4 ? 4 : slabs;
+  return {per, tiles_j * ((nx + per - 1) / per)};
+}
 
 }  // namespace icyc
 
@@ -684,18 +800,22 @@ int icyc_conv3d_k8(int32_t nx, int32_t ny, int32_t nz, const uint16_t* in, const
 
 int64_t icyc_wgrad_partials_size(int32_t nx, int32_t ny, int32_t nz) {
   if (!valid_grid(nx, ny, nz)) return 0;
-  return (int64_t)wgrad_blocks(nx, ny) * kLayer;
+  return (int64_t)wgrad_plan(nx, ny).blocks * kLayer;
 }
 
 int icyc_conv3d_wgrad(int32_t nx, int32_t ny, int32_t nz, const uint16_t* in, const uint16_t* dout,
                       float* partials, float* grad, void* stream) {
-  if (!valid_grid(nx, ny, nz) || nz % 16 != 0 || nz > kColumn || !in || !dout || !partials || !grad)
+  if (!valid_grid(nx, ny, nz) || nz % 16 != 0 || nz > kMaxColumn || !in || !dout || !partials || !grad)
     return ICYC_ERR_ARGUMENT;
   hipStream_t s = (hipStream_t)stream;
-  const int blocks = wgrad_blocks(nx, ny);
-  k_conv3d_wgrad<<<blocks, kGradThreads, 0, s>>>(nx, ny, nz, in, dout, partials);
+  const GradPlan plan = wgrad_plan(nx, ny);
+  auto kernel = nz == 16   ? k_conv3d_wgrad<1>
+                : nz == 32 ? k_conv3d_wgrad<2>
+                : nz == 48 ? k_conv3d_wgrad<3>
+                           : k_conv3d_wgrad<4>;
+  kernel<<<plan.blocks, kGradThreads, 0, s>>>(nx, ny, plan.per, in, dout, partials);
   if (int rc = status()) return rc;
-  k_fold<<<blocks_of(kLayer, kFoldThreads), kFoldThreads, 0, s>>>(partials, blocks, kLayer, grad);
+  k_fold<<<blocks_of(kLayer, kFoldThreads), kFoldThreads, 0, s>>>(partials, plan.blocks, kLayer, grad);
   return status();
 }
 

@@ -296,3 +296,8 @@ SWEEP_SHAPES = [(1, 1, 16), (1, 5, 48), (4, 7, 48), (3, 9, 64), (70, 17, 16), (3
 @pytest.mark.parametrize("shape", SWEEP_SHAPES)
 def test_conv_sweep_edges(shape):
     test_conv_forward_epilogues(shape)
+
+
+@pytest.mark.parametrize("shape", SWEEP_SHAPES)
+def test_weight_gradient_edges(shape):
+    test_weight_gradient(shape)
