@@ -1558,308 +1558,314 @@ __device__ __forceinline__ void store_streamed(const icy3d_grid& g, float* __res
 }
 
 // ---------------------------------------------------------------------------
-// Tiled HOME pull stream (home.py:286-321 for flags 0/1 and solid cells).
+// HOME pull stream, alone and fused with the collision (home.py:199-211 then
+// :286-345 for flags 0/1 and solid cells; k_stream_boundary does flag 2).
 //
-// A block owns a (kTileJ x kTileK) column of cells and sweeps kTileX x
-// slabs.  Each slab (with a one-cell j/k halo) is staged once in LDS as 17
-// per-cell terms of the reconstruction (home.py:30-53):
-//   P = p - 1.5 tr S,  U = 3u,  D_a = 4.5 S_aa,  O_ab = 9 S_ab,
-//   T_ab = 13.5 (S_aa u_b + 2 S_ab u_a - 2 u_a^2 u_b)  (a != b),
-//   X = 27 (S_xz u_y + S_yz u_x + S_xy u_z - 2 u_x u_y u_z).
-// For a fixed (c_y, c_z) the reconstruction is a quadratic in c_x,
-//   f(c) = w(c) (P0 + c_x P1 + c_x^2 P2),
-// so one read of neighbour (s, j+dy, k+dz) gives the three populations
-// pulled by cells x = s+1, s, s-1 (c_x = +1, 0, -1).  Cell s-1 is complete
-// after slab s.  A non-fluid neighbour sets the link's bit in the cell's
-// 27-bit mask; at completion the masked links take the halfway bounce-back
-// R_q(p, -u, S) = R_{-q}(p, u, S) of the cell's own post-collision moments.
-// The next slab's loads are issued before the current slab is consumed.
-constexpr int kTileJ = 8, kTileK = 32, kTileX = 16;
-constexpr int kHaloJ = kTileJ + 2, kHaloK = kTileK + 2, kSlabCells = kHaloJ * kHaloK;
-constexpr int kStaged = 17;
-constexpr int kStageRounds = (kSlabCells + kTileJ * kTileK - 1) / (kTileJ * kTileK);
-
-struct SlabFetch {
-  float m[10];
-  int label;
+// With c the direction, the reconstruction of home.py:30-53 is a weight times
+// a cubic in c, f(c) = w(c) sum P_abd cx^a cy^b cz^d with 17 terms P_abd per
+// cell, and w(c) = w1(cx) w1(cy) w1(cz).  So the streamed moments
+// sum_c c^(alpha,beta,gamma) f_c(x - c) factor into three passes of one axis:
+// on the line of P0, P1, P2 along z a cell sends up = P0 + P1 + P2 to its
+// upper neighbour and dn = P0 - P1 + P2 to its lower one, and gets
+// U + D + 4 P0, U - D and U + D for the powers 0, 1, 2 of cz (w1 = 1/6, 4/6,
+// 1/6; the 1/216 comes last); then the same along y and along x.  A non-fluid
+// cell sends zeros, and its links come back by the bounce below.  About 140
+// operations and 36 LDS words a cell; summing the 27 pulled populations took
+// 450 and 122.
+//
+// A block owns J rows by K cells of a (y, z) tile and sweeps X slabs of x.
+// The tile with its halo, (J + 2) rows of K + 2 cells, is laid flat over the
+// lanes, 62 cells a wave: the first and last lane of a wave repeat a
+// neighbour wave's cell, so the z pass is a shift between lanes, and only the
+// y pass goes through LDS (nine up and nine dn values a cell, double
+// buffered, one barrier a slab).  The x pass keeps the previous slabs' up
+// values and centres in registers.  Loads of the next slab are issued before
+// the barrier.  Fused, a staged cell is collided on load (the shear rate from
+// its phase, water volume and energy, the force from its HOME acceleration):
+// moments come from g.home and go to g.home_post (the caller swaps them), and
+// solid cells carry their moments over, so every cell of the destination is
+// defined; otherwise moments come from g.home_post and go to g.home.  u is
+// written in place: no later read of the pass depends on it (the boundary
+// pass reads u only at its own flag-2 cells, left alone here).
+//
+// Bounce: a missing link's population is R_(-c) of the cell's own
+// post-collision moments.  A cell whose nine links towards one z neighbour are
+// all missing and no others (the z walls, in every row) gets their sums in
+// closed form from its own z lines; every other pattern goes link by link.
+struct StreamTiles {
+  int J, K, X, tiles_j, tiles_k;
 };
-
-__device__ __forceinline__ void fetch_slab_cell(const icy3d_grid& g, int s, int j0, int k0, int t, SlabFetch& f) {
-  const int gj = j0 - 1 + t / kHaloK, gk = k0 - 1 + t % kHaloK;
-  f.label = -2;
-#pragma unroll
-  for (int m = 0; m < 10; ++m) f.m[m] = 0.0f;
-  if (t < kSlabCells && s >= 0 && s < g.nx && gj >= 0 && gj < g.ny && gk >= 0 && gk < g.nz) {
-    const size_t N = cells(g);
-    const int n = (s * g.ny + gj) * g.nz + gk;
-    f.label = g.id[n];
-#pragma unroll
-    for (int m = 0; m < 10; ++m) f.m[m] = g.home_post[m * N + n];
-  }
-}
-
-// The 17 reconstruction terms of one staged cell from its post-collision
-// moments (zeros for a non-fluid cell, whose links are masked).
-__device__ __forceinline__ void stage_terms(float (*sv)[kSlabCells], int8_t* sid, int t, int label, const float* m) {
-  sid[t] = (int8_t)label;
-  const bool fluid = label == -1;
-  const float p = m[0], ux = m[1], uy = m[2], uz = m[3];
-  const float sxx = m[4], syy = m[5], szz = m[6], sxy = m[7], sxz = m[8], syz = m[9];
-  float v[kStaged];
-  v[0] = p - 1.5f * (sxx + syy + szz);
-  v[1] = 3.0f * ux;
-  v[2] = 3.0f * uy;
-  v[3] = 3.0f * uz;
-  v[4] = 4.5f * sxx;
-  v[5] = 4.5f * syy;
-  v[6] = 4.5f * szz;
-  v[7] = 9.0f * sxy;
-  v[8] = 9.0f * sxz;
-  v[9] = 9.0f * syz;
-  v[10] = 13.5f * (sxx * uy + 2.0f * sxy * ux - 2.0f * ux * ux * uy);  // T_xy
-  v[11] = 13.5f * (sxx * uz + 2.0f * sxz * ux - 2.0f * ux * ux * uz);  // T_xz
-  v[12] = 13.5f * (syy * ux + 2.0f * sxy * uy - 2.0f * uy * uy * ux);  // T_yx
-  v[13] = 13.5f * (syy * uz + 2.0f * syz * uy - 2.0f * uy * uy * uz);  // T_yz
-  v[14] = 13.5f * (szz * ux + 2.0f * sxz * uz - 2.0f * uz * uz * ux);  // T_zx
-  v[15] = 13.5f * (szz * uy + 2.0f * syz * uz - 2.0f * uz * uz * uy);  // T_zy
-  v[16] = 27.0f * (sxz * uy + syz * ux + sxy * uz - 2.0f * ux * uy * uz);
-#pragma unroll
-  for (int q = 0; q < kStaged; ++q) sv[q][t] = fluid ? v[q] : 0.0f;
-}
-__device__ __forceinline__ void stage_slab_cell(float (*sv)[kSlabCells], int8_t* sid, int t, const SlabFetch& f) {
-  if (t >= kSlabCells) return;
-  stage_terms(sv, sid, t, f.label, f.m);
-}
-
-__host__ __device__ constexpr float lattice_weight(int order) {
-  return order == 0 ? 8.0f / 27.0f : order == 1 ? 2.0f / 27.0f : order == 2 ? 1.0f / 54.0f : 1.0f / 216.0f;
-}
-
-template <int DY, int DZ>
-__device__ __forceinline__ void pull_neighbour(const float (*sv)[kSlabCells], const int8_t* sid, int base,
-                                               MomentSums& prev, MomentSums& cur, MomentSums& next,
-                                               unsigned& mask_prev, unsigned& mask_cur, unsigned& mask_next) {
-  constexpr int CY = -DY, CZ = -DZ;  // pulled direction (c_x, CY, CZ) from (s, j+DY, k+DZ)
-  constexpr int QM = 3 * (CY + 1) + (CZ + 1), Q0 = 9 + QM, QP = 18 + QM;
-  constexpr int O = (CY != 0) + (CZ != 0);
-  constexpr float W0 = lattice_weight(O), W1 = lattice_weight(O + 1);
-  constexpr float fy = CY, fz = CZ, ay = fy * fy - 1.0f / 3.0f, az = fz * fz - 1.0f / 3.0f;
-  const int idx = base + DY * kHaloK + DZ;
-  if (sid[idx] != -1) {
-    mask_next |= 1u << QP;
-    mask_cur |= 1u << Q0;
-    mask_prev |= 1u << QM;
-    return;
-  }
-  float P0 = sv[0][idx], P1 = sv[1][idx], P2 = sv[4][idx];
-  float bx = 0.0f;
-  if (CY != 0) bx += fy * sv[10][idx];
-  if (CZ != 0) bx += fz * sv[11][idx];
-  if (CY != 0) P0 += fy * sv[2][idx] + sv[5][idx];
-  if (CZ != 0) P0 += fz * sv[3][idx] + sv[6][idx];
-  if (CY != 0 && CZ != 0) P0 += fy * fz * sv[9][idx];
-  if (CZ != 0) P0 += ay * fz * sv[13][idx];
-  if (CY != 0) P0 += az * fy * sv[15][idx];
-  if (CY != 0 || CZ != 0) P0 -= bx * (1.0f / 3.0f);
-  if (CY != 0) P1 += fy * sv[7][idx];
-  if (CZ != 0) P1 += fz * sv[8][idx];
-  P1 += ay * sv[12][idx] + az * sv[14][idx];
-  if (CY != 0 && CZ != 0) P1 += fy * fz * sv[16][idx];
-  if (CY != 0 || CZ != 0) P2 += bx;
-  const float a = P0 + P2;
-  accumulate<QP>(next, W1 * (a + P1));
-  accumulate<Q0>(cur, W0 * P0);
-  accumulate<QM>(prev, W1 * (a - P1));
-}
-
-template <int Q>
-__device__ __forceinline__ void add_bounce(const Moments& own, unsigned mask, MomentSums& s) {
-  if (mask & (1u << Q)) accumulate<Q>(s, reconstruct<26 - Q>(own));
-  if constexpr (Q + 1 < 27) add_bounce<Q + 1>(own, mask, s);
-}
-
-__device__ __forceinline__ void finish_streamed_cell(const icy3d_grid& g, int x, int j, int k, MomentSums& s,
-                                                     unsigned mask) {
-  if (x < 0 || x >= g.nx || j >= g.ny || k >= g.nz) return;
-  const size_t N = cells(g);
-  const int n = lin(g, x, j, k);
-  const int flag = g.flag[n];
-  if (flag == 0 || flag == 1) {
-    if (mask) add_bounce<0>(load_moments(g.home_post, N, n), mask, s);
-    store_streamed(g, g.home, n, s);
-  } else if (flag < 0) {
-    float v[3] = {0.0f, 0.0f, 0.0f};
-    const int b = g.id[n];
-    if (b >= 0) body_velocity_at(g, x + 0.5f, j + 0.5f, k + 0.5f, b, v);
-    g.u[n] = v[0];
-    g.u[N + n] = v[1];
-    g.u[2 * N + n] = v[2];
-  }
-}
-
-__global__ void __launch_bounds__(kTileJ* kTileK) k_stream_tiled(icy3d_grid g) {
-  __shared__ float sv[kStaged][kSlabCells];
-  __shared__ int8_t sid[kSlabCells];
-  const int tk = threadIdx.x % kTileK, tj = threadIdx.x / kTileK;
-  const int k0 = blockIdx.x * kTileK, j0 = blockIdx.y * kTileJ, x0 = blockIdx.z * kTileX;
-  const int j = j0 + tj, k = k0 + tk;
-  const int base = (tj + 1) * kHaloK + (tk + 1);
-  const MomentSums zero = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
-  MomentSums prev = zero, cur = zero, next = zero;
-  unsigned mask_prev = 0, mask_cur = 0, mask_next = 0;
-  const int x_end = min(x0 + kTileX, g.nx);
-  SlabFetch f[kStageRounds];
-#pragma unroll
-  for (int r = 0; r < kStageRounds; ++r) fetch_slab_cell(g, x0 - 1, j0, k0, threadIdx.x + r * blockDim.x, f[r]);
-  for (int s = x0 - 1; s <= x_end; ++s) {
-    __syncthreads();
-#pragma unroll
-    for (int r = 0; r < kStageRounds; ++r) stage_slab_cell(sv, sid, threadIdx.x + r * blockDim.x, f[r]);
-    if (s < x_end) {
-#pragma unroll
-      for (int r = 0; r < kStageRounds; ++r) fetch_slab_cell(g, s + 1, j0, k0, threadIdx.x + r * blockDim.x, f[r]);
-    }
-    __syncthreads();
-    pull_neighbour<-1, -1>(sv, sid, base, prev, cur, next, mask_prev, mask_cur, mask_next);
-    pull_neighbour<-1, 0>(sv, sid, base, prev, cur, next, mask_prev, mask_cur, mask_next);
-    pull_neighbour<-1, 1>(sv, sid, base, prev, cur, next, mask_prev, mask_cur, mask_next);
-    pull_neighbour<0, -1>(sv, sid, base, prev, cur, next, mask_prev, mask_cur, mask_next);
-    pull_neighbour<0, 0>(sv, sid, base, prev, cur, next, mask_prev, mask_cur, mask_next);
-    pull_neighbour<0, 1>(sv, sid, base, prev, cur, next, mask_prev, mask_cur, mask_next);
-    pull_neighbour<1, -1>(sv, sid, base, prev, cur, next, mask_prev, mask_cur, mask_next);
-    pull_neighbour<1, 0>(sv, sid, base, prev, cur, next, mask_prev, mask_cur, mask_next);
-    pull_neighbour<1, 1>(sv, sid, base, prev, cur, next, mask_prev, mask_cur, mask_next);
-    if (s - 1 >= x0) finish_streamed_cell(g, s - 1, j, k, prev, mask_prev);
-    prev = cur;
-    cur = next;
-    next = zero;
-    mask_prev = mask_cur;
-    mask_cur = mask_next;
-    mask_next = 0;
-  }
-}
-
-// ---------------------------------------------------------------------------
-// Fused HOME collide-stream (home.py:199-211 then :286-321 for flags 0/1
-// and solid cells): the slab pipeline of k_stream_tiled, staging each cell's
-// pre-collision state instead of stored post-collision moments.  A staged
-// fluid cell is collided on the way into LDS (the shear rate from its phase,
-// water volume and energy; the force from its HOME acceleration), so the
-// post-collision moments never reach HBM.  Moments are read from g.home and
-// the streamed moments written to g.home_post (the caller swaps the two
-// buffers afterwards); u is written in place, which no later read of this
-// pass depends on (the boundary pass reads u only at its own flag-2 cells,
-// which this kernel leaves alone).  Solid cells carry their moments over,
-// so every cell of the destination is defined.  Block (0,0,0) clears the
-// body loads that the boundary pass accumulates.
-struct FusedFetch {
+constexpr int kStreamThreads = 1024, kWaveCells = 62;
+constexpr int kStreamCells = kStreamThreads / 64 * kWaveCells;
+struct StreamFetch {
   float m[10], a[3], phi, volume, energy;
-  int label;
+  int label, flag;
 };
-
-__device__ __forceinline__ void fetch_fused_cell(const icy3d_grid& g, int s, int j0, int k0, int t, FusedFetch& f) {
-  const int gj = j0 - 1 + t / kHaloK, gk = k0 - 1 + t % kHaloK;
-  f.label = -2;
-#pragma unroll
-  for (int m = 0; m < 10; ++m) f.m[m] = 0.0f;
-  f.a[0] = f.a[1] = f.a[2] = 0.0f;
-  f.phi = f.volume = f.energy = 0.0f;
-  if (t < kSlabCells && s >= 0 && s < g.nx && gj >= 0 && gj < g.ny && gk >= 0 && gk < g.nz) {
-    const size_t N = cells(g);
-    const int n = (s * g.ny + gj) * g.nz + gk;
-    // Every load is issued at once, without waiting for the label (a
-    // non-fluid cell's values are discarded when it is staged): 5% faster
-    // than loading the moments of fluid cells only.
-    f.label = g.id[n];
-#pragma unroll
-    for (int m = 0; m < 10; ++m) f.m[m] = g.home[m * N + n];
-#pragma unroll
-    for (int a = 0; a < 3; ++a) f.a[a] = g.accel[a * N + n];
-    f.phi = g.phi[n];
-    f.volume = g.water_volume[n];
-    f.energy = g.water_energy[n];
-  }
+struct Line3 {
+  float up, dn, c;
+};
+// v of the previous / next lane of the wave.
+__device__ __forceinline__ float from_below(float v) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x138, 0xf, 0xf, true));
+}
+__device__ __forceinline__ float from_above(float v) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x130, 0xf, 0xf, true));
+}
+__device__ __forceinline__ int from_below(int v) { return __builtin_amdgcn_update_dpp(0, v, 0x138, 0xf, 0xf, true); }
+__device__ __forceinline__ int from_above(int v) { return __builtin_amdgcn_update_dpp(0, v, 0x130, 0xf, 0xf, true); }
+// An element of a plane at a byte offset below 2^31 (a grid has fewer than
+// 2^27 cells): a uniform base and a 32-bit lane offset.
+__device__ __forceinline__ float plane_get(const float* base, unsigned offset) {
+  return *reinterpret_cast<const float*>(reinterpret_cast<const char*>(base) + offset);
+}
+__device__ __forceinline__ void plane_set(float* base, unsigned offset, float v) {
+  *reinterpret_cast<float*>(reinterpret_cast<char*>(base) + offset) = v;
 }
 
-__device__ __forceinline__ void stage_fused_cell(const icy3d_grid& g, float (*sv)[kSlabCells], int8_t* sid, int t,
-                                                 const FusedFetch& f) {
-  if (t >= kSlabCells) return;
-  Moments post;
-  if (f.label == -1) {
-    Moments pre;
+template <bool Fused>
+__global__ void __launch_bounds__(kStreamThreads) k_stream_rows(icy3d_grid g, StreamTiles T) {
+  // The y pass's values of a slab: up then dn, nine each, as 4 + 4 + 1 words.
+  __shared__ float4 quad[2][4][kStreamCells];
+  __shared__ float single[2][2][kStreamCells];
+  __shared__ uint8_t links[2][kStreamCells];  // bits 0, 1, 2: fluid at k - 1, k, k + 1
+  if (Fused && blockIdx.x == 0)
+    for (int t = threadIdx.x; t < ICY3D_MAX_BODIES * 6; t += blockDim.x) (&g.control->loads[0][0])[t] = 0.0f;
+  const size_t N = cells(g);
+  const int L = T.K + 2, lane = threadIdx.x & 63;
+  const int tile_k = (int)blockIdx.x % T.tiles_k, tile_j = (int)blockIdx.x / T.tiles_k % T.tiles_j;
+  const int x0 = (int)blockIdx.x / T.tiles_k / T.tiles_j * T.X, x1 = min(x0 + T.X, g.nx);
+  const int t = (int)(threadIdx.x >> 6) * kWaveCells + lane - 1;
+  const int row = t < 0 ? 0 : t / L, col = t < 0 ? 0 : t - row * L;
+  const int j = tile_j * T.J - 1 + row, k = tile_k * T.K - 1 + col;
+  const bool present = t >= 0 && row < T.J + 2 && j >= 0 && j < g.ny && k >= 0 && k < g.nz;
+  const bool sends = lane >= 1 && lane <= kWaveCells && row < T.J + 2;
+  const bool owned = present && sends && row >= 1 && row <= T.J && col >= 1 && col <= T.K;
+  const unsigned in_plane = present ? (unsigned)(j * g.nz + k) : 0u, plane = (unsigned)(g.ny * g.nz);
+  const float* source = Fused ? g.home : g.home_post;
+  float* target = Fused ? g.home_post : g.home;
+
+  StreamFetch f;
+  auto fetch = [&](int s) __attribute__((always_inline)) {
+    f.label = -2;
+    f.flag = -1;
+    if (present && s >= 0 && s < g.nx) {
+      const unsigned n = (unsigned)s * plane + in_plane, o = 4u * n;
+      // Every load is issued at once, without waiting for the label: a
+      // non-fluid cell's values are discarded.
+      f.label = g.id[n];
+      f.flag = g.flag[n];
 #pragma unroll
-    for (int m = 0; m < 10; ++m) pre.m[m] = f.m[m];
-    const float rate = home_shear_rate(g, f.phi, f.volume, f.energy);
-    post = central_collision(pre, f.a[0], f.a[1], f.a[2], rate, g.bulk_rate);
-  } else {
+      for (int m = 0; m < 10; ++m) f.m[m] = plane_get(source + m * N, o);
+#pragma unroll
+      for (int e = 0; e < 3; ++e) f.a[e] = plane_get(g.accel + e * N, o);
+      if (Fused) {
+        f.phi = plane_get(g.phi, o);
+        f.volume = plane_get(g.water_volume, o);
+        f.energy = plane_get(g.water_energy, o);
+      }
+    }
+  };
+  fetch(x0 - 1);
+  // Of the x lines (beta, gamma) = 00, 10, 20, 01, 11, 02: the up values of
+  // the last two slabs and the centre of the last.
+  float up_a[6], up_b[6], centre[6];
+#pragma unroll
+  for (int l = 0; l < 6; ++l) up_a[l] = up_b[l] = centre[l] = 0.0f;
+  float wall[6] = {0, 0, 0, 0, 0, 0}, acc[3] = {0, 0, 0};  // of the last slab's cell
+  int flag = -1;
+  unsigned fluid = 0u;  // bit 9 (dx + 1) + 3 (dy + 1) + dz + 1: fluid at that neighbour of the last slab's cell
+
+  for (int s = x0 - 1; s <= x1; ++s) {
+    const int buffer = s & 1;
+    const bool is_fluid = f.label == -1;
+    Moments post;
 #pragma unroll
     for (int m = 0; m < 10; ++m) post.m[m] = 0.0f;
-  }
-  stage_terms(sv, sid, t, f.label, post.m);
-}
+    if (is_fluid) {
+      Moments pre;
+#pragma unroll
+      for (int m = 0; m < 10; ++m) pre.m[m] = f.m[m];
+      post = Fused ? central_collision(pre, f.a[0], f.a[1], f.a[2], home_shear_rate(g, f.phi, f.volume, f.energy),
+                                       g.bulk_rate)
+                   : pre;
+    } else if (owned && s >= x0 && s < x1) {
+      const unsigned n = (unsigned)s * plane + in_plane, o = 4u * n;
+      float v[3] = {0.0f, 0.0f, 0.0f};
+      if (f.label >= 0) body_velocity_at(g, s + 0.5f, j + 0.5f, k + 0.5f, f.label, v);
+#pragma unroll
+      for (int e = 0; e < 3; ++e) plane_set(g.u + e * N, o, v[e]);
+      if (Fused)
+#pragma unroll
+        for (int m = 0; m < 10; ++m) plane_set(target + m * N, o, f.m[m]);
+    }
+    const float acc_s[3] = {f.a[0], f.a[1], f.a[2]};
+    const int flag_s = f.flag;
+    if (s < x1) fetch(s + 1);
 
-__device__ __forceinline__ void finish_fused_cell(const icy3d_grid& g, int x, int j, int k, MomentSums& s,
-                                                  unsigned mask) {
-  if (x < 0 || x >= g.nx || j >= g.ny || k >= g.nz) return;
-  const size_t N = cells(g);
-  const int n = lin(g, x, j, k);
-  const int flag = g.flag[n];
-  if (flag == 0 || flag == 1) {
-    if (mask) add_bounce<0>(collide_at(g, n), mask, s);
-    store_streamed(g, g.home_post, n, s);
-  } else if (flag < 0) {
-    float v[3] = {0.0f, 0.0f, 0.0f};
-    const int b = g.id[n];
-    if (b >= 0) body_velocity_at(g, x + 0.5f, j + 0.5f, k + 0.5f, b, v);
-    g.u[n] = v[0];
-    g.u[N + n] = v[1];
-    g.u[2 * N + n] = v[2];
+    // z lines (a, b) = 00, 10, 01, 20, 02, 11, 12, 21.
+    const float ux = post.m[1], uy = post.m[2], uz = post.m[3];
+    const float sxx = post.m[4], syy = post.m[5], szz = post.m[6], sxy = post.m[7], sxz = post.m[8], syz = post.m[9];
+    const float xxy = 13.5f * (sxx * uy + 2.0f * ux * (sxy - ux * uy)), xxz = 13.5f * (sxx * uz + 2.0f * ux * (sxz - ux * uz));
+    const float xyy = 13.5f * (syy * ux + 2.0f * uy * (sxy - ux * uy)), yyz = 13.5f * (syy * uz + 2.0f * uy * (syz - uy * uz));
+    const float xzz = 13.5f * (szz * ux + 2.0f * uz * (sxz - ux * uz)), yzz = 13.5f * (szz * uy + 2.0f * uz * (syz - uy * uz));
+    const float xyz = 27.0f * (sxz * uy + syz * ux + uz * (sxy - 2.0f * ux * uy));
+    const float third = 1.0f / 3.0f;
+    const float z0[8] = {post.m[0] - 1.5f * (sxx + syy + szz), 3.0f * ux - third * (xyy + xzz),
+                         3.0f * uy - third * (xxy + yzz), 4.5f * sxx, 4.5f * syy, 9.0f * sxy, xyy, xxy};
+    const float z1[8] = {3.0f * uz - third * (xxz + yyz), 9.0f * sxz, 9.0f * syz, xxz, yyz, xyz, 0.0f, 0.0f};
+    const float even[8] = {z0[0] + 4.5f * szz, z0[1] + xzz, z0[2] + yzz, z0[3], z0[4], z0[5], xyy, xxy};
+    auto line = [](float p0, float p1, float p2) __attribute__((always_inline)) {
+      const float sum = p0 + p2;
+      return Line3{sum + p1, sum - p1, p0};
+    };
+    const int here = is_fluid ? 1 : 0;
+    const int z_links = from_below(here) | here << 1 | from_above(here) << 2;
+    // The closed-form bounce of the links towards a missing z neighbour (36
+    // times their sums): c_z of the returning populations is +1 from below.
+    float wall_s[6];
+    {
+      const float side = (z_links & 1) == 0 ? -1.0f : 1.0f;
+      float e[8];
 #pragma unroll
-    for (int m = 0; m < 10; ++m) g.home_post[m * N + n] = g.home[m * N + n];
-  }
-}
-
-__global__ void __launch_bounds__(kTileJ* kTileK) k_collide_stream_tiled(icy3d_grid g) {
-  __shared__ float sv[kStaged][kSlabCells];
-  __shared__ int8_t sid[kSlabCells];
-  if (blockIdx.x == 0 && blockIdx.y == 0 && blockIdx.z == 0)
-    for (int t = threadIdx.x; t < ICY3D_MAX_BODIES * 6; t += blockDim.x) (&g.control->loads[0][0])[t] = 0.0f;
-  const int tk = threadIdx.x % kTileK, tj = threadIdx.x / kTileK;
-  const int k0 = blockIdx.x * kTileK, j0 = blockIdx.y * kTileJ, x0 = blockIdx.z * kTileX;
-  const int j = j0 + tj, k = k0 + tk;
-  const int base = (tj + 1) * kHaloK + (tk + 1);
-  const MomentSums zero = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
-  MomentSums prev = zero, cur = zero, next = zero;
-  unsigned mask_prev = 0, mask_cur = 0, mask_next = 0;
-  const int x_end = min(x0 + kTileX, g.nx);
-  FusedFetch f[kStageRounds];
+      for (int l = 0; l < 8; ++l) e[l] = even[l] + side * z1[l];
+      wall_s[0] = 36.0f * e[0] + 12.0f * (e[3] + e[4]);
+      wall_s[1] = -12.0f * e[1] - 4.0f * e[6];
+      wall_s[2] = -12.0f * e[2] - 4.0f * e[7];
+      wall_s[3] = 12.0f * (e[0] + e[3]) + 4.0f * e[4];
+      wall_s[4] = 12.0f * (e[0] + e[4]) + 4.0f * e[3];
+      wall_s[5] = 4.0f * e[5];
+    }
+    float zp[8][3];
 #pragma unroll
-  for (int r = 0; r < kStageRounds; ++r) fetch_fused_cell(g, x0 - 1, j0, k0, threadIdx.x + r * blockDim.x, f[r]);
-  for (int s = x0 - 1; s <= x_end; ++s) {
-    __syncthreads();
+    for (int l = 0; l < 8; ++l) {
+      const float U = from_below(even[l] + z1[l]), D = from_above(even[l] - z1[l]);
+      zp[l][2] = U + D;
+      zp[l][1] = U - D;
+      zp[l][0] = zp[l][2] + 4.0f * z0[l];
+    }
+    // y lines (a, gamma): powers b = 0, 1, 2 of cy are z lines (a, b).
+    Line3 y[3][3];
 #pragma unroll
-    for (int r = 0; r < kStageRounds; ++r) stage_fused_cell(g, sv, sid, threadIdx.x + r * blockDim.x, f[r]);
-    if (s < x_end) {
-#pragma unroll
-      for (int r = 0; r < kStageRounds; ++r) fetch_fused_cell(g, s + 1, j0, k0, threadIdx.x + r * blockDim.x, f[r]);
+    for (int c = 0; c < 3; ++c) {
+      y[0][c] = line(zp[0][c], zp[2][c], zp[4][c]);
+      y[1][c] = line(zp[1][c], zp[5][c], zp[6][c]);
+      y[2][c] = line(zp[3][c], zp[7][c], 0.0f);
+    }
+    if (sends) {
+      quad[buffer][0][t] = make_float4(y[0][0].up, y[0][1].up, y[0][2].up, y[1][0].up);
+      quad[buffer][1][t] = make_float4(y[1][1].up, y[1][2].up, y[2][0].up, y[2][1].up);
+      quad[buffer][2][t] = make_float4(y[0][0].dn, y[0][1].dn, y[0][2].dn, y[1][0].dn);
+      quad[buffer][3][t] = make_float4(y[1][1].dn, y[1][2].dn, y[2][0].dn, y[2][1].dn);
+      single[buffer][0][t] = y[2][2].up;
+      single[buffer][1][t] = y[2][2].dn;
+      links[buffer][t] = (uint8_t)z_links;
     }
     __syncthreads();
-    pull_neighbour<-1, -1>(sv, sid, base, prev, cur, next, mask_prev, mask_cur, mask_next);
-    pull_neighbour<-1, 0>(sv, sid, base, prev, cur, next, mask_prev, mask_cur, mask_next);
-    pull_neighbour<-1, 1>(sv, sid, base, prev, cur, next, mask_prev, mask_cur, mask_next);
-    pull_neighbour<0, -1>(sv, sid, base, prev, cur, next, mask_prev, mask_cur, mask_next);
-    pull_neighbour<0, 0>(sv, sid, base, prev, cur, next, mask_prev, mask_cur, mask_next);
-    pull_neighbour<0, 1>(sv, sid, base, prev, cur, next, mask_prev, mask_cur, mask_next);
-    pull_neighbour<1, -1>(sv, sid, base, prev, cur, next, mask_prev, mask_cur, mask_next);
-    pull_neighbour<1, 0>(sv, sid, base, prev, cur, next, mask_prev, mask_cur, mask_next);
-    pull_neighbour<1, 1>(sv, sid, base, prev, cur, next, mask_prev, mask_cur, mask_next);
-    if (s - 1 >= x0) finish_fused_cell(g, s - 1, j, k, prev, mask_prev);
-    prev = cur;
-    cur = next;
-    next = zero;
-    mask_prev = mask_cur;
-    mask_cur = mask_next;
-    mask_next = 0;
+    if (owned) {
+      float U[3][3], D[3][3];
+      {
+        const float4 p = quad[buffer][0][t - L], q = quad[buffer][1][t - L];
+        const float4 v = quad[buffer][2][t + L], w = quad[buffer][3][t + L];
+        U[0][0] = p.x, U[0][1] = p.y, U[0][2] = p.z, U[1][0] = p.w;
+        U[1][1] = q.x, U[1][2] = q.y, U[2][0] = q.z, U[2][1] = q.w;
+        D[0][0] = v.x, D[0][1] = v.y, D[0][2] = v.z, D[1][0] = v.w;
+        D[1][1] = w.x, D[1][2] = w.y, D[2][0] = w.z, D[2][1] = w.w;
+        U[2][2] = single[buffer][0][t - L];
+        D[2][2] = single[buffer][1][t + L];
+      }
+      // The cell s - 1 is complete with this slab's dn values.
+      const unsigned slab_links = (unsigned)links[buffer][t - L] | (unsigned)z_links << 3 | (unsigned)links[buffer][t + L] << 6;
+      fluid |= slab_links << 18;
+      float h[3][6];  // power a of cx of the x lines
+#pragma unroll
+      for (int e = 0; e < 3; ++e) {
+        h[e][2] = U[e][0] + D[e][0];
+        h[e][1] = U[e][0] - D[e][0];
+        h[e][0] = h[e][2] + 4.0f * y[e][0].c;
+        h[e][4] = U[e][1] - D[e][1];
+        h[e][3] = U[e][1] + D[e][1] + 4.0f * y[e][1].c;
+        h[e][5] = U[e][2] + D[e][2] + 4.0f * y[e][2].c;
+      }
+      Line3 x[6];
+#pragma unroll
+      for (int l = 0; l < 6; ++l) x[l] = line(h[0][l], h[1][l], h[2][l]);
+      if (s > x0 && (flag == 0 || flag == 1)) {
+        MomentSums m;
+        float sides[6];
+#pragma unroll
+        for (int l = 0; l < 6; ++l) sides[l] = up_a[l] + x[l].dn;
+        m.p = sides[0] + 4.0f * centre[0];
+        m.jx = up_a[0] - x[0].dn;
+        m.xx = sides[0];
+        m.jy = sides[1] + 4.0f * centre[1];
+        m.xy = up_a[1] - x[1].dn;
+        m.yy = sides[2] + 4.0f * centre[2];
+        m.jz = sides[3] + 4.0f * centre[3];
+        m.xz = up_a[3] - x[3].dn;
+        m.yz = sides[4] + 4.0f * centre[4];
+        m.zz = sides[5] + 4.0f * centre[5];
+        const unsigned n = (unsigned)(s - 1) * plane + in_plane;
+        constexpr unsigned kAll = 0x7ffffffu, kBelow = 0x1249249u, kAbove = kBelow << 2;
+        const unsigned missing = ~fluid & kAll;
+        if (missing == kBelow || missing == kAbove) {
+          const float c = missing == kBelow ? 1.0f : -1.0f;
+          m.p += wall[0];
+          m.jx += wall[1];
+          m.jy += wall[2];
+          m.jz += c * wall[0];
+          m.xx += wall[3];
+          m.yy += wall[4];
+          m.zz += wall[0];
+          m.xy += wall[5];
+          m.xz += c * wall[1];
+          m.yz += c * wall[2];
+        } else if (missing) {
+          const Moments own = Fused ? collide_at(g, (int)n) : load_moments(g.home_post, N, (int)n);
+          for (int q = 0; q < 27; ++q) {  // the link towards neighbour q returns as direction 26 - q
+            if (!__any((missing >> q) & 1u)) continue;
+            const float r = (missing >> q) & 1u ? 216.0f * reconstruct_dyn(q, own) : 0.0f;
+            const float cxf = (float)-cx(q), cyf = (float)-cy(q), czf = (float)-cz(q);
+            m.p += r;
+            m.jx += cxf * r;
+            m.jy += cyf * r;
+            m.jz += czf * r;
+            m.xx += cxf * cxf * r;
+            m.yy += cyf * cyf * r;
+            m.zz += czf * czf * r;
+            m.xy += cxf * cyf * r;
+            m.xz += cxf * czf * r;
+            m.yz += cyf * czf * r;
+          }
+        }
+        constexpr float kScale = 1.0f / 216.0f;
+        const unsigned o = 4u * n;
+        const float p = kScale * m.p, p3 = p * third;
+        plane_set(target, o, p);
+        plane_set(target + N, o, kScale * m.jx);
+        plane_set(target + 2 * N, o, kScale * m.jy);
+        plane_set(target + 3 * N, o, kScale * m.jz);
+        plane_set(target + 4 * N, o, kScale * m.xx - p3);
+        plane_set(target + 5 * N, o, kScale * m.yy - p3);
+        plane_set(target + 6 * N, o, kScale * m.zz - p3);
+        plane_set(target + 7 * N, o, kScale * m.xy);
+        plane_set(target + 8 * N, o, kScale * m.xz);
+        plane_set(target + 9 * N, o, kScale * m.yz);
+        plane_set(g.u, o, kScale * m.jx + 0.5f * acc[0]);
+        plane_set(g.u + N, o, kScale * m.jy + 0.5f * acc[1]);
+        plane_set(g.u + 2 * N, o, kScale * m.jz + 0.5f * acc[2]);
+      }
+      fluid >>= 9;
+#pragma unroll
+      for (int l = 0; l < 6; ++l) {
+        up_a[l] = up_b[l];
+        up_b[l] = x[l].up;
+        centre[l] = x[l].c;
+        wall[l] = wall_s[l];
+      }
+    }
+    flag = flag_s;
+#pragma unroll
+    for (int e = 0; e < 3; ++e) acc[e] = acc_s[e];
   }
 }
 
@@ -2186,10 +2192,48 @@ int launch_recover(const icy3d_grid& g, int parity, int recover_flow, hipStream_
   ICY_LAUNCH_CHECK();
   return 0;
 }
+// The stream's tiles.  z is cut into as few tiles as leave ten rows a block
+// (eight of them its own).  Then the rows and slabs a block owns: a block
+// takes a CU to itself, a slab costs it a fixed latency and a time for each
+// wave, and it stages two rows and two slabs more than it owns, so the
+// cheapest cut is searched over the row tiles that fit and the slab chunks
+// that fill whole rounds of the 256 CUs (kSlabLatency, kWaveTime: microseconds
+// measured at 24x20x16 and 256x128x128).
+StreamTiles stream_tiles(const icy3d_grid& g) {
+  constexpr int kCus = 256;
+  constexpr double kSlabLatency = 1.6, kWaveTime = 0.24;
+  StreamTiles best = {};
+  int tiles_k = 1;
+  while (10 * ((g.nz + tiles_k - 1) / tiles_k + 2) > kStreamCells) ++tiles_k;
+  const int K = (g.nz + tiles_k - 1) / tiles_k, L = K + 2;
+  tiles_k = (g.nz + K - 1) / K;
+  const int most = kStreamCells / L - 2;
+  double least = 0.0;
+  for (int tiles_j = (g.ny + most - 1) / most; tiles_j <= g.ny; ++tiles_j) {
+    const int J = (g.ny + tiles_j - 1) / tiles_j, waves = ((J + 2) * L + kWaveCells - 1) / kWaveCells;
+    const int yz = tiles_k * ((g.ny + J - 1) / J);
+    for (int rounds = 1; rounds <= 4; ++rounds) {
+      const int chunks = yz >= kCus * rounds ? 1 : kCus * rounds / yz;
+      const int X = (g.nx + chunks - 1) / chunks, blocks = yz * ((g.nx + X - 1) / X);
+      const double cost = (double)((blocks + kCus - 1) / kCus) * (X + 2) * (kSlabLatency + kWaveTime * waves);
+      if (best.J == 0 || cost < least) {
+        least = cost;
+        best = {J, K, X, (g.ny + J - 1) / J, tiles_k};
+      }
+    }
+  }
+  return best;
+}
+template <bool Fused>
+void launch_stream_rows(const icy3d_grid& g, hipStream_t s) {
+  const StreamTiles T = stream_tiles(g);
+  const unsigned blocks = (unsigned)(T.tiles_k * T.tiles_j * ((g.nx + T.X - 1) / T.X));
+  const int waves = ((T.J + 2) * (T.K + 2) + kWaveCells - 1) / kWaveCells;
+  k_stream_rows<Fused><<<blocks, waves * 64, 0, s>>>(g, T);
+}
 int launch_stream(const icy3d_grid& g, hipStream_t s) {
   if ((int)(kListBlocks * kLoadSlots) > g.partials_capacity) return ICY3D_ERR_ARGUMENT;
-  const dim3 tiles((g.nz + kTileK - 1) / kTileK, (g.ny + kTileJ - 1) / kTileJ, (g.nx + kTileX - 1) / kTileX);
-  k_stream_tiled<<<tiles, kTileJ * kTileK, 0, s>>>(g);
+  launch_stream_rows<false>(g, s);
   k_stream_boundary<false><<<kListBlocks, kBlock, 0, s>>>(g);
   if (g.bodies > 0) k_finish_loads<<<g.bodies * 6, 256, 0, s>>>(g, (int)kListBlocks);
   ICY_LAUNCH_CHECK();
@@ -2199,8 +2243,7 @@ int launch_stream(const icy3d_grid& g, hipStream_t s) {
 // caller swaps the buffers), body loads cleared and accumulated.
 int launch_collide_stream(const icy3d_grid& g, hipStream_t s) {
   if ((int)(kListBlocks * kLoadSlots) > g.partials_capacity) return ICY3D_ERR_ARGUMENT;
-  const dim3 tiles((g.nz + kTileK - 1) / kTileK, (g.ny + kTileJ - 1) / kTileJ, (g.nx + kTileX - 1) / kTileX);
-  k_collide_stream_tiled<<<tiles, kTileJ * kTileK, 0, s>>>(g);
+  launch_stream_rows<true>(g, s);
   k_stream_boundary<true><<<kListBlocks, kBlock, 0, s>>>(g);
   if (g.bodies > 0) k_finish_loads<<<g.bodies * 6, 256, 0, s>>>(g, (int)kListBlocks);
   ICY_LAUNCH_CHECK();
