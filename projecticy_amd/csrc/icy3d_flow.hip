@@ -720,18 +720,6 @@ __global__ void k_export_phase(icy3d_grid g, int parity, float* __restrict__ out
 
 // ---------------------------------------------------------------------------
 // Forces (simulator.py:418-519) and HOME acceleration (home.py:127-197).
-enum Mode { kGeneral = 0, kInterior = 1, kTank = 2 };
-
-template <int MODE>
-__device__ __forceinline__ bool link_fluid(const icy3d_grid& g, int i, int j, int k) {
-  if (MODE == kInterior) return true;
-  if (MODE == kTank) {
-    const int b = g.boundary;
-    return i >= b && i < g.nx - b && j >= b && j < g.ny - b && k >= b && k < g.nz - b;
-  }
-  return fluid_at(g, i, j, k);
-}
-
 // simulator.py:193-215
 __device__ bool connected(const icy3d_grid& g, int i, int j, int k, int dx, int dy, int dz) {
   if (!fluid_at(g, i + dx, j + dy, k + dz)) return false;
@@ -790,7 +778,6 @@ __device__ void capillary_neighbor(const icy3d_grid& g, int i, int j, int k, int
   stress_of(g, v[0], v[1], v[2], s);
 }
 
-template <int MODE>
 __device__ void force_at(const icy3d_grid& g, const Cell& c, bool with_flux, float f[3]) {
   const size_t N = cells(g);
   const int n = c.n;
@@ -810,15 +797,7 @@ __device__ void force_at(const icy3d_grid& g, const Cell& c, bool with_flux, flo
       int i = c.i + cx(q), j = c.j + cy(q), k = c.k + cz(q);
       float v[3];
       bool valid = false;
-      if (MODE == kTank) {
-        const int b = g.boundary;
-        int K[3] = {min(max(i, b), g.nx - b - 1), min(max(j, b), g.ny - b - 1), min(max(k, b), g.nz - b - 1)};
-        load_grad(g, lin(g, K[0], K[1], K[2]), v);
-        if (K[0] != i) v[0] = -v[0];
-        if (K[1] != j) v[1] = -v[1];
-        if (K[2] != k) v[2] = -v[2];
-        valid = true;
-      } else if (link_fluid<MODE>(g, i, j, k)) {
+      if (fluid_at(g, i, j, k)) {
         load_grad(g, lin(g, i, j, k), v);
         valid = true;
       } else {
@@ -833,7 +812,7 @@ __device__ void force_at(const icy3d_grid& g, const Cell& c, bool with_flux, flo
         f[2] += coef * (gg * (float)cz(q) - gc * v[2]);
       }
     }
-    if (MODE == kGeneral && wall) {
+    if (wall) {
       for (int q = 0; q < 27; ++q) {
         if (q == 13) continue;
         int dx = cx(q), dy = cy(q), dz = cz(q);
@@ -854,7 +833,7 @@ __device__ void force_at(const icy3d_grid& g, const Cell& c, bool with_flux, flo
       for (int sign = 0; sign < 2; ++sign) {
         const int d = 2 * sign - 1;
         int i = c.i + (a == 0) * d, j = c.j + (a == 1) * d, k = c.k + (a == 2) * d;
-        if (!link_fluid<MODE>(g, i, j, k)) continue;
+        if (!fluid_at(g, i, j, k)) continue;
         const int m = lin(g, i, j, k);
         const float mass_flux = 0.5f * (g.flux[a * N + n] + g.flux[a * N + m]);
         const bool own = (float)d * mass_flux >= 0.0f;
@@ -908,7 +887,6 @@ __device__ void stress_neighbor_velocity(const icy3d_grid& g, int i, int j, int 
   }
 }
 
-template <int MODE>
 __device__ void acceleration_at(const icy3d_grid& g, const Cell& c, const float f[3], bool moment_pressure, float a[3]) {
   const size_t N = cells(g);
   const int n = c.n;
@@ -921,7 +899,7 @@ __device__ void acceleration_at(const icy3d_grid& g, const Cell& c, const float 
   for (int q = 0; q < 27; ++q) {
     if (q == 13) continue;
     int i = c.i + cx(q), j = c.j + cy(q), k = c.k + cz(q);
-    if (!link_fluid<MODE>(g, i, j, k)) continue;
+    if (!fluid_at(g, i, j, k)) continue;
     const int m = lin(g, i, j, k);
     const float rj = density(g, g.phi[m]);
     float term;
@@ -945,33 +923,11 @@ __device__ void acceleration_at(const icy3d_grid& g, const Cell& c, const float 
     for (int axis = 0; axis < 3; ++axis) {
       const int ex = axis == 0, ey = axis == 1, ez = axis == 2;
       float d[3];
-      if (MODE == kInterior) {
-        int p = lin(g, c.i + ex, c.j + ey, c.k + ez), m = lin(g, c.i - ex, c.j - ey, c.k - ez);
+      float plus[3], minus[3];
+      stress_neighbor_velocity(g, c.i, c.j, c.k, ex, ey, ez, plus);
+      stress_neighbor_velocity(g, c.i, c.j, c.k, -ex, -ey, -ez, minus);
 #pragma unroll
-        for (int e = 0; e < 3; ++e) d[e] = 0.5f * (g.u[e * N + p] - g.u[e * N + m]);
-      } else if (MODE == kTank) {
-        float left[3], right[3];
-#pragma unroll
-        for (int e = 0; e < 3; ++e) left[e] = right[e] = -g.u[e * N + n];
-        if (link_fluid<kTank>(g, c.i - ex, c.j - ey, c.k - ez)) {
-          int m = lin(g, c.i - ex, c.j - ey, c.k - ez);
-#pragma unroll
-          for (int e = 0; e < 3; ++e) left[e] = g.u[e * N + m];
-        }
-        if (link_fluid<kTank>(g, c.i + ex, c.j + ey, c.k + ez)) {
-          int p = lin(g, c.i + ex, c.j + ey, c.k + ez);
-#pragma unroll
-          for (int e = 0; e < 3; ++e) right[e] = g.u[e * N + p];
-        }
-#pragma unroll
-        for (int e = 0; e < 3; ++e) d[e] = 0.5f * (right[e] - left[e]);
-      } else {
-        float plus[3], minus[3];
-        stress_neighbor_velocity(g, c.i, c.j, c.k, ex, ey, ez, plus);
-        stress_neighbor_velocity(g, c.i, c.j, c.k, -ex, -ey, -ez, minus);
-#pragma unroll
-        for (int e = 0; e < 3; ++e) d[e] = 0.5f * (plus[e] - minus[e]);
-      }
+      for (int e = 0; e < 3; ++e) d[e] = 0.5f * (plus[e] - minus[e]);
 #pragma unroll
       for (int e = 0; e < 3; ++e) G[e][axis] = d[e];
     }
@@ -982,154 +938,62 @@ __device__ void acceleration_at(const icy3d_grid& g, const Cell& c, const float 
   }
 }
 
-template <int MODE>
-__device__ __forceinline__ void forces_cell(const icy3d_grid& g, int n, int with_flux, int moment_pressure) {
-  const size_t N = cells(g);
-  const Cell c = cell_of(g, n);
-  float f[3], a[3];
-  force_at<MODE>(g, c, with_flux != 0, f);
-  acceleration_at<MODE>(g, c, f, moment_pressure != 0, a);
-#pragma unroll
-  for (int e = 0; e < 3; ++e) {
-    g.force[e * N + n] = f[e];
-    g.accel[e * N + n] = a[e];
-  }
+// ---------------------------------------------------------------------------
+// Tiles of the row sweeps (k_forces_rows, k_stream_rows): J rows by K cells of
+// y and z, X slabs; the tile with its halo laid flat over the lanes, 62 cells
+// a wave.
+struct StreamTiles {
+  int J, K, X, tiles_j, tiles_k;
+};
+constexpr int kWaveCells = 62;
+constexpr int kStreamThreads = 1024, kForceThreads = 768;
+constexpr int sweep_cells(int threads) { return threads / 64 * kWaveCells; }
+// v of the previous / next lane of the wave.
+__device__ __forceinline__ float from_below(float v) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x138, 0xf, 0xf, true));
 }
-// Tiled interior forces (simulator.py:418-519 and home.py:127-197 for
-// flag-0 cells, every link fluid).  The two 26-neighbour sums factor with
-// the D3Q27 weights w(c) = w1(cx) w1(cy) w1(cz):
+__device__ __forceinline__ float from_above(float v) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x130, 0xf, 0xf, true));
+}
+__device__ __forceinline__ int from_below(int v) { return __builtin_amdgcn_update_dpp(0, v, 0x138, 0xf, 0xf, true); }
+__device__ __forceinline__ int from_above(int v) { return __builtin_amdgcn_update_dpp(0, v, 0x130, 0xf, 0xf, true); }
+// An element of a plane at a byte offset below 2^31 (a grid has fewer than
+// 2^27 cells): a uniform base and a 32-bit lane offset.
+__device__ __forceinline__ float plane_get(const float* base, unsigned offset) {
+  return *reinterpret_cast<const float*>(reinterpret_cast<const char*>(base) + offset);
+}
+__device__ __forceinline__ void plane_set(float* base, unsigned offset, float v) {
+  *reinterpret_cast<float*>(reinterpret_cast<char*>(base) + offset) = v;
+}
+
+// Interior forces (simulator.py:418-519 and home.py:127-197 for cells of
+// flag 0 and 1: every link fluid or a tank wall).  The two 26-neighbour sums
+// factor with the D3Q27 weights w(c) = w1(cx) w1(cy) w1(cz):
 //   capillary  f_a = kcap sum_q w_q (c_a |g|^2 - (c.g) g_a)
 //                  = kcap [D_a(|g|^2 - g_a^2) - sum_{b != a} D_b(g_a g_b)],
 //   pressure   a  += sum_q w_q c p*_m (rho - rho_m) / rho = D(p*) - D(p* rho_m) / rho
 //              (3 p_m (1/rho_m - 1/rho) = D(3 p/rho_m) - D(3 p) / rho without moments),
 // where D_a applies (u+ - u-)/6 along a and (u- + 4 u0 + u+)/6 along the
-// other two axes.  Per slab the eight staged quantities (|g|^2 - g_a^2,
-// g_a g_b, and the two pressure fields) sit in LDS; each thread forms the
-// y/z parts for its column and the x combination runs in registers over
-// three slabs.  The six face-neighbour terms (donor phase flux, viscous
-// velocity gradient) read u, flux and phi directly, the x neighbours from the
-// same register pipeline.
-constexpr int kForceJ = 4, kForceK = 64, kForceX = 32;
-constexpr int kForceHJ = kForceJ + 2, kForceHK = kForceK + 2, kForceSlab = kForceHJ * kForceHK;
-constexpr int kForceRounds = (kForceSlab + kForceJ * kForceK - 1) / (kForceJ * kForceK);
-// Staged per cell: Ax, Ay, Az, Bxy, Bxz, Byz, X1, X2 (stencil sums), then
-// u (3), phi and the mass flux (3) for the face-neighbour terms, and a wall
-// marker.
-constexpr int kForceQ = 16;
-constexpr int kStencilQ = 8, kU = 8, kPhi = 11, kFlux = 12, kWall = 15;
-
-// Raw values prefetched for one staged cell: grad (3), phi, pressure field,
-// u (3), flux (3).  A position inside the tank walls is fetched from its
-// mirror, the nearest cell of the fluid box (simulator.py:418-519, tank
-// links), with `wall` holding the mirrored axes; staging then turns it into
-// what the tank formulas use: the gradient with the mirrored components
-// negated (capillary), no pressure term, the velocity -u of the mirror cell
-// (halfway no-slip), and no donor flux.
+// other two axes.  The sweep, the tiles and the order of the axes are those of
+// k_stream_rows: z between lanes, y through LDS (twelve sums and the five
+// values that the y faces need, double buffered), x in registers over three
+// slabs.  The six face-neighbour terms (donor phase flux, viscous velocity
+// gradient) take the same way.
+// A position inside the tank walls is fetched from its mirror, the nearest
+// cell of the fluid box, and staged as the tank formulas use it: the gradient
+// with the mirrored components negated (capillary), no pressure term, the
+// velocity -u of the mirror cell (halfway no-slip), and no donor flux.
+// Bound by memory: 77 bytes a cell and the tile's halo.  Tiles of 4 x 64
+// cells with every quantity's 3 x 3 window read from LDS took 168 us at
+// 256x128x128, 406 at 450x150x90 and 90 at 24x20x16; 110, 182 and 6 now (with
+// twelve waves a block: sixteen spill 33 registers, 209 us at 256x128x128).
 struct ForceFetch {
-  float grad[3], phi, p, u[3], flux[3];
-  int wall;
+  float grad[3], phi, p, u[3], flux[3], volume, energy;
+  int flag;
 };
-__device__ __forceinline__ void fetch_force_cell(const icy3d_grid& g, int i, int j, int k, int moment_pressure,
-                                                 ForceFetch& f) {
-  const int b = g.boundary;
-  const int ci = min(max(i, b), g.nx - b - 1), cj = min(max(j, b), g.ny - b - 1), ck = min(max(k, b), g.nz - b - 1);
-  f.wall = (ci != i) | ((cj != j) << 1) | ((ck != k) << 2);
-  i = ci;
-  j = cj;
-  k = ck;
-  const size_t N = cells(g);
-  const int n = lin(g, i, j, k);
-#pragma unroll
-  for (int e = 0; e < 3; ++e) {
-    f.grad[e] = g.grad[e * N + n];
-    f.u[e] = g.u[e * N + n];
-    f.flux[e] = g.flux[e * N + n];
-  }
-  f.phi = g.phi[n];
-  f.p = moment_pressure ? g.home[n] : g.pressure[n];
-}
-__device__ __forceinline__ void stage_force_cell(const icy3d_grid& g, float (*sq)[kForceSlab], int t, int moment_pressure,
-                                                 const ForceFetch& f) {
-  const float gx = (f.wall & 1) ? -f.grad[0] : f.grad[0];
-  const float gy = (f.wall & 2) ? -f.grad[1] : f.grad[1];
-  const float gz = (f.wall & 4) ? -f.grad[2] : f.grad[2];
-  sq[0][t] = gy * gy + gz * gz;
-  sq[1][t] = gx * gx + gz * gz;
-  sq[2][t] = gx * gx + gy * gy;
-  sq[3][t] = gx * gy;
-  sq[4][t] = gx * gz;
-  sq[5][t] = gy * gz;
-  const float rho = density(g, f.phi);
-  if (f.wall) {
-    sq[6][t] = 0.0f;
-    sq[7][t] = 0.0f;
-  } else if (moment_pressure) {
-    sq[6][t] = f.p;
-    sq[7][t] = f.p * rho;
-  } else {
-    sq[6][t] = 3.0f * f.p / rho;
-    sq[7][t] = 3.0f * f.p;
-  }
-#pragma unroll
-  for (int e = 0; e < 3; ++e) {
-    sq[kU + e][t] = f.wall ? -f.u[e] : f.u[e];
-    sq[kFlux + e][t] = f.flux[e];
-  }
-  sq[kPhi][t] = f.phi;
-  sq[kWall][t] = f.wall ? 1.0f : 0.0f;
-}
-struct SlabParts {
-  float px[5], qy[5], qz[5];  // D_x parts of Ax Bxy Bxz X1 X2; D_y of Ay Bxy Byz X1 X2; D_z of Az Bxz Byz X1 X2
-};
-__device__ __forceinline__ void yz_parts(const float* q, int base, float& P, float& Qy, float& Qz) {
-  const float sixth = 1.0f / 6.0f;
-  float sz[3], dz[3];
-#pragma unroll
-  for (int r = 0; r < 3; ++r) {
-    const float a = q[base + r * kForceHK], b = q[base + r * kForceHK + 1], c = q[base + r * kForceHK + 2];
-    sz[r] = (a + 4.0f * b + c) * sixth;
-    dz[r] = (c - a) * sixth;
-  }
-  P = (sz[0] + 4.0f * sz[1] + sz[2]) * sixth;
-  Qy = (sz[2] - sz[0]) * sixth;
-  Qz = (dz[0] + 4.0f * dz[1] + dz[2]) * sixth;
-}
-__device__ __forceinline__ SlabParts slab_parts(const float (*sq)[kForceSlab], int base) {
-  SlabParts r;
-  float P, Qy, Qz;
-  yz_parts(sq[0], base, P, Qy, Qz);  // Ax: D_x
-  r.px[0] = P;
-  yz_parts(sq[1], base, P, Qy, Qz);  // Ay: D_y
-  r.qy[0] = Qy;
-  yz_parts(sq[2], base, P, Qy, Qz);  // Az: D_z
-  r.qz[0] = Qz;
-  yz_parts(sq[3], base, P, Qy, Qz);  // Bxy: D_x, D_y
-  r.px[1] = P;
-  r.qy[1] = Qy;
-  yz_parts(sq[4], base, P, Qy, Qz);  // Bxz: D_x, D_z
-  r.px[2] = P;
-  r.qz[1] = Qz;
-  yz_parts(sq[5], base, P, Qy, Qz);  // Byz: D_y, D_z
-  r.qy[2] = Qy;
-  r.qz[2] = Qz;
-  yz_parts(sq[6], base, P, Qy, Qz);  // X1
-  r.px[3] = P;
-  r.qy[3] = Qy;
-  r.qz[3] = Qz;
-  yz_parts(sq[7], base, P, Qy, Qz);  // X2
-  r.px[4] = P;
-  r.qy[4] = Qy;
-  r.qz[4] = Qz;
-  return r;
-}
-// Own-column values carried between slabs.
+// Own-column values of a slab's cell, kept while the slabs after it pass.
 struct ColumnCell {
-  float u[3], flux_x, phi, wall;
-};
-// Terms of the y and z faces, formed while the cell's own slab is in LDS:
-// the donor-flux force of those four faces and the y/z derivatives of u.
-struct FaceTerms {
-  float f[3], dudy[3], dudz[3];
+  float u[3], flux_x, phi;
 };
 // Donor phase-flux momentum term of one face (simulator.py:499-519).
 __device__ __forceinline__ void face_flux(const icy3d_grid& g, float d, float flux_own, float flux_nb, float rho,
@@ -1150,150 +1014,222 @@ __device__ __forceinline__ void face_flux(const icy3d_grid& g, float d, float fl
   f[1] -= d * fl[1];
   f[2] -= d * fl[2];
 }
-__device__ __forceinline__ FaceTerms face_terms(const icy3d_grid& g, const float (*sq)[kForceSlab], int centre,
-                                                int with_flux) {
-  FaceTerms t = {{0.0f, 0.0f, 0.0f}, {0.0f, 0.0f, 0.0f}, {0.0f, 0.0f, 0.0f}};
-  const float u_own[3] = {sq[kU][centre], sq[kU + 1][centre], sq[kU + 2][centre]};
-  const float rho = density(g, sq[kPhi][centre]);
-  // faces -y, +y, -z, +z
-  const int off[4] = {-kForceHK, kForceHK, -1, 1};
-#pragma unroll
-  for (int a = 0; a < 2; ++a) {
-    const int comp = 1 + a;  // flux component along y or z
-    const float flux_own = sq[kFlux + comp][centre];
-    float un[2][3];
-#pragma unroll
-    for (int side = 0; side < 2; ++side) {
-      const int m = centre + off[2 * a + side];
-#pragma unroll
-      for (int e = 0; e < 3; ++e) un[side][e] = sq[kU + e][m];
-      if (with_flux && sq[kWall][m] == 0.0f)
-        face_flux(g, side == 0 ? -1.0f : 1.0f, flux_own, sq[kFlux + comp][m], rho, sq[kPhi][m], u_own, un[side], t.f);
-    }
+
+__global__ void __launch_bounds__(kForceThreads) k_forces_rows(icy3d_grid g, StreamTiles T, int with_flux,
+                                                                int moment_pressure) {
+  __shared__ float4 quad[2][4][sweep_cells(kForceThreads)];
+  __shared__ float single[2][sweep_cells(kForceThreads)];
+  const size_t N = cells(g);
+  const int L = T.K + 2, lane = threadIdx.x & 63, b = g.boundary;
+  const int tile_k = (int)blockIdx.x % T.tiles_k, tile_j = (int)blockIdx.x / T.tiles_k % T.tiles_j;
+  const int x0 = (int)blockIdx.x / T.tiles_k / T.tiles_j * T.X, x1 = min(x0 + T.X, g.nx);
+  const int t = (int)(threadIdx.x >> 6) * kWaveCells + lane - 1;
+  const int row = t < 0 ? 0 : t / L, col = t < 0 ? 0 : t - row * L;
+  const int j = tile_j * T.J - 1 + row, k = tile_k * T.K - 1 + col;
+  const bool sends = lane >= 1 && lane <= kWaveCells && row < T.J + 2;
+  const bool owned = t >= 0 && sends && row >= 1 && row <= T.J && col >= 1 && col <= T.K && j < g.ny && k < g.nz;
+  const int cj = min(max(j, b), g.ny - b - 1), ck = min(max(k, b), g.nz - b - 1);
+  const unsigned plane = (unsigned)(g.ny * g.nz), own_plane = owned ? (unsigned)(j * g.nz + k) : 0u;
+  const unsigned clamped = (unsigned)(cj * g.nz + ck);
+  const bool wall_y = cj != j, wall_z = ck != k;
+  // Whether the neighbours across the y and z faces are inside the walls.
+  const bool open_y[2] = {j - 1 >= b, j + 1 < g.ny - b}, open_z[2] = {k - 1 >= b, k + 1 < g.nz - b};
+  const float* pressure = moment_pressure ? g.home : g.pressure;
+
+  ForceFetch f;
+  auto fetch = [&](int s) __attribute__((always_inline)) {
+    const unsigned o = 4u * ((unsigned)min(max(s, b), g.nx - b - 1) * plane + clamped);
 #pragma unroll
     for (int e = 0; e < 3; ++e) {
-      const float d = 0.5f * (un[1][e] - un[0][e]);
-      if (a == 0) t.dudy[e] = d;
-      else t.dudz[e] = d;
+      f.grad[e] = plane_get(g.grad + e * N, o);
+      f.u[e] = plane_get(g.u + e * N, o);
+      f.flux[e] = plane_get(g.flux + e * N, o);
     }
-  }
-  return t;
-}
+    f.phi = plane_get(g.phi, o);
+    f.p = plane_get(pressure, o);
+    f.flag = -1;
+    f.volume = f.energy = 0.0f;
+    if (owned && s >= x0 && s < x1) {
+      const unsigned n = (unsigned)s * plane + own_plane;
+      f.flag = g.flag[n];
+      f.volume = plane_get(g.water_volume, 4u * n);
+      f.energy = plane_get(g.water_energy, 4u * n);
+    }
+  };
+  fetch(x0 - 1);
+  const float sixth = 1.0f / 6.0f, kcap = 4.5f * g.sigma * g.width;
+  // x differences (capillary of f_x, f_y, f_z, then the pressure fields): the
+  // last two slabs; x averages (the same, and the pressure fields along y and
+  // z): the last two slabs.
+  float diff_a[5] = {}, diff_b[5] = {}, mean_a[7] = {}, mean_b[7] = {};
+  ColumnCell col_a = {}, col_b = {};
+  // The last slab's cell: y and z face terms, its gradient, temperature, flag.
+  float face_f[3] = {}, du_dy[3] = {}, du_dz[3] = {}, grad_b[3] = {}, temperature_b = 0.0f;
+  int flag_b = -1;
 
-__global__ void __launch_bounds__(kForceJ* kForceK) k_forces_tiled(icy3d_grid g, int with_flux, int moment_pressure) {
-  __shared__ float sq[kForceQ][kForceSlab];
-  const size_t N = cells(g);
-  const int tk = threadIdx.x % kForceK, tj = threadIdx.x / kForceK;
-  const int k0 = blockIdx.x * kForceK, j0 = blockIdx.y * kForceJ, x0 = blockIdx.z * kForceX;
-  const int x_end = min(x0 + kForceX, g.nx);
-  const int j = j0 + tj, k = k0 + tk;
-  const bool mine = j < g.ny && k < g.nz;
-  const int base = tj * kForceHK + tk;            // top-left of the thread's 3x3 (j, k) window
-  const int centre = base + kForceHK + 1;
-  ForceFetch fetched[kForceRounds];
+  for (int s = x0 - 1; s <= x1; ++s) {
+    const int buffer = s & 1;
+    const bool wall_x = s < b || s >= g.nx - b, wall = wall_x || wall_y || wall_z;
+    const float gx = wall_x ? -f.grad[0] : f.grad[0], gy = wall_y ? -f.grad[1] : f.grad[1];
+    const float gz = wall_z ? -f.grad[2] : f.grad[2];
+    const float rho = density(g, f.phi);
+    ColumnCell now;
 #pragma unroll
-  for (int r = 0; r < kForceRounds; ++r) {
-    const int t = threadIdx.x + r * blockDim.x;
-    if (t < kForceSlab) fetch_force_cell(g, x0 - 1, j0 - 1 + t / kForceHK, k0 - 1 + t % kForceHK, moment_pressure, fetched[r]);
-  }
-  SlabParts prev2 = {}, prev1 = {};
-  ColumnCell col_m1 = {}, col_0 = {};
-  FaceTerms faces_0 = {};
-  const float kcap = 4.5f * g.sigma * g.width;
-  for (int s = x0 - 1; s <= x_end; ++s) {
-    __syncthreads();
+    for (int e = 0; e < 3; ++e) now.u[e] = wall ? -f.u[e] : f.u[e];
+    now.flux_x = f.flux[0];
+    now.phi = f.phi;
+    const float flux_y = f.flux[1], flux_z = f.flux[2];
+    const float temperature = water_temperature_of(g, f.volume, f.energy);
+    const int flag = f.flag;
+    float p1 = moment_pressure ? f.p : 3.0f * f.p / rho, p2 = moment_pressure ? f.p * rho : 3.0f * f.p;
+    if (wall) p1 = p2 = 0.0f;
+    // z sums and differences (6 times): of Ax, Ay, Bxy, Bxz, Byz, X1, X2 the
+    // average, of Az, Bxz, Byz, X1, X2 the difference.
+    const float stage[8] = {gy * gy + gz * gz, gx * gx + gz * gz, gx * gy, gx * gz, gy * gz, p1, p2, gx * gx + gy * gy};
+    float below[8], above[8];
 #pragma unroll
-    for (int r = 0; r < kForceRounds; ++r) {
-      const int t = threadIdx.x + r * blockDim.x;
-      if (t < kForceSlab) stage_force_cell(g, sq, t, moment_pressure, fetched[r]);
+    for (int q = 0; q < 8; ++q) {
+      below[q] = from_below(stage[q]);
+      above[q] = from_above(stage[q]);
     }
-    if (s < x_end) {
+    float zs[7], zd[5];
 #pragma unroll
-      for (int r = 0; r < kForceRounds; ++r) {
-        const int t = threadIdx.x + r * blockDim.x;
-        if (t < kForceSlab)
-          fetch_force_cell(g, s + 1, j0 - 1 + t / kForceHK, k0 - 1 + t % kForceHK, moment_pressure, fetched[r]);
+    for (int q = 0; q < 7; ++q) zs[q] = below[q] + above[q] + 4.0f * stage[q];
+    zd[0] = above[7] - below[7];
+#pragma unroll
+    for (int q = 1; q < 5; ++q) zd[q] = above[q + 2] - below[q + 2];
+    // z faces.
+    float ff[3] = {0.0f, 0.0f, 0.0f}, dz_u[3];
+    {
+      float un[2][3];
+#pragma unroll
+      for (int e = 0; e < 3; ++e) {
+        un[0][e] = from_below(now.u[e]);
+        un[1][e] = from_above(now.u[e]);
+        dz_u[e] = 0.5f * (un[1][e] - un[0][e]);
       }
+      const float flux_n[2] = {from_below(flux_z), from_above(flux_z)}, phi_n[2] = {from_below(now.phi), from_above(now.phi)};
+      if (with_flux)
+#pragma unroll
+        for (int side = 0; side < 2; ++side)
+          if (open_z[side])
+            face_flux(g, side == 0 ? -1.0f : 1.0f, flux_z, flux_n[side], rho, phi_n[side], now.u, un[side], ff);
     }
+    if (sends) {
+      quad[buffer][0][t] = make_float4(zs[0], zs[1], zs[2], zs[3]);
+      quad[buffer][1][t] = make_float4(zs[4], zs[5], zs[6], zd[0]);
+      quad[buffer][2][t] = make_float4(zd[1], zd[2], zd[3], zd[4]);
+      quad[buffer][3][t] = make_float4(now.u[0], now.u[1], now.u[2], flux_y);
+      single[buffer][t] = now.phi;
+    }
+    if (s < x1) fetch(s + 1);
     __syncthreads();
-    const SlabParts cur = slab_parts(sq, base);
-    ColumnCell col_p1;
+    if (owned) {
+      // y averages of Ax, Bxy, Bxz, X1, X2 (for the x differences), and what
+      // the x averages take: y differences and the y averages of the z ones.
+      float diff[5], mean[7], dy_u[3];
+      {
+        const float4 m0 = quad[buffer][0][t - L], p0 = quad[buffer][0][t + L];
+        const float4 m1 = quad[buffer][1][t - L], p1v = quad[buffer][1][t + L];
+        const float4 m2 = quad[buffer][2][t - L], p2v = quad[buffer][2][t + L];
+        diff[0] = m0.x + p0.x + 4.0f * zs[0];
+        diff[1] = m0.z + p0.z + 4.0f * zs[2];
+        diff[2] = m0.w + p0.w + 4.0f * zs[3];
+        diff[3] = m1.y + p1v.y + 4.0f * zs[5];
+        diff[4] = m1.z + p1v.z + 4.0f * zs[6];
+        const float az = m1.w + p1v.w + 4.0f * zd[0];
+        const float bxz = m2.x + p2v.x + 4.0f * zd[1], byz = m2.y + p2v.y + 4.0f * zd[2];
+        const float byz_y = p1v.x - m1.x;
+        mean[0] = -((p0.z - m0.z) + bxz);
+        mean[1] = (p0.y - m0.y) - byz;
+        mean[2] = az - byz_y;
+        mean[3] = p1v.y - m1.y;
+        mean[4] = p1v.z - m1.z;
+        mean[5] = m2.z + p2v.z + 4.0f * zd[3];
+        mean[6] = m2.w + p2v.w + 4.0f * zd[4];
+      }
+      {
+        const float4 m3 = quad[buffer][3][t - L], p3 = quad[buffer][3][t + L];
+        const float um[3] = {m3.x, m3.y, m3.z}, up[3] = {p3.x, p3.y, p3.z};
 #pragma unroll
-    for (int e = 0; e < 3; ++e) col_p1.u[e] = sq[kU + e][centre];
-    col_p1.flux_x = sq[kFlux][centre];
-    col_p1.phi = sq[kPhi][centre];
-    col_p1.wall = sq[kWall][centre];
-    const FaceTerms faces_p1 = face_terms(g, sq, centre, with_flux);
-    const int x = s - 1;
-    if (x >= x0 && mine) {
-      const int n = lin(g, x, j, k);
-      const int8_t flag = g.flag[n];
-      if (flag == 0 || flag == 1) {  // bulk and tank-adjacent cells
-        const float sixth = 1.0f / 6.0f;
-        const float phi = col_0.phi, rho = density(g, phi);
-        float f[3] = {faces_0.f[0], (rho - g.ref_density[j]) * g.gravity_y + faces_0.f[1], faces_0.f[2]};
-        f[1] -= fmaxf(0.0f, 2.0f * phi - 1.0f) * g.expansion * (water_temperature(g, n) - g.water_t0) * g.gravity_y;
-        // x parts: D_x = (P(x+1) - P(x-1)) / 6; y, z parts: S_x = (Q(x-1) + 4 Q(x) + Q(x+1)) / 6
-        float dx[5], dy[5], dz[5];
-#pragma unroll
-        for (int m = 0; m < 5; ++m) {
-          dx[m] = (cur.px[m] - prev2.px[m]) * sixth;
-          dy[m] = (prev2.qy[m] + 4.0f * prev1.qy[m] + cur.qy[m]) * sixth;
-          dz[m] = (prev2.qz[m] + 4.0f * prev1.qz[m] + cur.qz[m]) * sixth;
+        for (int e = 0; e < 3; ++e) dy_u[e] = 0.5f * (up[e] - um[e]);
+        if (with_flux) {
+          if (open_y[0]) face_flux(g, -1.0f, flux_y, m3.w, rho, single[buffer][t - L], now.u, um, ff);
+          if (open_y[1]) face_flux(g, 1.0f, flux_y, p3.w, rho, single[buffer][t + L], now.u, up, ff);
         }
+      }
+      if (s > x0 && (flag_b == 0 || flag_b == 1)) {  // the cell s - 1
+        const unsigned o = 4u * ((unsigned)(s - 1) * plane + own_plane);
+        const float phi = col_b.phi, rho_b = density(g, phi);
+        constexpr float kScale = 1.0f / 216.0f;
+        float dx[5], avg[7];
+#pragma unroll
+        for (int q = 0; q < 5; ++q) dx[q] = (diff[q] - diff_a[q]) * kScale;
+#pragma unroll
+        for (int q = 0; q < 7; ++q) avg[q] = (mean_a[q] + 4.0f * mean_b[q] + mean[q]) * kScale;
+        float force[3] = {face_f[0], (rho_b - g.ref_density[j]) * g.gravity_y + face_f[1], face_f[2]};
+        force[1] -= fmaxf(0.0f, 2.0f * phi - 1.0f) * g.expansion * (temperature_b - g.water_t0) * g.gravity_y;
         if (g.sigma > 0.0f) {
-          f[0] += kcap * (dx[0] - dy[1] - dz[1]);
-          f[1] += kcap * (dy[0] - dx[1] - dz[2]);
-          f[2] += kcap * (dz[0] - dx[2] - dy[2]);
+          force[0] += kcap * (dx[0] + avg[0]);
+          force[1] += kcap * (avg[1] - dx[1]);
+          force[2] += kcap * (avg[2] - dx[2]);
         }
         if (with_flux) {
-          if (col_m1.wall == 0.0f) face_flux(g, -1.0f, col_0.flux_x, col_m1.flux_x, rho, col_m1.phi, col_0.u, col_m1.u, f);
-          if (col_p1.wall == 0.0f) face_flux(g, 1.0f, col_0.flux_x, col_p1.flux_x, rho, col_p1.phi, col_0.u, col_p1.u, f);
+          if (s - 2 >= b) face_flux(g, -1.0f, col_b.flux_x, col_a.flux_x, rho_b, col_a.phi, col_b.u, col_a.u, force);
+          if (s < g.nx - b) face_flux(g, 1.0f, col_b.flux_x, now.flux_x, rho_b, now.phi, col_b.u, now.u, force);
         }
-        // home.py:127-197
-        const float inv_rho = 1.0f / rho;
-        float acc[3] = {f[0] / rho, f[1] / rho, f[2] / rho};
-        acc[0] += dx[3] - dx[4] * inv_rho;
-        acc[1] += dy[3] - dy[4] * inv_rho;
-        acc[2] += dz[3] - dz[4] * inv_rho;
+        const float inv_rho = 1.0f / rho_b;
+        float acc[3] = {force[0] / rho_b + dx[3] - dx[4] * inv_rho, force[1] / rho_b + avg[3] - avg[4] * inv_rho,
+                        force[2] / rho_b + avg[5] - avg[6] * inv_rho};
         const float dr = 1.0f - g.rho_air;
-        const float gr[3] = {g.grad[n] * dr, g.grad[N + n] * dr, g.grad[2 * N + n] * dr};
+        const float gr[3] = {grad_b[0] * dr, grad_b[1] * dr, grad_b[2] * dr};
         if (gr[0] * gr[0] + gr[1] * gr[1] + gr[2] * gr[2] > 0.0f) {
           float G[3][3];
 #pragma unroll
           for (int e = 0; e < 3; ++e) {
-            G[e][0] = 0.5f * (col_p1.u[e] - col_m1.u[e]);
-            G[e][1] = faces_0.dudy[e];
-            G[e][2] = faces_0.dudz[e];
+            G[e][0] = 0.5f * (now.u[e] - col_a.u[e]);
+            G[e][1] = du_dy[e];
+            G[e][2] = du_dz[e];
           }
-          const float coef = lattice_nu(g, n) / rho;
+          const float coef =
+              mixture_nu(phi, temperature_b, g.rho_water_si, g.rho_air_si, g.mu_air) * g.nu_scale / rho_b;
 #pragma unroll
           for (int e = 0; e < 3; ++e)
             acc[e] += coef * ((G[e][0] + G[0][e]) * gr[0] + (G[e][1] + G[1][e]) * gr[1] + (G[e][2] + G[2][e]) * gr[2]);
         }
 #pragma unroll
         for (int e = 0; e < 3; ++e) {
-          g.force[e * N + n] = f[e];
-          g.accel[e * N + n] = acc[e];
+          plane_set(g.force + e * N, o, force[e]);
+          plane_set(g.accel + e * N, o, acc[e]);
         }
       }
+#pragma unroll
+      for (int q = 0; q < 5; ++q) {
+        diff_a[q] = diff_b[q];
+        diff_b[q] = diff[q];
+      }
+#pragma unroll
+      for (int q = 0; q < 7; ++q) {
+        mean_a[q] = mean_b[q];
+        mean_b[q] = mean[q];
+      }
+#pragma unroll
+      for (int e = 0; e < 3; ++e) {
+        face_f[e] = ff[e];
+        du_dy[e] = dy_u[e];
+        du_dz[e] = dz_u[e];
+      }
     }
-    prev2 = prev1;
-    prev1 = cur;
-    col_m1 = col_0;
-    col_0 = col_p1;
-    faces_0 = faces_p1;
+    col_a = col_b;
+    col_b = now;
+    grad_b[0] = gx;
+    grad_b[1] = gy;
+    grad_b[2] = gz;
+    temperature_b = temperature;
+    flag_b = flag;
   }
 }
 
-__global__ void k_forces_interior(icy3d_grid g, int with_flux, int moment_pressure) {
-  int n = blockIdx.x * blockDim.x + threadIdx.x;
-  if (n >= (int)cells(g) || g.flag[n] != 0) return;
-  forces_cell<kInterior>(g, n, with_flux, moment_pressure);
-}
-__global__ void k_forces_tank(icy3d_grid g, int with_flux, int moment_pressure) {
-  ICY_FOR_LIST(g.tank_cells, g.control->tank_count, n) forces_cell<kTank>(g, n, with_flux, moment_pressure);
-}
 // simulator.py:418-519 and home.py:127-197 for ice-adjacent cells, one lane
 // per link: capillary (fluid link or mirrored stress), product-rule pressure
 // term, donor phase-flux term (lanes 0..5) and the six neighbour velocities
@@ -1414,8 +1350,8 @@ __global__ void k_refill_forces(icy3d_grid g, Box box) {
   if (!(g.id[c.n] == -1 && g.prev_id[c.n] != -1)) return;
   const size_t N = cells(g);
   float f[3], a[3];
-  force_at<kGeneral>(g, c, false, f);
-  acceleration_at<kGeneral>(g, c, f, false, a);
+  force_at(g, c, false, f);
+  acceleration_at(g, c, f, false, a);
 #pragma unroll
   for (int e = 0; e < 3; ++e) {
     g.force[e * N + c.n] = f[e];
@@ -1430,8 +1366,8 @@ __global__ void k_generic_forces(icy3d_grid g, float* __restrict__ out) {
   float f[3] = {0, 0, 0}, a[3] = {0, 0, 0};
   if (g.id[n] == -1) {
     const Cell c = cell_of(g, n);
-    force_at<kGeneral>(g, c, true, f);
-    acceleration_at<kGeneral>(g, c, f, true, a);
+    force_at(g, c, true, f);
+    acceleration_at(g, c, f, true, a);
   }
 #pragma unroll
   for (int e = 0; e < 3; ++e) {
@@ -1592,11 +1528,6 @@ __device__ __forceinline__ void store_streamed(const icy3d_grid& g, float* __res
 // post-collision moments.  A cell whose nine links towards one z neighbour are
 // all missing and no others (the z walls, in every row) gets their sums in
 // closed form from its own z lines; every other pattern goes link by link.
-struct StreamTiles {
-  int J, K, X, tiles_j, tiles_k;
-};
-constexpr int kStreamThreads = 1024, kWaveCells = 62;
-constexpr int kStreamCells = kStreamThreads / 64 * kWaveCells;
 struct StreamFetch {
   float m[10], a[3], phi, volume, energy;
   int label, flag;
@@ -1604,30 +1535,13 @@ struct StreamFetch {
 struct Line3 {
   float up, dn, c;
 };
-// v of the previous / next lane of the wave.
-__device__ __forceinline__ float from_below(float v) {
-  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x138, 0xf, 0xf, true));
-}
-__device__ __forceinline__ float from_above(float v) {
-  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x130, 0xf, 0xf, true));
-}
-__device__ __forceinline__ int from_below(int v) { return __builtin_amdgcn_update_dpp(0, v, 0x138, 0xf, 0xf, true); }
-__device__ __forceinline__ int from_above(int v) { return __builtin_amdgcn_update_dpp(0, v, 0x130, 0xf, 0xf, true); }
-// An element of a plane at a byte offset below 2^31 (a grid has fewer than
-// 2^27 cells): a uniform base and a 32-bit lane offset.
-__device__ __forceinline__ float plane_get(const float* base, unsigned offset) {
-  return *reinterpret_cast<const float*>(reinterpret_cast<const char*>(base) + offset);
-}
-__device__ __forceinline__ void plane_set(float* base, unsigned offset, float v) {
-  *reinterpret_cast<float*>(reinterpret_cast<char*>(base) + offset) = v;
-}
 
 template <bool Fused>
 __global__ void __launch_bounds__(kStreamThreads) k_stream_rows(icy3d_grid g, StreamTiles T) {
   // The y pass's values of a slab: up then dn, nine each, as 4 + 4 + 1 words.
-  __shared__ float4 quad[2][4][kStreamCells];
-  __shared__ float single[2][2][kStreamCells];
-  __shared__ uint8_t links[2][kStreamCells];  // bits 0, 1, 2: fluid at k - 1, k, k + 1
+  __shared__ float4 quad[2][4][sweep_cells(kStreamThreads)];
+  __shared__ float single[2][2][sweep_cells(kStreamThreads)];
+  __shared__ uint8_t links[2][sweep_cells(kStreamThreads)];  // bits 0, 1, 2: fluid at k - 1, k, k + 1
   if (Fused && blockIdx.x == 0)
     for (int t = threadIdx.x; t < ICY3D_MAX_BODIES * 6; t += blockDim.x) (&g.control->loads[0][0])[t] = 0.0f;
   const size_t N = cells(g);
@@ -2175,39 +2089,23 @@ int launch_gradients_list(const icy3d_grid& g, const BoxList& L, hipStream_t s) 
 int launch_gradients(const icy3d_grid& g, const Box& b, bool, hipStream_t s) {
   return launch_gradients_list(g, one_box(g, b), s);
 }
-int launch_forces(const icy3d_grid& g, int with_flux, int moment_pressure, hipStream_t s) {
-  const dim3 tiles((g.nz + kForceK - 1) / kForceK, (g.ny + kForceJ - 1) / kForceJ, (g.nx + kForceX - 1) / kForceX);
-  k_forces_tiled<<<tiles, kForceJ * kForceK, 0, s>>>(g, with_flux, moment_pressure);  // bulk and tank cells
-  k_forces_general<<<kForceListBlocks, kBlock, 0, s>>>(g, with_flux, moment_pressure);
-  ICY_LAUNCH_CHECK();
-  return 0;
-}
-int launch_recover(const icy3d_grid& g, int parity, int recover_flow, hipStream_t s) {
-  bool scan = recover_flow && g.check_stability;
-  const unsigned blocks = icy_blocks(grid_cells(g));
-  if ((int)blocks > g.partials_capacity) return ICY3D_ERR_ARGUMENT;
-  if (scan && 3 * (int)blocks > g.partials_capacity) return ICY3D_ERR_ARGUMENT;
-  k_recover_phase<<<blocks, kBlock, 0, s>>>(g, parity, recover_flow);
-  k_fold_recovery<<<1, kFinishThreads, 0, s>>>(g, (int)blocks, scan ? 1 : 0);
-  ICY_LAUNCH_CHECK();
-  return 0;
-}
-// The stream's tiles.  z is cut into as few tiles as leave ten rows a block
+// The row sweeps' tiles.  z is cut into as few tiles as leave ten rows a block
 // (eight of them its own).  Then the rows and slabs a block owns: a block
 // takes a CU to itself, a slab costs it a fixed latency and a time for each
 // wave, and it stages two rows and two slabs more than it owns, so the
 // cheapest cut is searched over the row tiles that fit and the slab chunks
 // that fill whole rounds of the 256 CUs (kSlabLatency, kWaveTime: microseconds
 // measured at 24x20x16 and 256x128x128).
-StreamTiles stream_tiles(const icy3d_grid& g) {
+StreamTiles stream_tiles(const icy3d_grid& g, int threads) {
   constexpr int kCus = 256;
   constexpr double kSlabLatency = 1.6, kWaveTime = 0.24;
+  const int cells_most = sweep_cells(threads);
   StreamTiles best = {};
   int tiles_k = 1;
-  while (10 * ((g.nz + tiles_k - 1) / tiles_k + 2) > kStreamCells) ++tiles_k;
+  while (10 * ((g.nz + tiles_k - 1) / tiles_k + 2) > cells_most) ++tiles_k;
   const int K = (g.nz + tiles_k - 1) / tiles_k, L = K + 2;
   tiles_k = (g.nz + K - 1) / K;
-  const int most = kStreamCells / L - 2;
+  const int most = cells_most / L - 2;
   double least = 0.0;
   for (int tiles_j = (g.ny + most - 1) / most; tiles_j <= g.ny; ++tiles_j) {
     const int J = (g.ny + tiles_j - 1) / tiles_j, waves = ((J + 2) * L + kWaveCells - 1) / kWaveCells;
@@ -2224,12 +2122,33 @@ StreamTiles stream_tiles(const icy3d_grid& g) {
   }
   return best;
 }
+unsigned stream_blocks(const icy3d_grid& g, const StreamTiles& T) {
+  return (unsigned)(T.tiles_k * T.tiles_j * ((g.nx + T.X - 1) / T.X));
+}
+unsigned stream_threads(const StreamTiles& T) {
+  return (unsigned)(((T.J + 2) * (T.K + 2) + kWaveCells - 1) / kWaveCells * 64);
+}
+int launch_forces(const icy3d_grid& g, int with_flux, int moment_pressure, hipStream_t s) {
+  const StreamTiles T = stream_tiles(g, kForceThreads);
+  k_forces_rows<<<stream_blocks(g, T), stream_threads(T), 0, s>>>(g, T, with_flux, moment_pressure);  // bulk and tank cells
+  k_forces_general<<<kForceListBlocks, kBlock, 0, s>>>(g, with_flux, moment_pressure);
+  ICY_LAUNCH_CHECK();
+  return 0;
+}
+int launch_recover(const icy3d_grid& g, int parity, int recover_flow, hipStream_t s) {
+  bool scan = recover_flow && g.check_stability;
+  const unsigned blocks = icy_blocks(grid_cells(g));
+  if ((int)blocks > g.partials_capacity) return ICY3D_ERR_ARGUMENT;
+  if (scan && 3 * (int)blocks > g.partials_capacity) return ICY3D_ERR_ARGUMENT;
+  k_recover_phase<<<blocks, kBlock, 0, s>>>(g, parity, recover_flow);
+  k_fold_recovery<<<1, kFinishThreads, 0, s>>>(g, (int)blocks, scan ? 1 : 0);
+  ICY_LAUNCH_CHECK();
+  return 0;
+}
 template <bool Fused>
 void launch_stream_rows(const icy3d_grid& g, hipStream_t s) {
-  const StreamTiles T = stream_tiles(g);
-  const unsigned blocks = (unsigned)(T.tiles_k * T.tiles_j * ((g.nx + T.X - 1) / T.X));
-  const int waves = ((T.J + 2) * (T.K + 2) + kWaveCells - 1) / kWaveCells;
-  k_stream_rows<Fused><<<blocks, waves * 64, 0, s>>>(g, T);
+  const StreamTiles T = stream_tiles(g, kStreamThreads);
+  k_stream_rows<Fused><<<stream_blocks(g, T), stream_threads(T), 0, s>>>(g, T);
 }
 int launch_stream(const icy3d_grid& g, hipStream_t s) {
   if ((int)(kListBlocks * kLoadSlots) > g.partials_capacity) return ICY3D_ERR_ARGUMENT;
