@@ -275,6 +275,13 @@ int icy3d_apply_thermal_fluxes(const icy3d_grid* g, float dt, int advect, void* 
  * from the grid's planes); on return the caller swaps them with
  * water_volume / water_energy.  energy_flux and volume_flux are not written. */
 int icy3d_advect_water(const icy3d_grid* g, float dt, float* volume_out, float* energy_out, void* stream);
+/* icy3d_synchronize_water, one advection substep of dt (icy3d_thermal_fluxes
+ * and icy3d_apply_thermal_fluxes with advect = 1) and icy3d_synchronize_water
+ * again (thermal.py:98-184) in one pass: the remapped water goes to
+ * volume_out / energy_out ([N] each, distinct from the grid's planes), which
+ * the caller swaps with water_volume / water_energy on return; the remap
+ * energy takes both remaps' sums.  No intermediate plane is written. */
+int icy3d_remap_advect_remap(const icy3d_grid* g, float dt, float* volume_out, float* energy_out, void* stream);
 /* icy3d_thermal_fluxes then icy3d_apply_thermal_fluxes with advect = 0
  * (thermal.py:133-184, the conduction update) in one pass: the updated water
  * energy goes to energy_out ([N], distinct from water_energy), which the

@@ -939,33 +939,6 @@ __device__ void acceleration_at(const icy3d_grid& g, const Cell& c, const float 
 }
 
 // ---------------------------------------------------------------------------
-// Tiles of the row sweeps (k_forces_rows, k_stream_rows): J rows by K cells of
-// y and z, X slabs; the tile with its halo laid flat over the lanes, 62 cells
-// a wave.
-struct StreamTiles {
-  int J, K, X, tiles_j, tiles_k;
-};
-constexpr int kWaveCells = 62;
-constexpr int kStreamThreads = 1024, kForceThreads = 768;
-constexpr int sweep_cells(int threads) { return threads / 64 * kWaveCells; }
-// v of the previous / next lane of the wave.
-__device__ __forceinline__ float from_below(float v) {
-  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x138, 0xf, 0xf, true));
-}
-__device__ __forceinline__ float from_above(float v) {
-  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x130, 0xf, 0xf, true));
-}
-__device__ __forceinline__ int from_below(int v) { return __builtin_amdgcn_update_dpp(0, v, 0x138, 0xf, 0xf, true); }
-__device__ __forceinline__ int from_above(int v) { return __builtin_amdgcn_update_dpp(0, v, 0x130, 0xf, 0xf, true); }
-// An element of a plane at a byte offset below 2^31 (a grid has fewer than
-// 2^27 cells): a uniform base and a 32-bit lane offset.
-__device__ __forceinline__ float plane_get(const float* base, unsigned offset) {
-  return *reinterpret_cast<const float*>(reinterpret_cast<const char*>(base) + offset);
-}
-__device__ __forceinline__ void plane_set(float* base, unsigned offset, float v) {
-  *reinterpret_cast<float*>(reinterpret_cast<char*>(base) + offset) = v;
-}
-
 // Interior forces (simulator.py:418-519 and home.py:127-197 for cells of
 // flag 0 and 1: every link fluid or a tank wall).  The two 26-neighbour sums
 // factor with the D3Q27 weights w(c) = w1(cx) w1(cy) w1(cz):
@@ -2088,45 +2061,6 @@ int launch_gradients_list(const icy3d_grid& g, const BoxList& L, hipStream_t s) 
 }
 int launch_gradients(const icy3d_grid& g, const Box& b, bool, hipStream_t s) {
   return launch_gradients_list(g, one_box(g, b), s);
-}
-// The row sweeps' tiles.  z is cut into as few tiles as leave ten rows a block
-// (eight of them its own).  Then the rows and slabs a block owns: a block
-// takes a CU to itself, a slab costs it a fixed latency and a time for each
-// wave, and it stages two rows and two slabs more than it owns, so the
-// cheapest cut is searched over the row tiles that fit and the slab chunks
-// that fill whole rounds of the 256 CUs (kSlabLatency, kWaveTime: microseconds
-// measured at 24x20x16 and 256x128x128).
-StreamTiles stream_tiles(const icy3d_grid& g, int threads) {
-  constexpr int kCus = 256;
-  constexpr double kSlabLatency = 1.6, kWaveTime = 0.24;
-  const int cells_most = sweep_cells(threads);
-  StreamTiles best = {};
-  int tiles_k = 1;
-  while (10 * ((g.nz + tiles_k - 1) / tiles_k + 2) > cells_most) ++tiles_k;
-  const int K = (g.nz + tiles_k - 1) / tiles_k, L = K + 2;
-  tiles_k = (g.nz + K - 1) / K;
-  const int most = cells_most / L - 2;
-  double least = 0.0;
-  for (int tiles_j = (g.ny + most - 1) / most; tiles_j <= g.ny; ++tiles_j) {
-    const int J = (g.ny + tiles_j - 1) / tiles_j, waves = ((J + 2) * L + kWaveCells - 1) / kWaveCells;
-    const int yz = tiles_k * ((g.ny + J - 1) / J);
-    for (int rounds = 1; rounds <= 4; ++rounds) {
-      const int chunks = yz >= kCus * rounds ? 1 : kCus * rounds / yz;
-      const int X = (g.nx + chunks - 1) / chunks, blocks = yz * ((g.nx + X - 1) / X);
-      const double cost = (double)((blocks + kCus - 1) / kCus) * (X + 2) * (kSlabLatency + kWaveTime * waves);
-      if (best.J == 0 || cost < least) {
-        least = cost;
-        best = {J, K, X, (g.ny + J - 1) / J, tiles_k};
-      }
-    }
-  }
-  return best;
-}
-unsigned stream_blocks(const icy3d_grid& g, const StreamTiles& T) {
-  return (unsigned)(T.tiles_k * T.tiles_j * ((g.nx + T.X - 1) / T.X));
-}
-unsigned stream_threads(const StreamTiles& T) {
-  return (unsigned)(((T.J + 2) * (T.K + 2) + kWaveCells - 1) / kWaveCells * 64);
 }
 int launch_forces(const icy3d_grid& g, int with_flux, int moment_pressure, hipStream_t s) {
   const StreamTiles T = stream_tiles(g, kForceThreads);

@@ -248,6 +248,170 @@ __global__ void k_advect_water(icy3d_grid g, float dt, float* __restrict__ volum
   energy_out[n] = g.water_energy[n] - dt * de;
   volume_out[n] = g.water_volume[n] - dt * dv;
 }
+// The step's water update in one pass: remap to the phase field
+// (thermal.py:98-127), one advection substep (:133-184) and the remap again,
+// as k_synchronize_water_into, k_advect_water and k_synchronize_water_into
+// form them, face by face and in their order of adds.  A row sweep
+// (k_stream_rows): each cell is remapped once on load, z neighbours come from
+// the neighbour lanes, y neighbours through LDS, x neighbours from the slab
+// before; a cell that the advection empties takes the mean of its advected
+// neighbours, formed again from the planes (such cells are rare).  Bound by
+// memory: 37 bytes a cell and the halo, where the three passes moved 60 and
+// divided seven times a cell: 115 us at 256x128x128 with their two sums'
+// folds, 63 here.
+struct Water {
+  float volume, energy;
+};
+__device__ __forceinline__ Water remapped_cell(const icy3d_grid& g, int n) {
+  const float target = water_target(g, n);
+  return {target, remapped_energy(g, n, target)};
+}
+// The flux through the face from cell p to cell q along one axis (advect_face
+// on remapped cells; a dry or non-fluid cell has no volume).
+__device__ __forceinline__ Water face_of(const icy3d_grid& g, Water p, Water q, float up, float uq) {
+  Water f = {0.0f, 0.0f};
+  if (!(p.volume > 1e-30f && q.volume > 1e-30f)) return f;
+  const float speed = 0.5f * (up + uq) * g.velocity_m_s;
+  const Water donor = speed < 0.0f ? q : p;
+  f.volume = speed * fminf(1.0f, donor.volume / g.cell_volume) * (g.dx * g.dx);
+  f.energy = f.volume * donor.energy / donor.volume;
+  return f;
+}
+__device__ __forceinline__ Water advected_cell(const icy3d_grid& g, int i, int j, int k, float dt) {
+  const size_t N = cells(g);
+  const int n = lin(g, i, j, k);
+  const Water own = remapped_cell(g, n);
+  float de = 0.0f, dv = 0.0f;
+#pragma unroll 1
+  for (int face = 0; face < 6; ++face) {  // +x, -x, +y, -y, +z, -z
+    const int a = face >> 1, d = (face & 1) ? -1 : 1;
+    const int mi = i + (a == 0 ? d : 0), mj = j + (a == 1 ? d : 0), mk = k + (a == 2 ? d : 0);
+    if (!inside(g, mi, mj, mk)) continue;
+    const int m = lin(g, mi, mj, mk);
+    const Water other = remapped_cell(g, m);
+    const float u_own = g.u[a * N + n], u_other = g.u[a * N + m];
+    const Water f = d > 0 ? face_of(g, own, other, u_own, u_other) : face_of(g, other, own, u_other, u_own);
+    de += (float)d * f.energy;
+    dv += (float)d * f.volume;
+  }
+  return {own.volume - dt * dv, own.energy - dt * de};
+}
+__device__ __forceinline__ float advected_mean(const icy3d_grid& g, int i, int j, int k, float dt) {
+  float specific = 0.0f, total = 0.0f;
+#pragma unroll 1
+  for (int q = 0; q < 27; ++q) {
+    const int ni = i + cx(q), nj = j + cy(q), nk = k + cz(q);
+    if (!inside(g, ni, nj, nk)) continue;
+    const Water w = advected_cell(g, ni, nj, nk, dt);
+    if (w.volume > 1e-30f) {
+      specific += w.energy;
+      total += w.volume;
+    }
+  }
+  return total > 1e-30f ? specific / total : specific;
+}
+__global__ void __launch_bounds__(kWaterThreads)
+    k_water_rows(icy3d_grid g, StreamTiles T, float dt, float* __restrict__ volume_out,
+                 float* __restrict__ energy_out) {
+  __shared__ float row_v[2][sweep_cells(kWaterThreads)], row_e[2][sweep_cells(kWaterThreads)],
+      row_u[2][sweep_cells(kWaterThreads)];
+  const size_t N = cells(g);
+  const int L = T.K + 2, lane = threadIdx.x & 63;
+  const int tile_k = (int)blockIdx.x % T.tiles_k, tile_j = (int)blockIdx.x / T.tiles_k % T.tiles_j;
+  const int x0 = (int)blockIdx.x / T.tiles_k / T.tiles_j * T.X, x1 = min(x0 + T.X, g.nx);
+  const int t = (int)(threadIdx.x >> 6) * kWaveCells + lane - 1;
+  const int row = t < 0 ? 0 : t / L, col = t < 0 ? 0 : t - row * L;
+  const int j = tile_j * T.J - 1 + row, k = tile_k * T.K - 1 + col;
+  const bool present = t >= 0 && row < T.J + 2 && j >= 0 && j < g.ny && k >= 0 && k < g.nz;
+  const bool sends = lane >= 1 && lane <= kWaveCells && row < T.J + 2;
+  const bool owned = present && sends && row >= 1 && row <= T.J && col >= 1 && col <= T.K;
+  const unsigned in_plane = present ? (unsigned)(j * g.nz + k) : 0u, plane = (unsigned)(g.ny * g.nz);
+  int label = -2;
+  float phi = 0.0f, volume = 0.0f, energy = 0.0f, u[3] = {0.0f, 0.0f, 0.0f};
+  auto fetch = [&](int s) __attribute__((always_inline)) {
+    label = -2;
+    phi = volume = energy = 0.0f;
+    if (present && s >= 0 && s < g.nx) {
+      const unsigned n = (unsigned)s * plane + in_plane, o = 4u * n;
+      label = g.id[n];
+      phi = plane_get(g.phi, o);
+      volume = plane_get(g.water_volume, o);
+      energy = plane_get(g.water_energy, o);
+#pragma unroll
+      for (int e = 0; e < 3; ++e) u[e] = plane_get(g.u + e * N, o);
+    }
+  };
+  fetch(x0 - 1);
+  // The last slab's cell: its remapped water, x velocity, the flux through
+  // its lower x face and those through its y and z faces (upper, lower).
+  Water last = {0.0f, 0.0f}, x_in = {0.0f, 0.0f}, y_up = {0.0f, 0.0f}, y_lo = {0.0f, 0.0f}, z_up = {0.0f, 0.0f},
+        z_lo = {0.0f, 0.0f};
+  float last_u = 0.0f, first_change = 0.0f, second_change = 0.0f;
+  for (int s = x0 - 1; s <= x1; ++s) {
+    const int buffer = s & 1;
+    // The first remap, as water_target and remapped_energy.
+    Water now = {label == -1 && phi > 1e-3f ? phi * g.cell_volume : 0.0f, 0.0f};
+    if (now.volume > 0.0f) {
+      if (volume > 1e-30f) {
+#pragma clang fp contract(off)
+        now.energy = now.volume * (energy / volume);
+      } else {
+        now.energy = remapped_energy(g, s * (int)plane + (int)in_plane, now.volume);
+      }
+    }
+    if (owned && s >= x0 && s < x1) first_change += now.energy - energy;
+    const float ux = u[0], uy = u[1], uz = u[2];
+    if (s < x1) fetch(s + 1);
+    const Water below = {from_below(now.volume), from_below(now.energy)};
+    const Water above = {from_above(now.volume), from_above(now.energy)};
+    const Water z_lo_s = face_of(g, below, now, from_below(uz), uz), z_up_s = face_of(g, now, above, uz, from_above(uz));
+    if (sends) {
+      row_v[buffer][t] = now.volume;
+      row_e[buffer][t] = now.energy;
+      row_u[buffer][t] = uy;
+    }
+    __syncthreads();
+    if (owned) {
+      const Water y_lo_s = face_of(g, Water{row_v[buffer][t - L], row_e[buffer][t - L]}, now, row_u[buffer][t - L], uy);
+      const Water y_up_s = face_of(g, now, Water{row_v[buffer][t + L], row_e[buffer][t + L]}, uy, row_u[buffer][t + L]);
+      const Water x_face = face_of(g, last, now, last_u, ux);  // between the slabs s - 1 and s
+      if (s > x0) {
+        const float de = ((((x_face.energy - x_in.energy) + y_up.energy) - y_lo.energy) + z_up.energy) - z_lo.energy;
+        const float dv = ((((x_face.volume - x_in.volume) + y_up.volume) - y_lo.volume) + z_up.volume) - z_lo.volume;
+        const float e2 = last.energy - dt * de, v2 = last.volume - dt * dv, target = last.volume;
+        float out = 0.0f;
+        if (target > 0.0f) {
+#pragma clang fp contract(off)
+          out = target * (v2 > 1e-30f ? e2 / v2 : advected_mean(g, s - 1, j, k, dt));
+        }
+        second_change += out - e2;
+        const unsigned o = 4u * ((unsigned)(s - 1) * plane + in_plane);
+        plane_set(volume_out, o, target);
+        plane_set(energy_out, o, out);
+      }
+      x_in = x_face;
+      y_up = y_up_s;
+      y_lo = y_lo_s;
+      z_up = z_up_s;
+      z_lo = z_lo_s;
+    }
+    last = now;
+    last_u = ux;
+  }
+  const float first = block_sum(first_change), second = block_sum(second_change);
+  if (threadIdx.x == 0) {
+    g.partials[blockIdx.x] = first;
+    g.partials[gridDim.x + blockIdx.x] = second;
+  }
+}
+// Adds both remaps' sums to the remap energy, the first remap's first.
+__global__ void __launch_bounds__(kFinishThreads) k_fold_remaps(icy3d_grid g, int blocks) {
+  const float first = finish_total(g.partials, blocks), second = finish_total(g.partials + blocks, blocks);
+  if (threadIdx.x == 0) {
+    g.control->remap_energy += first;
+    g.control->remap_energy += second;
+  }
+}
 // thermal.py:186-206
 __global__ void k_measure_outflow(icy3d_grid g) {
   int n = blockIdx.x * blockDim.x + threadIdx.x;
@@ -640,6 +804,17 @@ int icy3d_apply_thermal_fluxes(const icy3d_grid* g, float dt, int advect, void* 
 int icy3d_advect_water(const icy3d_grid* g, float dt, float* volume_out, float* energy_out, void* stream) {
   if (!ok_grid(g) || !volume_out || !energy_out) return ICY3D_ERR_ARGUMENT;
   k_advect_water<<<icy_blocks(n_cells(*g)), kBlock, 0, (hipStream_t)stream>>>(*g, dt, volume_out, energy_out);
+  ICY_LAUNCH_CHECK();
+  return 0;
+}
+int icy3d_remap_advect_remap(const icy3d_grid* g, float dt, float* volume_out, float* energy_out, void* stream) {
+  if (!ok_grid(g) || !volume_out || !energy_out) return ICY3D_ERR_ARGUMENT;
+  hipStream_t s = (hipStream_t)stream;
+  const StreamTiles T = stream_tiles(*g, kWaterThreads);
+  const unsigned blocks = stream_blocks(*g, T);
+  if ((size_t)2 * blocks > (size_t)g->partials_capacity) return ICY3D_ERR_ARGUMENT;
+  k_water_rows<<<blocks, stream_threads(T), 0, s>>>(*g, T, dt, volume_out, energy_out);
+  k_fold_remaps<<<1, kFinishThreads, 0, s>>>(*g, (int)blocks);
   ICY_LAUNCH_CHECK();
   return 0;
 }

@@ -635,6 +635,11 @@ class IceFlow3D:
         (target_energy is not written)."""
         self._into_spare_water("synchronize_water_into")
 
+    def _remap_advect_remap(self, dt):
+        """``_synchronize_water_fused``, ``_advect_water(dt)`` and
+        ``_synchronize_water_fused`` in one pass into the spare water planes."""
+        self._into_spare_water("remap_advect_remap", float(dt))
+
     def _into_spare_water(self, name, *args):
         t, g = self._t, self._grid
         self._call(name, *args, ctypes.c_void_p(t["water_volume_next"].data_ptr()),
@@ -783,7 +788,8 @@ class IceFlow3D:
             self._raise_unstable(control.invalid_index)
         return float(control.maximum_speed)
 
-    def _refresh_geometry(self, phase_changed=True, current=None, cavity=(), full_gradients=False, guarded=False):
+    def _refresh_geometry(self, phase_changed=True, current=None, cavity=(), full_gradients=False, guarded=False,
+                          remap=True):
         """simulator.py:708-736 over the boxes of ``_raster_boxes`` (outside
         them the reference's passes change nothing); the refill loop reads
         one counter per sweep.  ``current``: the bodies' coverage boxes and
@@ -793,7 +799,8 @@ class IceFlow3D:
         ``guarded``: the refresh was queued before the host read the flow
         step's stability scan; if that scan found an invalid cell, the
         refresh kernels changed nothing, and None is returned with the box
-        history as it was."""
+        history as it was.  ``remap`` False: the caller remaps the water to
+        the refreshed phase itself, before anything reads it."""
         history, raster_full = self._box_history, self._raster_full
         boxes = self._raster_boxes(current, cavity)
         count, lo_p, hi_p = len(boxes[0]), boxes[0].ctypes.data, boxes[1].ctypes.data
@@ -844,9 +851,20 @@ class IceFlow3D:
         self._flags_valid = True
         if has_openings or covered:
             self._call("project_refill", self._parity, int3(lower), int3(v + 1 for v in upper))
-        if phase_changed or has_openings or covered:
+        if remap and (phase_changed or has_openings or covered):
             self._synchronize_water_fused()
         return Control.from_buffer_copy(control)
+
+    def _advance_water(self, speed_bound=None):
+        """The remap to the refreshed phase and thermal.py:208-226.  One
+        substep whose count needs no measurement is fused with the remaps
+        around it."""
+        th = self.config.thermal
+        if th.advection_enabled and speed_bound is not None and 3 * speed_bound <= th.max_courant_number:
+            self._remap_advect_remap(self.scales.dt_s)
+            return
+        self._synchronize_water_fused()
+        self._advance_advection(speed_bound)
 
     def _advance_advection(self, speed_bound=None):
         """thermal.py:208-226."""
@@ -988,13 +1006,13 @@ class IceFlow3D:
             # The geometry refresh's first control read follows the recovery's
             # stability scan in stream order.
             control = self._refresh_geometry(current=current, cavity=cavity, full_gradients=profile is None,
-                                             guarded=True)
+                                             guarded=True, remap=False)
             if control is None:
                 self._raise_if_unstable(saved_rigid, saved_rows, profile is None)
             speed_bound = None
             if self.config.check_stability:
                 speed_bound = float(control.maximum_speed)
-            self._advance_advection(speed_bound)
+            self._advance_water(speed_bound)
             self._thermal_pending += 1
             if self._thermal_pending >= self.config.thermal.update_interval_lbm_steps:
                 self._advance_conduction(self._thermal_pending * self.scales.dt_s)

@@ -36,3 +36,41 @@ def test_tiled_kernel_matches_oracle(kernel, shape):
     run(sim)
     for name in outputs:
         assert_close(getattr(sim, name).to_numpy(), getattr(ref, name).to_numpy(), 2e-5, f"{kernel}:{name}")
+
+
+@pytest.mark.parametrize("shape", SHAPES)
+def test_fused_water_update_equals_its_three_passes(shape):
+    """The step's remap, advection and remap in one pass give the water planes
+    and the remap energy of the three passes: the same expressions, with FMA
+    contraction chosen per kernel (2 FP32 ulps of scale; the remap energy's
+    sum over N cells in another order: sqrt(N) ulps of the largest energy for
+    the terms and 4 ulps of the sum for its two partial and two final adds).
+    The phase moves by a cell so that cells dry out and newly wet, and the
+    velocity is strong enough that the advection empties some."""
+    from tests.cases3d import restore_fields, snapshot_fields
+
+    sim, _ = prepared(tank(*shape), seed=7 + sum(shape))
+    rng = np.random.default_rng(3)
+    phi = np.roll(sim.water_phase.to_numpy(), 1, axis=1)
+    phi[rng.random(phi.shape) < 0.02] = 1.1e-3
+    sim.water_phase.from_numpy(phi * (sim.solid_body_id.to_numpy() == -1))
+    u = sim.velocity_lattice.to_numpy()
+    sim.velocity_lattice.from_numpy(150.0 * u)
+    saved = snapshot_fields(sim)
+    dt = sim.scales.dt_s
+    sim.remap_energy[None] = 0.0
+    sim._synchronize_water_fused()
+    sim._advect_water(dt)
+    emptied = (sim.water_volume.to_numpy() <= 1e-30) & (phi > 1e-3) & (sim.solid_body_id.to_numpy() == -1)
+    sim._synchronize_water_fused()
+    expected = {name: getattr(sim, name).to_numpy() for name in ("water_volume", "water_energy")}
+    remap = float(sim.remap_energy[None])
+    restore_fields(sim, saved)
+    sim.remap_energy[None] = 0.0
+    sim._remap_advect_remap(dt)
+    assert emptied.any()
+    np.testing.assert_array_equal(sim.water_volume.to_numpy(), expected["water_volume"])
+    got, value = sim.water_energy.to_numpy(), expected["water_energy"]
+    assert np.abs(got - value).max() <= 2.0 ** -22 * np.abs(value).max()
+    assert abs(float(sim.remap_energy[None]) - remap) <= 2.0 ** -23 * (np.sqrt(value.size) * np.abs(value).max()
+                                                                      + 4.0 * abs(remap))
