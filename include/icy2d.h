@@ -187,6 +187,7 @@ int icy2d_measure_aperture(const icy2d_grid* g, void* stream);             /* :6
 int icy2d_build_aperture_targets(const icy2d_grid* g, void* stream);       /* :716-827 */
 int icy2d_apply_aperture_transfer(const icy2d_grid* g, void* stream);      /* :829-859 */
 int icy2d_finish_aperture_transfer(const icy2d_grid* g, void* stream);     /* :861-877 */
+int icy2d_transfer_aperture(const icy2d_grid* g, void* stream);            /* apply, then finish, in one pass */
 int icy2d_body_conduction(const icy2d_grid* g, double dt, void* stream);   /* :879-907 */
 /* axis 0 resets the boundary power (:630-631) before adding its faces; axis 1 adds. */
 int icy2d_conduction_flux(const icy2d_grid* g, int axis, void* stream);    /* :909-1010, :1063-1164 */
@@ -279,6 +280,7 @@ int icy2d_batch_measure_aperture(const icy2d_batch* b, void* stream);
 int icy2d_batch_build_aperture_targets(const icy2d_batch* b, void* stream);
 int icy2d_batch_apply_aperture_transfer(const icy2d_batch* b, void* stream);
 int icy2d_batch_finish_aperture_transfer(const icy2d_batch* b, void* stream);
+int icy2d_batch_transfer_aperture(const icy2d_batch* b, void* stream);
 int icy2d_batch_body_conduction(const icy2d_batch* b, const double* dt, void* stream);
 int icy2d_batch_conduction_flux(const icy2d_batch* b, int axis, void* stream);
 int icy2d_batch_advection_flux(const icy2d_batch* b, int axis, void* stream);

@@ -73,7 +73,7 @@ CALLS = {
     "apply_projection_residual": [_d, _d], "snapshot_melt_momentum": [], "reduce_provisional_momentum": [],
     "melt_weight_geometry": [], "apply_melt_correction": [], "reduce_final_momentum": [],
     "local_melt_correction": [], "finish_melt_momentum": [], "measure_aperture": [], "build_aperture_targets": [],
-    "apply_aperture_transfer": [], "finish_aperture_transfer": [], "body_conduction": [_d],
+    "apply_aperture_transfer": [], "finish_aperture_transfer": [], "transfer_aperture": [], "body_conduction": [_d],
     "conduction_flux": [_i], "advection_flux": [_i], "update_water": [_d, _i], "reset_interval_sources": [], "accumulate_boundary_heat": [_d],
     "exchange_heat": [_d], "phase_change": [], "freeze_eligibility": [], "inject_melt": [], "measure_fallback": [],
     "apply_fallback": [_i], "reduce_totals": [],

@@ -281,8 +281,7 @@ class IceFlowEnsemble2D:
         """simulator.py:511-548."""
         self._call("measure_aperture", active=active)
         self._call("build_aperture_targets", active=active)
-        self._call("apply_aperture_transfer", active=active)
-        self._call("finish_aperture_transfer", active=active)
+        self._call("transfer_aperture", active=active)
 
     def step(self, num_steps=1):
         """Advance every case by ``num_steps`` steps (simulator.py:2194-2227 per case)."""

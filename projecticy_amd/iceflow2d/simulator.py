@@ -826,8 +826,7 @@ class IceFlow2D:
         """simulator.py:511-548 (the capacity check runs on the device)."""
         self._call("measure_aperture")
         self._call("build_aperture_targets")
-        self._call("apply_aperture_transfer")
-        self._call("finish_aperture_transfer")
+        self._call("transfer_aperture")
 
     def _finalize_melt_momentum_coupling(self):
         """simulator.py:2989-3012."""
