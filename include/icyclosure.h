@@ -61,6 +61,16 @@ int64_t icyc_wgrad_partials_size(int32_t nx, int32_t ny, int32_t nz);
 int icyc_conv3d_wgrad(int32_t nx, int32_t ny, int32_t nz, const uint16_t* in, const uint16_t* dout,
                       float* partials, float* grad, void* stream);
 
+/* Backward data and weight gradient of a layer with one output channel, whose
+ * output gradient ``dout`` is one BF16 value a cell (icyc_weighted_mse_plane):
+ * what icyc_conv3d with ICYC_MASKED_BF16 and icyc_conv3d_wgrad give for a
+ * 32-channel gradient that is zero beyond channel 0 (``weights`` in the
+ * backward-data layout, ``partials`` of icyc_wgrad_partials_size floats). */
+int icyc_conv3d_scalar_data(int32_t nx, int32_t ny, int32_t nz, const uint16_t* dout, const uint16_t* weights,
+                            const uint16_t* mask_act, uint16_t* out_bf16, void* stream);
+int icyc_conv3d_scalar_wgrad(int32_t nx, int32_t ny, int32_t nz, const uint16_t* in, const uint16_t* dout,
+                             float* partials, float* grad, void* stream);
+
 /* Weighted squared error of channel 0: loss = sum_n w[n] (pred[n] -
  * target[n])^2; writes dloss/dpred into channel 0 of ``dout`` (BF16, other
  * channels zero) and the loss into loss[0] (FP32, via ``partials`` of
@@ -68,6 +78,10 @@ int icyc_conv3d_wgrad(int32_t nx, int32_t ny, int32_t nz, const uint16_t* in, co
 int64_t icyc_loss_partials_size(int64_t cells);
 int icyc_weighted_mse(int64_t cells, const float* pred, const float* target, const float* weight, uint16_t* dout,
                       float* partials, float* loss, void* stream);
+
+/* The same loss with ``dout`` as one BF16 value a cell. */
+int icyc_weighted_mse_plane(int64_t cells, const float* pred, const float* target, const float* weight,
+                            uint16_t* dout, float* partials, float* loss, void* stream);
 
 /* Adam step on ``count`` layer parameter blocks (ICYC_LAYER_PARAMS each):
  * updates master weights and moments, and writes the BF16 forward and

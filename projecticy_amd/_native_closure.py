@@ -21,6 +21,9 @@ SIGNATURES = {
     "icyc_conv3d_k8": ([_i, _i, _i, _p, _p, _p, _i, _p, _p, _p], ctypes.c_int),
     "icyc_wgrad_partials_size": ([_i, _i, _i], _i64),
     "icyc_conv3d_wgrad": ([_i, _i, _i, _p, _p, _p, _p, _p], ctypes.c_int),
+    "icyc_conv3d_scalar_data": ([_i, _i, _i, _p, _p, _p, _p, _p], ctypes.c_int),
+    "icyc_conv3d_scalar_wgrad": ([_i, _i, _i, _p, _p, _p, _p, _p], ctypes.c_int),
+    "icyc_weighted_mse_plane": ([_i64, _p, _p, _p, _p, _p, _p, _p], ctypes.c_int),
     "icyc_loss_partials_size": ([_i64], _i64),
     "icyc_weighted_mse": ([_i64, _p, _p, _p, _p, _p, _p, _p], ctypes.c_int),
     "icyc_adam": ([_i, _p, _p, _p, _p, _f, _f, _f, _f, _i, _p, _p, _p], ctypes.c_int),

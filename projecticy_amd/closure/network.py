@@ -42,7 +42,8 @@ class ClosureNet:
         self.wb = torch.zeros_like(self.wf)
         act = lambda: torch.zeros(self.cells * C, dtype=torch.int16, device=dev)  # noqa: E731
         self.acts = [act() for _ in range(LAYERS)]  # input features, a1, a2, a3
-        self.dpre = [act() for _ in range(LAYERS)]  # gradients of each layer's pre-activation
+        self.dpre = [act() for _ in range(LAYERS - 1)]  # gradients of the hidden layers' pre-activations
+        self.dpred = torch.zeros(self.cells, dtype=torch.int16, device=dev)  # of the prediction, one BF16 a cell
         self.pred = torch.zeros(self.cells, dtype=torch.float32, device=dev)
         self.loss = torch.zeros(1, dtype=torch.float32, device=dev)
         self.wgrad_partials = torch.zeros(int(self.lib.icyc_wgrad_partials_size(nx, ny, nz)), dtype=torch.float32,
@@ -112,14 +113,22 @@ class ClosureNet:
         gradient (into ``grad``); returns the loss tensor (device, FP32)."""
         nx, ny, nz = self.shape
         s = self._stream()
-        native.check(self.lib.icyc_weighted_mse(self.cells, _ptr(self.pred), _ptr(target), _ptr(weight),
-                                                _ptr(self.dpre[LAYERS - 1]), _ptr(self.loss_partials),
-                                                _ptr(self.loss), s), "icyc_weighted_mse")
+        native.check(self.lib.icyc_weighted_mse_plane(self.cells, _ptr(self.pred), _ptr(target), _ptr(weight),
+                                                      _ptr(self.dpred), _ptr(self.loss_partials), _ptr(self.loss), s),
+                     "icyc_weighted_mse_plane")
         for layer in reversed(range(LAYERS)):
+            grad = self._layer(self.grad, layer, native.LAYER_PARAMS)
+            if layer == LAYERS - 1:  # one output channel
+                native.check(self.lib.icyc_conv3d_scalar_wgrad(nx, ny, nz, _ptr(self.acts[layer]), _ptr(self.dpred),
+                                                               _ptr(self.wgrad_partials), grad, s),
+                             "icyc_conv3d_scalar_wgrad")
+                native.check(self.lib.icyc_conv3d_scalar_data(nx, ny, nz, _ptr(self.dpred),
+                                                              self._layer(self.wb, layer, native.WEIGHTS),
+                                                              _ptr(self.acts[layer]), _ptr(self.dpre[layer - 1]), s),
+                             "icyc_conv3d_scalar_data")
+                continue
             native.check(self.lib.icyc_conv3d_wgrad(nx, ny, nz, _ptr(self.acts[layer]), _ptr(self.dpre[layer]),
-                                                    _ptr(self.wgrad_partials),
-                                                    self._layer(self.grad, layer, native.LAYER_PARAMS), s),
-                         "icyc_conv3d_wgrad")
+                                                    _ptr(self.wgrad_partials), grad, s), "icyc_conv3d_wgrad")
             if layer > 0:
                 native.check(self.lib.icyc_conv3d(nx, ny, nz, _ptr(self.dpre[layer]),
                                                   self._layer(self.wb, layer, native.WEIGHTS), None,

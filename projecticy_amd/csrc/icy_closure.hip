@@ -146,8 +146,7 @@ constexpr int kSweepColumn = (kMaxColumn + 2) * 4, kSweepSlab = (kSweepCols + 2)
 template <int Epi, int T>
 __global__ void __launch_bounds__(kSweepThreads, 2)
     k_conv3d_sweep(int nx, int ny, int per, const uint16_t* __restrict__ in, const uint16_t* __restrict__ w,
-                   const float* __restrict__ bias, const uint16_t* __restrict__ mask, uint16_t* __restrict__ out,
-                   float* __restrict__ out_f32) {
+                   const float* __restrict__ bias, const uint16_t* __restrict__ mask, uint16_t* __restrict__ out) {
   constexpr int nz = 16 * T;  // four columns of nz cells are 4 T tiles, T a wave
   constexpr int kPieces = (kSweepCols + 2) * nz * 4;
   constexpr int kFetch = (kPieces + kSweepThreads - 1) / kSweepThreads;  // 16-byte pieces a thread stages
@@ -253,20 +252,16 @@ __global__ void __launch_bounds__(kSweepThreads, 2)
         const int j = j0 + cell_j[tl];
         if (j >= ny) continue;
         const long cell = ((long)(s - 1) * ny + j) * nz + cell_k[tl];
-        if (Epi == ICYC_LINEAR_F32) {
-          if (channels + group == 0) out_f32[cell] = P[tl][0] + bias[0];
-        } else {
-          float v[4];
+        float v[4];
 #pragma unroll
-          for (int r = 0; r < 4; ++r) v[r] = Epi == ICYC_RELU_BF16 ? fmaxf(0.0f, P[tl][r] + bias_r[r]) : P[tl][r];
-          uint2 packed = make_uint2(pack2(v[0], v[1]), pack2(v[2], v[3]));
-          const long at_c = cell * kC + channels + 4 * group;
-          if (Epi == ICYC_MASKED_BF16) {
-            const uint2 m = *reinterpret_cast<const uint2*>(mask + at_c);
-            packed = make_uint2(keep_positive(packed.x, m.x), keep_positive(packed.y, m.y));
-          }
-          *reinterpret_cast<uint2*>(out + at_c) = packed;
+        for (int r = 0; r < 4; ++r) v[r] = Epi == ICYC_RELU_BF16 ? fmaxf(0.0f, P[tl][r] + bias_r[r]) : P[tl][r];
+        uint2 packed = make_uint2(pack2(v[0], v[1]), pack2(v[2], v[3]));
+        const long at_c = cell * kC + channels + 4 * group;
+        if (Epi == ICYC_MASKED_BF16) {
+          const uint2 m = *reinterpret_cast<const uint2*>(mask + at_c);
+          packed = make_uint2(keep_positive(packed.x, m.x), keep_positive(packed.y, m.y));
         }
+        *reinterpret_cast<uint2*>(out + at_c) = packed;
       }
     }
     current ^= 1;
@@ -282,73 +277,268 @@ __global__ void __launch_bounds__(kSweepThreads, 2)
   }
 }
 
-constexpr int kColumnTile = 2, kStageCols = (kColumnTile + 2) * (kColumnTile + 2);
 // The first layer's form: its input has 8 real channels (the features), so
-// one MFMA takes four taps' 8 channels as its 32-deep K (lane group g: tap
-// 4m + g), 7 MFMAs per output tile instead of 27 over zero-padded channels;
-// only the first 16 bytes of each cell are staged.
-template <int Epi>
-__global__ void __launch_bounds__(kConvThreads)
-    k_conv3d_columns_k8(int nx, int ny, int nz, const uint16_t* __restrict__ in, const uint16_t* __restrict__ w,
-                        const float* __restrict__ bias, uint16_t* __restrict__ out, float* __restrict__ out_f32) {
-  __shared__ uint4 xs[kStageCols][kMaxColumn + 2];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int row = lane & 15, group = lane >> 4;
-  const int tiles_j = (ny + kColumnTile - 1) / kColumnTile;
-  const int i0 = (int)(blockIdx.x / tiles_j) * kColumnTile, j0 = (int)(blockIdx.x % tiles_j) * kColumnTile;
-  const int depth = nz + 2;
-  for (int e = threadIdx.x; e < kStageCols * depth; e += blockDim.x) {
-    const int col = e / depth, cell = e - col * depth;
-    const int i = i0 - 1 + col / 4, j = j0 - 1 + col % 4, k = cell - 1;
-    uint4 v = make_uint4(0u, 0u, 0u, 0u);
-    if (i >= 0 && i < nx && j >= 0 && j < ny && k >= 0 && k < nz)
-      v = *reinterpret_cast<const uint4*>(in + (((long)i * ny + j) * nz + k) * kC);
-    xs[col][cell] = v;
+// one v_mfma_f32_16x16x32_bf16 takes four taps' 8 channels as its reduction
+// (lane group g: tap 4 m + g), 7 products for 16 cells x 16 channels.  Bound
+// by memory (64 bytes a cell in, of which 16 count but a line comes whole, 64
+// out).  The sweep of k_conv3d_sweep with one output slab: the last slabs'
+// pieces stay in a ring of four.  2 x 2 columns a block, staged with all their
+// neighbours and stored a channel at a time, took 33 us at 128x64x64,
+// this 20.
+template <int Epi, int T>
+__global__ void __launch_bounds__(kSweepThreads)
+    k_conv3d_first(int nx, int ny, int per, const uint16_t* __restrict__ in, const uint16_t* __restrict__ w,
+                   const float* __restrict__ bias, uint16_t* __restrict__ out, float* __restrict__ out_f32) {
+  constexpr int nz = 16 * T, kCells = (kSweepCols + 2) * nz, kFetch = (kCells + kSweepThreads - 1) / kSweepThreads;
+  constexpr int kColumn = kMaxColumn + 2, kSlab = (kSweepCols + 2) * kColumn, kGroups = (kTaps + 3) / 4;
+  __shared__ u32x4 ring[4][kSlab];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, row = lane & 15, group = lane >> 4;
+  const int channels = (wave & 1) * 16, tile0 = (wave >> 1) * T;
+  const int tiles_j = (ny + kSweepCols - 1) / kSweepCols;
+  const int j0 = (int)(blockIdx.x % tiles_j) * kSweepCols, x0 = (int)(blockIdx.x / tiles_j) * per;
+  const int x1 = min(nx, x0 + per);
+  const u32x4 zero = {0u, 0u, 0u, 0u};
+  for (int e = threadIdx.x; e < 4 * kSlab; e += kSweepThreads) (&ring[0][0])[e] = zero;
+  bf16x8 wr[kGroups];
+  int di[kGroups], at[kGroups];  // of this lane's tap in each product: slab shift, offset in a slab
+#pragma unroll
+  for (int m = 0; m < kGroups; ++m) {
+    const int t = min(4 * m + group, kTaps - 1);
+    wr[m] = __builtin_bit_cast(bf16x8, zero);
+    if (4 * m + group < kTaps) wr[m] = *reinterpret_cast<const bf16x8*>(w + ((long)t * kC + channels + row) * kC);
+    di[m] = t / 9;
+    at[m] = t / 3 % 3 * kColumn + t % 3;
+  }
+  int src[kFetch], dst[kFetch];
+#pragma unroll
+  for (int f = 0; f < kFetch; ++f) {
+    const int e = threadIdx.x + f * kSweepThreads, col = e / nz, k = e % nz, j = j0 - 1 + col;
+    const bool mine = e < kCells && j >= 0 && j < ny;
+    src[f] = mine ? (j * nz + k) * 4 : 0;
+    dst[f] = mine ? col * kColumn + k + 1 : -1;
+  }
+  u32x4 fetched[kFetch];
+  auto fetch = [&](int s) __attribute__((always_inline)) {
+    const u32x4* slab = reinterpret_cast<const u32x4*>(in) + (long)min(max(s, 0), nx - 1) * ny * nz * 4;
+#pragma unroll
+    for (int f = 0; f < kFetch; ++f) fetched[f] = slab[src[f]];
+  };
+  auto stage = [&](int s) __attribute__((always_inline)) {
+    const bool real = s >= 0 && s < nx;
+#pragma unroll
+    for (int f = 0; f < kFetch; ++f)
+      if (dst[f] >= 0) ring[s & 3][dst[f]] = real ? fetched[f] : zero;
+  };
+  __syncthreads();
+  fetch(x0 - 1);
+  stage(x0 - 1);
+  fetch(x0);
+  stage(x0);
+  fetch(x0 + 1);
+  for (int i = x0; i < x1; ++i) {
+    stage(i + 1);  // the slot of slab i - 3, which no wave reads any more
+    __syncthreads();
+    if (i + 1 < x1) fetch(i + 2);
+    floatx4 acc[T];
+#pragma unroll
+    for (int tl = 0; tl < T; ++tl) acc[tl] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int m = 0; m < kGroups; ++m) {
+      const u32x4* slab = &ring[0][0] + ((i - 1 + di[m]) & 3) * kSlab + at[m];
+#pragma unroll
+      for (int tl = 0; tl < T; ++tl) {
+        const int f = (tile0 + tl) * 16 + row;
+        u32x4 x = slab[f / nz * kColumn + f % nz];
+        if (4 * m + 3 >= kTaps && 4 * m + group >= kTaps) x = zero;
+        acc[tl] = mfma(wr[m], __builtin_bit_cast(bf16x8, x), acc[tl]);
+      }
+    }
+#pragma unroll
+    for (int tl = 0; tl < T; ++tl) {
+      const int f = (tile0 + tl) * 16 + row, j = j0 + f / nz;
+      if (j >= ny) continue;
+      const long cell = ((long)i * ny + j) * nz + f % nz;
+      if (Epi == ICYC_LINEAR_F32) {
+        if (channels + group == 0) out_f32[cell] = acc[tl][0] + bias[0];
+      } else {
+        float v[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) v[r] = fmaxf(0.0f, acc[tl][r] + bias[channels + 4 * group + r]);
+        *reinterpret_cast<uint2*>(out + cell * kC + channels + 4 * group) =
+            make_uint2(pack2(v[0], v[1]), pack2(v[2], v[3]));
+      }
+    }
+  }
+}
+
+// ------------------------------------------------------- the scalar layer
+// The last layer has one output, so its convolution and both gradients are
+// narrow: 27 taps by 32 channels.  The taps become a matrix dimension.
+typedef float floatx16 __attribute__((ext_vector_type(16)));
+__device__ __forceinline__ floatx16 mfma32(bf16x8 a, bf16x8 b, floatx16 c) {
+  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
+}
+constexpr int kScalarCols = 8;
+// Forward: Y[t][x] = sum over ci of w[t][0][ci] in[x][ci] (two products of 32
+// taps x 32 cells, operands straight from memory: every line is read whole),
+// then out[x] = bias + sum over t of Y[t][x + off(t)] from LDS, three output
+// slabs in a thread's registers.  Bound by reading the input once; as one of
+// 16 channels of the general form 30 us at 128x64x64, 14 here.
+constexpr int kTapThreads = 512, kTapColumn = kMaxColumn + 2, kTapRow = (kScalarCols + 2) * kTapColumn + 4;
+template <int T>
+__global__ void __launch_bounds__(kTapThreads)
+    k_conv3d_taps(int nx, int ny, int per, const uint16_t* __restrict__ in, const uint16_t* __restrict__ w,
+                  const float* __restrict__ bias, float* __restrict__ out) {
+  constexpr int nz = 16 * T, kTiles = ((kScalarCols + 2) * nz + 31) / 32;
+  constexpr int kPerWave = (kTiles + kTapThreads / 64 - 1) / (kTapThreads / 64);
+  __shared__ float y[kTaps][kTapRow];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, half = lane >> 5;
+  const int tiles_j = (ny + kScalarCols - 1) / kScalarCols;
+  const int j0 = (int)(blockIdx.x % tiles_j) * kScalarCols, x0 = (int)(blockIdx.x / tiles_j) * per;
+  const int x1 = min(nx, x0 + per);
+  for (int e = threadIdx.x; e < kTaps * kTapRow; e += kTapThreads) (&y[0][0])[e] = 0.0f;
+  bf16x8 wr[2];
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    wr[h] = as_bf16x8(make_uint4(0u, 0u, 0u, 0u));
+    if ((lane & 31) < kTaps)
+      wr[h] = *reinterpret_cast<const bf16x8*>(w + (long)(lane & 31) * kC * kC + 16 * h + 8 * half);
+  }
+  // This lane's cell of the wave's tiles (none: -1) and its place in a row of y.
+  int src[kPerWave], dst[kPerWave];
+#pragma unroll
+  for (int p = 0; p < kPerWave; ++p) {
+    const int f = (wave + p * (kTapThreads / 64)) * 32 + (lane & 31), col = f / nz, k = f % nz, j = j0 - 1 + col;
+    const bool mine = f < (kScalarCols + 2) * nz && j >= 0 && j < ny;
+    src[p] = mine ? (j * nz + k) * 4 + half : -1;
+    dst[p] = col * kTapColumn + k + 1;
+  }
+  u32x4 fetched[kPerWave][2];
+  auto fetch = [&](int s) __attribute__((always_inline)) {
+    const u32x4* slab = reinterpret_cast<const u32x4*>(in) + (long)s * ny * nz * 4;
+#pragma unroll
+    for (int p = 0; p < kPerWave; ++p)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) fetched[p][h] = slab[max(src[p], 0) + 2 * h];
+  };
+  const int own_j = threadIdx.x / nz, own_k = threadIdx.x % nz;
+  const bool owned = (int)threadIdx.x < kScalarCols * nz && j0 + own_j < ny;
+  const int own = own_j * kTapColumn + own_k;
+  float before = 0.0f, here = 0.0f;  // the sums of slabs s - 1 and s so far
+  if (x0 > 0) fetch(x0 - 1);
+  for (int s = x0 - 1; s <= x1; ++s) {
+    float after = 0.0f;
+    __syncthreads();  // the last slab's y has been read
+    if (s >= 0 && s < nx) {
+#pragma unroll
+      for (int p = 0; p < kPerWave; ++p) {
+        floatx16 d;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) d[r] = 0.0f;
+#pragma unroll
+        for (int h = 0; h < 2; ++h) d = mfma32(wr[h], __builtin_bit_cast(bf16x8, fetched[p][h]), d);
+        if (src[p] >= 0)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) {
+            const int t = 8 * (r / 4) + 4 * half + r % 4;
+            if (t < kTaps) y[t][dst[p]] = d[r];
+          }
+      }
+    }
+    if (s + 1 <= x1 && s + 1 < nx) fetch(s + 1);
+    __syncthreads();
+    if (owned && s >= 0 && s < nx) {
+#pragma unroll
+      for (int e = 0; e < 9; ++e) {
+        const int o = own + e / 3 * kTapColumn + e % 3;
+        after += y[e][o];
+        here += y[9 + e][o];
+        before += y[18 + e][o];
+      }
+    }
+    if (owned && s > x0) out[((long)(s - 1) * ny + j0 + own_j) * nz + own_k] = before + bias[0];
+    before = here;
+    here = after;
+  }
+}
+// Data gradient: out[x][ci] = sum over t of wb[t][ci][0] g[x + off(t)] where
+// the activation is positive, else 0: one product of 32 channels x 32 cells
+// with the taps as its reduction (two of depth 16), the gradient plane's
+// values gathered from LDS.  Bound by the mask read and the gradient written;
+// 40 us at 128x64x64 through the general form, 19 here.
+__device__ __forceinline__ void channel_pieces(const floatx16& v, uint4 (&piece)[2]) {
+  // Lane l holds channels 8 q + 4 (l / 32) + e of its cell in v[4 q + e]; on
+  // return piece[0], piece[1] are its cell's 16-byte pieces 2 (l / 32) + {0, 1}.
+  uint32_t p[4][2];
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    p[q][0] = pack2(v[4 * q], v[4 * q + 1]);
+    p[q][1] = pack2(v[4 * q + 2], v[4 * q + 3]);
+  }
+#pragma unroll
+  for (int q = 0; q < 2; ++q) {
+#pragma unroll
+    for (int d = 0; d < 2; ++d) {
+      const auto swapped = __builtin_amdgcn_permlane32_swap(p[q][d], p[q + 2][d], false, false);
+      p[q][d] = swapped[0];
+      p[q + 2][d] = swapped[1];
+    }
+    piece[q] = make_uint4(p[q][0], p[q][1], p[q + 2][0], p[q + 2][1]);
+  }
+}
+constexpr int kSpreadThreads = 256, kSpreadSlab = (kScalarCols + 2) * kTapColumn;
+template <int T>
+__global__ void __launch_bounds__(kSpreadThreads)
+    k_conv3d_spread(int nx, int ny, const uint16_t* __restrict__ g, const uint16_t* __restrict__ wb,
+                    const uint16_t* __restrict__ mask, uint16_t* __restrict__ out) {
+  constexpr int nz = 16 * T;
+  __shared__ uint16_t gs[3 * kSpreadSlab];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, half = lane >> 5;
+  const int tiles_j = (ny + kScalarCols - 1) / kScalarCols;
+  const int j0 = (int)(blockIdx.x % tiles_j) * kScalarCols, i = (int)(blockIdx.x / tiles_j);
+  for (int e = threadIdx.x; e < 3 * kSpreadSlab; e += kSpreadThreads) {
+    const int s = i - 1 + e / kSpreadSlab, j = j0 - 1 + e % kSpreadSlab / kTapColumn, k = e % kTapColumn - 1;
+    gs[e] = s >= 0 && s < nx && j >= 0 && j < ny && k >= 0 && k < nz ? g[((long)s * ny + j) * nz + k] : (uint16_t)0;
+  }
+  typedef uint16_t u16x8 __attribute__((ext_vector_type(8)));
+  bf16x8 wr[2];
+  int at[2][8];
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    u16x8 v;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const int t = 16 * h + 8 * half + e;
+      v[e] = t < kTaps ? wb[((long)t * kC + (lane & 31)) * kC] : (uint16_t)0;
+      at[h][e] = t < kTaps ? t / 9 * kSpreadSlab + t / 3 % 3 * kTapColumn + t % 3 : -1;
+    }
+    wr[h] = __builtin_bit_cast(bf16x8, v);
   }
   __syncthreads();
-  const int wi = wave >> 1, wj = wave & 1, i = i0 + wi, j = j0 + wj;
-  if (i >= nx || j >= ny) return;
-  const int mtiles = nz / 16;
-  constexpr int kGroups = (kTaps + 3) / 4;
-  constexpr int kTiles = Epi == ICYC_LINEAR_F32 ? 1 : 2;  // one output: only channels 0..15 are formed
-  floatx4 acc[4][2];
+  for (int tile = wave; tile * 32 < kScalarCols * nz; tile += kSpreadThreads / 64) {
+    const int f = tile * 32 + (lane & 31), jl = f / nz, k = f % nz, j = j0 + jl;
+    const uint16_t* cell_g = gs + jl * kTapColumn + k;
+    floatx16 d;
 #pragma unroll
-  for (int mt = 0; mt < 4; ++mt) acc[mt][0] = acc[mt][1] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
-  for (int m = 0; m < kGroups; ++m) {
-    const int t = 4 * m + group;
-    bf16x8 b0 = as_bf16x8(make_uint4(0u, 0u, 0u, 0u)), b1 = b0;
-    int col = 0, dk = 0;
-    if (t < kTaps) {
-      const int di = t / 9 - 1, dj = (t / 3) % 3 - 1;
-      dk = t % 3 - 1;
-      col = (wi + 1 + di) * 4 + (wj + 1 + dj);
-      const uint4* wt = reinterpret_cast<const uint4*>(w + (long)t * kC * kC);
-      b0 = as_bf16x8(wt[row * 4]);
-      if (kTiles == 2) b1 = as_bf16x8(wt[(16 + row) * 4]);
+    for (int r = 0; r < 16; ++r) d[r] = 0.0f;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      u16x8 v;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[e] = at[h][e] >= 0 ? cell_g[at[h][e]] : (uint16_t)0;
+      d = mfma32(wr[h], __builtin_bit_cast(bf16x8, v), d);
     }
+    uint4 piece[2];
+    channel_pieces(d, piece);
+    if (j >= ny) continue;
+    const long at_c = (((long)i * ny + j) * nz + k) * kC + 16 * half;
+    const uint4* positive = reinterpret_cast<const uint4*>(mask + at_c);
+    uint4* line = reinterpret_cast<uint4*>(out + at_c);
 #pragma unroll
-    for (int mt = 0; mt < 4; ++mt) {
-      if (mt < mtiles) {
-        const bf16x8 a = t < kTaps ? as_bf16x8(xs[col][mt * 16 + row + 1 + dk]) : b0;  // b0 is zero past the taps
-        acc[mt][0] = mfma(a, b0, acc[mt][0]);
-        if (kTiles == 2) acc[mt][1] = mfma(a, b1, acc[mt][1]);
-      }
-    }
-  }
-  const long base = ((long)i * ny + j) * nz;
-#pragma unroll
-  for (int mt = 0; mt < 4; ++mt) {
-    if (mt >= mtiles) continue;
-#pragma unroll
-    for (int nt = 0; nt < kTiles; ++nt) {
-      const int co = nt * 16 + row;
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const long cell = base + mt * 16 + group * 4 + r;
-        const float x = acc[mt][nt][r];
-        if (Epi == ICYC_RELU_BF16) out[cell * kC + co] = f2bf(fmaxf(0.0f, x + bias[co]));
-        else if (co == 0) out_f32[cell] = x + bias[0];
-      }
+    for (int q = 0; q < 2; ++q) {
+      const uint4 m = positive[q];
+      line[q] = make_uint4(keep_positive(piece[q].x, m.x), keep_positive(piece[q].y, m.y),
+                           keep_positive(piece[q].z, m.z), keep_positive(piece[q].w, m.w));
     }
   }
 }
@@ -374,10 +564,6 @@ __global__ void __launch_bounds__(kConvThreads)
 // A block that staged each column's nine neighbours transposed, element by
 // element, took 109 us a layer at 128x64x64; 40 us now, and the fold of half as
 // many partials 7 us instead of 12.
-typedef float floatx16 __attribute__((ext_vector_type(16)));
-__device__ __forceinline__ floatx16 mfma32(bf16x8 a, bf16x8 b, floatx16 c) {
-  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
-}
 typedef short shortx4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) shortx4* lds_shortx4;
 // 16 rows (cells) of 32 channels from `rows`, as the operand of one product:
@@ -554,6 +740,133 @@ __global__ void __launch_bounds__(kGradThreads, 2)
   }
 }
 
+// The scalar layer's weight gradient: dW[t][0][ci] = sum over x of
+// g[x - off(t)] in[x][ci], one product of 32 taps x 32 channels for 16 cells
+// (the taps' shifts are in the gathered gradient values, so the input is read
+// without a halo).  Bound by reading the input; 40 us at 128x64x64 through the
+// general form, 10 here.  A partial row: 27 x 32 sums, then the bias.
+constexpr int kScalarGradCols = 4, kScalarGradRow = kTaps * kC + 8, kScalarGradSlab = (kScalarGradCols + 2) * kTapColumn;
+template <int T>
+__global__ void __launch_bounds__(kGradThreads)
+    k_scalar_wgrad(int nx, int ny, int per, const uint16_t* __restrict__ in, const uint16_t* __restrict__ g,
+                   float* __restrict__ partials) {
+  constexpr int nz = 16 * T, kPieces = kScalarGradCols * nz * 4, kFetch = (kPieces + kGradThreads - 1) / kGradThreads;
+  __shared__ __attribute__((aligned(16))) char xs[2][kScalarGradCols * kMaxColumn * kGradRow];
+  __shared__ uint16_t gs[2][3 * kScalarGradSlab];
+  __shared__ float red[kGradThreads / 64][kC * kC];
+  __shared__ float bias_part[kGradThreads / 64];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, half = lane >> 5;
+  const int tiles_j = (ny + kScalarGradCols - 1) / kScalarGradCols;
+  const int j0 = (int)(blockIdx.x % tiles_j) * kScalarGradCols, x0 = (int)(blockIdx.x / tiles_j) * per;
+  const int x1 = min(nx, x0 + per);
+  u32x4 fetched[kFetch];
+  bool mine[kFetch];
+  int src[kFetch];
+#pragma unroll
+  for (int f = 0; f < kFetch; ++f) {
+    const int e = tid + f * kGradThreads, col = e / (nz * 4), j = j0 + col;
+    mine[f] = e < kPieces && j < ny;
+    src[f] = mine[f] ? j * nz * 4 + e % (nz * 4) : 0;
+  }
+  float bias_acc = 0.0f;
+  constexpr int kGather = (3 * kScalarGradSlab + kGradThreads - 1) / kGradThreads;
+  uint16_t gathered[kGather];
+  auto fetch = [&](int s) __attribute__((always_inline)) {
+    const u32x4* slab = reinterpret_cast<const u32x4*>(in) + (long)s * ny * nz * 4;
+#pragma unroll
+    for (int f = 0; f < kFetch; ++f) fetched[f] = slab[src[f]];
+#pragma unroll
+    for (int f = 0; f < kGather; ++f) {
+      const int e = tid + f * kGradThreads;
+      const int i = s - 1 + e / kScalarGradSlab, j = j0 - 1 + e % kScalarGradSlab / kTapColumn, k = e % kTapColumn - 1;
+      const bool real = e < 3 * kScalarGradSlab && i >= 0 && i < nx && j >= 0 && j < ny && k >= 0 && k < nz;
+      gathered[f] = real ? g[((long)i * ny + j) * nz + k] : (uint16_t)0;
+    }
+  };
+  auto stage = [&](int buffer) __attribute__((always_inline)) {
+#pragma unroll
+    for (int f = 0; f < kFetch; ++f) {
+      const int e = tid + f * kGradThreads;
+      if (e < kPieces)
+        *reinterpret_cast<u32x4*>(xs[buffer] + (e / (nz * 4) * kMaxColumn * 4 + e % (nz * 4)) * 16) =
+            mine[f] ? fetched[f] : u32x4{0u, 0u, 0u, 0u};
+    }
+#pragma unroll
+    for (int f = 0; f < kGather; ++f) {
+      const int e = tid + f * kGradThreads;
+      if (e < 3 * kScalarGradSlab) gs[buffer][e] = gathered[f];
+      // the slab's own gradient, each cell by the block that owns it
+      const int col = e % kScalarGradSlab / kTapColumn;
+      if (e / kScalarGradSlab == 1 && col >= 1 && col <= kScalarGradCols) bias_acc += bf2f(gathered[f]);
+    }
+  };
+  const int t = lane & 31;
+  const bool tap = t < kTaps;
+  const int tap_at = tap ? (2 - t / 9) * kScalarGradSlab + (2 - t / 3 % 3) * kTapColumn + 2 - t % 3 + 8 * half : 0;
+  const int lane_offset = (8 * half + ((lane & 15) >> 2)) * kGradRow + ((lane >> 4) & 1) * 32 + (lane & 3) * 8;
+  floatx16 acc;
+#pragma unroll
+  for (int r = 0; r < 16; ++r) acc[r] = 0.0f;
+  fetch(x0);
+  stage(0);
+  for (int s = x0; s < x1; ++s) {
+    const int buffer = (s - x0) & 1;
+    __syncthreads();
+    if (s + 1 < x1) fetch(s + 1);
+    for (int unit = wave; unit < kScalarGradCols * T; unit += kGradThreads / 64) {
+      const int col = unit / T, k0 = unit % T * 16;
+      typedef uint16_t u16x8 __attribute__((ext_vector_type(8)));
+      u16x8 v;
+      const uint16_t* cell_g = gs[buffer] + col * kTapColumn + k0 + tap_at;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[e] = tap ? cell_g[e] : (uint16_t)0;
+      const bf16x8 x = column_operand(xs[buffer] + (col * kMaxColumn + k0) * kGradRow, lane_offset);
+      acc = mfma32(__builtin_bit_cast(bf16x8, v), x, acc);
+    }
+    if (s + 1 < x1) stage(buffer ^ 1);
+  }
+#pragma unroll
+  for (int r = 0; r < 16; ++r) red[wave][(8 * (r / 4) + 4 * half + r % 4) * kC + t] = acc[r];
+  for (int off = 1; off < 64; off <<= 1) bias_acc += __shfl_xor(bias_acc, off);
+  if (lane == 0) bias_part[wave] = bias_acc;
+  __syncthreads();
+  float* result = partials + (long)blockIdx.x * kScalarGradRow;
+  for (int e = tid; e < kTaps * kC; e += kGradThreads) {
+    float sum = 0.0f;
+#pragma unroll
+    for (int v = 0; v < kGradThreads / 64; ++v) sum += red[v][e];
+    result[e] = sum;
+  }
+  if (tid == 0) {
+    float sum = 0.0f;
+    for (int v = 0; v < kGradThreads / 64; ++v) sum += bias_part[v];
+    result[kTaps * kC] = sum;
+  }
+}
+// The layer's gradient from the partial rows, in block order; zero for the
+// output channels that the layer does not have.  64 loads in flight: a row is
+// a serial step of the sum.
+__global__ void __launch_bounds__(64) k_fold_scalar(const float* __restrict__ partials, int blocks,
+                                                    float* __restrict__ grad) {
+  const int p = blockIdx.x * 64 + threadIdx.x;
+  if (p >= kLayer) return;
+  const int channel = p < kWeights ? p / kC % kC : p - kWeights;
+  const int at = p < kWeights ? p / (kC * kC) * kC + p % kC : kTaps * kC;
+  float s = 0.0f;
+  if (channel == 0) {
+    int b = 0;
+    for (; b + 64 <= blocks; b += 64) {
+      float v[64];
+#pragma unroll
+      for (int e = 0; e < 64; ++e) v[e] = partials[(long)(b + e) * kScalarGradRow + at];
+#pragma unroll
+      for (int e = 0; e < 64; ++e) s += v[e];
+    }
+    for (; b < blocks; ++b) s += partials[(long)b * kScalarGradRow + at];
+  }
+  grad[p] = s;
+}
+
 // grad[p] = sum over blocks of partials[b][p], in block order.  Bound by
 // reading the partials (28 MB for 256 blocks): one thread a parameter, the
 // adds in order, but kFoldBatch loads in flight and 64-thread blocks so that
@@ -579,6 +892,8 @@ __global__ void __launch_bounds__(kFoldThreads)
 
 // ------------------------------------------------------------------ loss
 constexpr int kLossThreads = 256;
+// Plane: dout is one value a cell; otherwise channel 0 of 32, the rest zero.
+template <bool Plane>
 __global__ void __launch_bounds__(kLossThreads)
     k_weighted_mse(long cells, const float* __restrict__ pred, const float* __restrict__ target,
                    const float* __restrict__ weight, uint16_t* __restrict__ dout, float* __restrict__ partials) {
@@ -588,10 +903,14 @@ __global__ void __launch_bounds__(kLossThreads)
   if (n < cells) {
     const float d = pred[n] - target[n], w = weight[n];
     loss = w * d * d;
-    uint4* o = reinterpret_cast<uint4*>(dout + n * kC);
-    const uint32_t g = f2bf(2.0f * w * d);
-    o[0] = make_uint4(g, 0u, 0u, 0u);
-    o[1] = o[2] = o[3] = make_uint4(0u, 0u, 0u, 0u);
+    const uint16_t g = f2bf(2.0f * w * d);
+    if (Plane) {
+      dout[n] = g;
+    } else {
+      uint4* o = reinterpret_cast<uint4*>(dout + n * kC);
+      o[0] = make_uint4(g, 0u, 0u, 0u);
+      o[1] = o[2] = o[3] = make_uint4(0u, 0u, 0u, 0u);
+    }
   }
   for (int off = 32; off > 0; off >>= 1) loss += __shfl_xor(loss, off);
   if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = loss;
@@ -602,7 +921,6 @@ __global__ void __launch_bounds__(kLossThreads)
     partials[blockIdx.x] = s;
   }
 }
-
 // The loss from the block sums: one block, strided shares, then a fixed tree
 // (a single thread over the 2048 sums of 128x64x64 took 30 us).
 constexpr int kLossFoldThreads = 512;
@@ -708,14 +1026,21 @@ int sweep_slabs(int nx, int tiles_j) {
 }
 template <int Epi>
 void launch_sweep(int nx, int ny, int nz, const uint16_t* in, const uint16_t* w, const float* bias,
-                  const uint16_t* mask, uint16_t* out, float* out_f32, hipStream_t s) {
+                  const uint16_t* mask, uint16_t* out, hipStream_t s) {
   const int tiles_j = (ny + kSweepCols - 1) / kSweepCols, per = sweep_slabs(nx, tiles_j);
   const unsigned blocks = (unsigned)(tiles_j * ((nx + per - 1) / per));
   auto kernel = nz == 16   ? k_conv3d_sweep<Epi, 1>
                 : nz == 32 ? k_conv3d_sweep<Epi, 2>
                 : nz == 48 ? k_conv3d_sweep<Epi, 3>
                            : k_conv3d_sweep<Epi, 4>;
-  kernel<<<blocks, kSweepThreads, 0, s>>>(nx, ny, per, in, w, bias, mask, out, out_f32);
+  kernel<<<blocks, kSweepThreads, 0, s>>>(nx, ny, per, in, w, bias, mask, out);
+}
+void launch_taps(int nx, int ny, int nz, const uint16_t* in, const uint16_t* w, const float* bias, float* out,
+                 hipStream_t s) {
+  const int tiles_j = (ny + kScalarCols - 1) / kScalarCols, per = sweep_slabs(nx, tiles_j);
+  const unsigned blocks = (unsigned)(tiles_j * ((nx + per - 1) / per));
+  auto kernel = nz == 16 ? k_conv3d_taps<1> : nz == 32 ? k_conv3d_taps<2> : nz == 48 ? k_conv3d_taps<3> : k_conv3d_taps<4>;
+  kernel<<<blocks, kTapThreads, 0, s>>>(nx, ny, per, in, w, bias, out);
 }
 // Weight-gradient blocks: pairs of columns times chunks of slabs, one block
 // for each of the 256 CUs where the grid has as many, but four slabs a chunk
@@ -743,15 +1068,15 @@ int icyc_conv3d(int32_t nx, int32_t ny, int32_t nz, const uint16_t* in, const ui
     switch (epilogue) {
       case ICYC_RELU_BF16:
         if (!bias || !out_bf16) return ICYC_ERR_ARGUMENT;
-        launch_sweep<ICYC_RELU_BF16>(nx, ny, nz, in, weights, bias, nullptr, out_bf16, nullptr, s);
+        launch_sweep<ICYC_RELU_BF16>(nx, ny, nz, in, weights, bias, nullptr, out_bf16, s);
         break;
       case ICYC_LINEAR_F32:
         if (!bias || !out_f32) return ICYC_ERR_ARGUMENT;
-        launch_sweep<ICYC_LINEAR_F32>(nx, ny, nz, in, weights, bias, nullptr, nullptr, out_f32, s);
+        launch_taps(nx, ny, nz, in, weights, bias, out_f32, s);
         break;
       case ICYC_MASKED_BF16:
         if (!mask_act || !out_bf16) return ICYC_ERR_ARGUMENT;
-        launch_sweep<ICYC_MASKED_BF16>(nx, ny, nz, in, weights, nullptr, mask_act, out_bf16, nullptr, s);
+        launch_sweep<ICYC_MASKED_BF16>(nx, ny, nz, in, weights, nullptr, mask_act, out_bf16, s);
         break;
       default:
         return ICYC_ERR_ARGUMENT;
@@ -786,15 +1111,23 @@ int icyc_conv3d_k8(int32_t nx, int32_t ny, int32_t nz, const uint16_t* in, const
   if (!valid_grid(nx, ny, nz) || !in || !weights || !bias || nz % 16 != 0 || nz > kMaxColumn)
     return ICYC_ERR_ARGUMENT;
   hipStream_t s = (hipStream_t)stream;
-  const unsigned tiles = (unsigned)(((nx + kColumnTile - 1) / kColumnTile) * ((ny + kColumnTile - 1) / kColumnTile));
-  if (epilogue == ICYC_RELU_BF16 && out_bf16)
-    k_conv3d_columns_k8<ICYC_RELU_BF16><<<tiles, kConvThreads, 0, s>>>(nx, ny, nz, in, weights, bias, out_bf16,
-                                                                      nullptr);
-  else if (epilogue == ICYC_LINEAR_F32 && out_f32)
-    k_conv3d_columns_k8<ICYC_LINEAR_F32><<<tiles, kConvThreads, 0, s>>>(nx, ny, nz, in, weights, bias, nullptr,
-                                                                       out_f32);
-  else
+  const int tiles_j = (ny + kSweepCols - 1) / kSweepCols, per = sweep_slabs(nx, tiles_j);
+  const unsigned blocks = (unsigned)(tiles_j * ((nx + per - 1) / per));
+  if (epilogue == ICYC_RELU_BF16 && out_bf16) {
+    auto kernel = nz == 16   ? k_conv3d_first<ICYC_RELU_BF16, 1>
+                  : nz == 32 ? k_conv3d_first<ICYC_RELU_BF16, 2>
+                  : nz == 48 ? k_conv3d_first<ICYC_RELU_BF16, 3>
+                             : k_conv3d_first<ICYC_RELU_BF16, 4>;
+    kernel<<<blocks, kSweepThreads, 0, s>>>(nx, ny, per, in, weights, bias, out_bf16, nullptr);
+  } else if (epilogue == ICYC_LINEAR_F32 && out_f32) {
+    auto kernel = nz == 16   ? k_conv3d_first<ICYC_LINEAR_F32, 1>
+                  : nz == 32 ? k_conv3d_first<ICYC_LINEAR_F32, 2>
+                  : nz == 48 ? k_conv3d_first<ICYC_LINEAR_F32, 3>
+                             : k_conv3d_first<ICYC_LINEAR_F32, 4>;
+    kernel<<<blocks, kSweepThreads, 0, s>>>(nx, ny, per, in, weights, bias, nullptr, out_f32);
+  } else {
     return ICYC_ERR_ARGUMENT;
+  }
   return status();
 }
 
@@ -819,17 +1152,56 @@ int icyc_conv3d_wgrad(int32_t nx, int32_t ny, int32_t nz, const uint16_t* in, co
   return status();
 }
 
+int icyc_conv3d_scalar_data(int32_t nx, int32_t ny, int32_t nz, const uint16_t* dout, const uint16_t* weights,
+                            const uint16_t* mask_act, uint16_t* out_bf16, void* stream) {
+  if (!valid_grid(nx, ny, nz) || nz % 16 != 0 || nz > kMaxColumn || !dout || !weights || !mask_act || !out_bf16)
+    return ICYC_ERR_ARGUMENT;
+  const unsigned blocks = (unsigned)(nx * ((ny + kScalarCols - 1) / kScalarCols));
+  auto kernel = nz == 16   ? k_conv3d_spread<1>
+                : nz == 32 ? k_conv3d_spread<2>
+                : nz == 48 ? k_conv3d_spread<3>
+                           : k_conv3d_spread<4>;
+  kernel<<<blocks, kSpreadThreads, 0, (hipStream_t)stream>>>(nx, ny, dout, weights, mask_act, out_bf16);
+  return status();
+}
+
+int icyc_conv3d_scalar_wgrad(int32_t nx, int32_t ny, int32_t nz, const uint16_t* in, const uint16_t* dout,
+                             float* partials, float* grad, void* stream) {
+  if (!valid_grid(nx, ny, nz) || nz % 16 != 0 || nz > kMaxColumn || !in || !dout || !partials || !grad)
+    return ICYC_ERR_ARGUMENT;
+  hipStream_t s = (hipStream_t)stream;
+  const int tiles_j = (ny + kScalarGradCols - 1) / kScalarGradCols, slabs = sweep_slabs(nx, tiles_j);
+  const int per = slabs < 4 ? 4 : slabs, blocks = tiles_j * ((nx + per - 1) / per);
+  auto kernel = nz == 16   ? k_scalar_wgrad<1>
+                : nz == 32 ? k_scalar_wgrad<2>
+                : nz == 48 ? k_scalar_wgrad<3>
+                           : k_scalar_wgrad<4>;
+  kernel<<<(unsigned)blocks, kGradThreads, 0, s>>>(nx, ny, per, in, dout, partials);
+  if (int rc = status()) return rc;
+  k_fold_scalar<<<blocks_of(kLayer, 64), 64, 0, s>>>(partials, blocks, grad);
+  return status();
+}
+
 int64_t icyc_loss_partials_size(int64_t cells) { return cells > 0 ? (int64_t)blocks_of(cells, kLossThreads) : 0; }
 
-int icyc_weighted_mse(int64_t cells, const float* pred, const float* target, const float* weight, uint16_t* dout,
-                      float* partials, float* loss, void* stream) {
+static int weighted_mse(bool plane, int64_t cells, const float* pred, const float* target, const float* weight,
+                        uint16_t* dout, float* partials, float* loss, void* stream) {
   if (cells <= 0 || !pred || !target || !weight || !dout || !partials || !loss) return ICYC_ERR_ARGUMENT;
   hipStream_t s = (hipStream_t)stream;
   const unsigned blocks = blocks_of(cells, kLossThreads);
-  k_weighted_mse<<<blocks, kLossThreads, 0, s>>>(cells, pred, target, weight, dout, partials);
+  auto kernel = plane ? k_weighted_mse<true> : k_weighted_mse<false>;
+  kernel<<<blocks, kLossThreads, 0, s>>>(cells, pred, target, weight, dout, partials);
   if (int rc = status()) return rc;
   k_fold_loss<<<1, kLossFoldThreads, 0, s>>>(partials, (int)blocks, loss);
   return status();
+}
+int icyc_weighted_mse(int64_t cells, const float* pred, const float* target, const float* weight, uint16_t* dout,
+                      float* partials, float* loss, void* stream) {
+  return weighted_mse(false, cells, pred, target, weight, dout, partials, loss, stream);
+}
+int icyc_weighted_mse_plane(int64_t cells, const float* pred, const float* target, const float* weight,
+                            uint16_t* dout, float* partials, float* loss, void* stream) {
+  return weighted_mse(true, cells, pred, target, weight, dout, partials, loss, stream);
 }
 
 int icyc_adam(int32_t layers, float* master, float* m, float* v, const float* grad, float lr, float beta1,

@@ -301,3 +301,52 @@ def test_conv_sweep_edges(shape):
 @pytest.mark.parametrize("shape", SWEEP_SHAPES)
 def test_weight_gradient_edges(shape):
     test_weight_gradient(shape)
+
+
+@pytest.mark.parametrize("shape", SWEEP_SHAPES)
+def test_first_layer_edges(shape):
+    test_conv_forward_with_eight_input_channels(shape)
+
+
+@pytest.mark.parametrize("shape", SHAPES + SWEEP_SHAPES)
+def test_scalar_layer_gradients(shape):
+    """The one-output layer's loss, data and weight gradients from a gradient
+    plane: the plane is channel 0 of the 32-channel form bit for bit, the
+    gradients the oracle's for a 32-channel gradient that is zero beyond
+    channel 0 (the tolerances of the general kernels)."""
+    from projecticy_amd import _native_closure as nc
+
+    lib = nc.lib()
+    rng = np.random.default_rng(11 + sum(shape))
+    nx, ny, nz = shape
+    cells = nx * ny * nz
+    x = co.bf16_round(rng.normal(size=shape + (co.C,)))
+    wf = co.bf16_round(rng.normal(scale=0.1, size=(co.TAPS, co.C, co.C)))
+    wf[:, 1:, :] = 0.0
+    wb = co.bf16_round(wf[::-1].transpose(0, 2, 1))
+    f32 = lambda: torch.from_numpy(rng.normal(size=cells).astype(np.float32)).cuda()  # noqa: E731
+    pred, target, weight = f32(), f32(), f32().abs()
+    wide = torch.zeros(cells * co.C, dtype=torch.int16, device="cuda")
+    plane = torch.zeros(cells, dtype=torch.int16, device="cuda")
+    parts = torch.zeros(int(lib.icyc_loss_partials_size(cells)), dtype=torch.float32, device="cuda")
+    losses = torch.zeros(2, dtype=torch.float32, device="cuda")
+    nc.check(lib.icyc_weighted_mse(cells, ptr(pred), ptr(target), ptr(weight), ptr(wide), ptr(parts), ptr(losses),
+                                   stream()), "mse")
+    nc.check(lib.icyc_weighted_mse_plane(cells, ptr(pred), ptr(target), ptr(weight), ptr(plane), ptr(parts),
+                                         ptr(losses[1:]), stream()), "mse plane")
+    torch.cuda.synchronize()
+    assert torch.equal(wide.view(cells, co.C)[:, 0], plane) and losses[0] == losses[1]
+    dout = values_of(wide, shape + (co.C,)).astype(np.float32)
+    out = torch.zeros(cells * co.C, dtype=torch.int16, device="cuda")
+    xt, wbt = bits_tensor(x), bits_tensor(wb)
+    nc.check(lib.icyc_conv3d_scalar_data(nx, ny, nz, ptr(plane), ptr(wbt), ptr(xt), ptr(out), stream()), "data")
+    torch.cuda.synchronize()
+    assert_bf16_close(values_of(out, shape + (co.C,)), np.where(x > 0, co.conv3d_backward_data(dout, wf), 0.0))
+    partials = torch.zeros(int(lib.icyc_wgrad_partials_size(nx, ny, nz)), dtype=torch.float32, device="cuda")
+    grad = torch.ones(co.LAYER_PARAMS, dtype=torch.float32, device="cuda")
+    nc.check(lib.icyc_conv3d_scalar_wgrad(nx, ny, nz, ptr(xt), ptr(plane), ptr(partials), ptr(grad), stream()), "wgrad")
+    dw, db = co.conv3d_weight_grad(x, dout)
+    got = grad.cpu().numpy().astype(np.float64)
+    weights = co.TAPS * co.C * co.C
+    assert np.abs(got[:weights] - dw.ravel()).max() <= 2e-6 * np.abs(dw).max() * max(1.0, cells / 64)
+    assert np.abs(got[weights:] - db).max() <= 1e-5 * max(np.abs(db).max(), 1.0)
