@@ -50,11 +50,11 @@ XCDS = 8  # GRBM_GUI_ACTIVE is reported summed over the eight XCDs
 # bench's kernel groups (bench.py KERNEL_BYTES for the 3D flow step).
 WORKLOADS = {
     "dam_break": {
-        "title": "D3Q27 HOME dam break 256x128x128", "cells": 256 * 128 * 128, "first": "k_collide_stream_tiled",
+        "title": "D3Q27 HOME dam break 256x128x128", "cells": 256 * 128 * 128, "first": "k_stream_rows",
         "groups": {
             "phase_collide": ("k_collide_phase",),
-            "forces": ("k_forces_tiled", "k_forces_general", "k_classify", "k_scatter_flags"),
-            "home_collide_stream": ("k_collide_stream_tiled", "k_stream_boundary", "k_finish_loads"),
+            "forces": ("k_forces_rows", "k_forces_general", "k_classify", "k_scatter_flags"),
+            "home_collide_stream": ("k_stream_rows", "k_stream_boundary", "k_finish_loads"),
             "phase_recover": ("k_recover_phase", "k_fold_recovery"),
             "gradients": ("k_gradients_tiled", "k_gradients_general_list"),
         },

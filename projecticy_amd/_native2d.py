@@ -84,7 +84,7 @@ SHAPES = 12  # ICY2D_SHAPES
 
 class Batch2D(ctypes.Structure):
     _fields_ = [
-        ("ncases", _i), ("collide_threads", _i), ("stream_threads", _i), ("reserved", _i),
+        ("ncases", _i), ("collide_threads", _i), ("stream_threads", _i), ("storage", _i),
         ("grids", _p), ("active", _p), ("first_block", _p), ("total_blocks", _i * SHAPES),
     ]
 

@@ -82,11 +82,30 @@ __device__ __forceinline__ __half half_stochastic(float x, uint32_t salt, uint32
   const float flo = __half2float(lo);
   if (flo == x || !(fabsf(x) < 65504.0f)) return __float2half(x);
   const __half hi = __ushort_as_half((unsigned short)(__half_as_ushort(lo) + 1));  // next step away from zero
-  const float fhi = __half2float(hi);
-  const float p = (x - flo) / (fhi - flo);
+  // The step is a power of two and x - flo has no more bits than x, so the
+  // quotient is exact as a product with the step's inverse.
+  const uint32_t step_bits = __float_as_uint(__half2float(hi) - flo), sign = step_bits & 0x80000000u;
+  const float p = (x - flo) * __uint_as_float(sign | ((254u << 23) - (step_bits & 0x7f800000u)));
   const uint32_t key = mix32(salt * 0x9e3779b1u ^ mix32(step + 0x7f4a7c15u));
   const float r = (float)(mix32(__float_as_uint(x) ^ key) >> 8) * (1.0f / 16777216.0f);
   return r < p ? hi : lo;
+}
+// The step counter as a constant: no kernel that stores populations changes
+// it.  Read like any other word it would be loaded again, and waited for with
+// all stores before it, at every store.
+__device__ __forceinline__ uint32_t rounding_step(const icy2d_grid& g) {
+  return *(const __attribute__((address_space(4))) uint32_t*)&g.control->rounding_step;
+}
+// A stored population's bits, and its value from them.
+template <int Kind>
+__device__ __forceinline__ uint32_t pop_raw(const float* base, const icy2d_grid& g, int idx) {
+  if (half_storage<Kind>(g)) return reinterpret_cast<const uint16_t*>(base)[idx];
+  return reinterpret_cast<const uint32_t*>(base)[idx];
+}
+template <int Kind>
+__device__ __forceinline__ float pop_value(const icy2d_grid& g, uint32_t raw) {
+  if (half_storage<Kind>(g)) return __half2float(__ushort_as_half((unsigned short)raw)) * g.population_inverse_scale;
+  return __uint_as_float(raw);
 }
 template <int Kind>
 __device__ __forceinline__ float pop_get(const float* base, const icy2d_grid& g, int idx) {
@@ -98,7 +117,7 @@ __device__ __forceinline__ void pop_set(float* base, const icy2d_grid& g, int id
   if (half_storage<Kind>(g)) {
     const float x = v * g.population_scale;
     reinterpret_cast<__half*>(base)[idx] =
-        (g.half_populations & 4) ? half_stochastic(x, (uint32_t)idx * 2u + (uint32_t)Kind, g.control->rounding_step)
+        (g.half_populations & 4) ? half_stochastic(x, (uint32_t)idx * 2u + (uint32_t)Kind, rounding_step(g))
                                  : __float2half(x);
   } else {
     base[idx] = v;
@@ -780,41 +799,68 @@ __device__ __forceinline__ PhaseStencil phase_stencil_tile(const W& t, int a, in
 template <class W>
 __device__ __forceinline__ void stage_window(const icy2d_grid& g, W& t, int i0, int j0, int rows) {
   constexpr int PH = W::kPhaseHalo, VH = W::kVelocityHalo;
-  const int N = cells(g);
-  for (int e = threadIdx.x; e < (rows + 2 * PH) * W::kPC; e += blockDim.x) {
-    const int a = e / W::kPC, b = e - a * W::kPC, i = i0 - PH + a, j = j0 - PH + b;
-    // label and phase are loaded together; a wall's or ice cell's is dropped
-    const bool in = inside(g, i, j);
-    const int m = in ? at(g, i, j) : 0;
-    const float phase = g.phi[m];
-    const bool fluid = in && !wall_at(g, i, j) && g.solid[m] == 0;
-    t.fluid[a][b] = fluid;
-    t.phi[a][b] = fluid ? phase : 0.0f;
+  const int N = cells(g), threads = (int)blockDim.x;
+  // All of a thread's values are loaded before the first is used (one after
+  // the other they cost a memory latency each): up to four of the phase and
+  // three of the velocity for tiles of 2, 4 or 8 rows of 64 threads.
+  constexpr int kPhases = ((2 + 2 * PH) * W::kPC + 127) / 128, kVelocities = ((2 + 2 * VH) * W::kUC + 127) / 128;
+  const int phases = (rows + 2 * PH) * W::kPC, velocities = (rows + 2 * VH) * W::kUC;
+  float phase[kPhases], vx[kVelocities], vy[kVelocities];
+  int label[kPhases], solid[kVelocities];
+  bool free[kPhases], in[kVelocities], open[kVelocities];
+#pragma unroll
+  for (int f = 0; f < kPhases; ++f) {
+    if (f * threads >= phases) continue;
+    const int e = (int)threadIdx.x + f * threads, a = e / W::kPC, b = e - a * W::kPC, i = i0 - PH + a, j = j0 - PH + b;
+    const bool inner = inside(g, i, j);
+    const int m = inner ? at(g, i, j) : 0;
+    phase[f] = g.phi[m];
+    label[f] = g.solid[m];
+    free[f] = inner && !wall_at(g, i, j);
   }
-  for (int e = threadIdx.x; e < (rows + 2 * VH) * W::kUC; e += blockDim.x) {
-    const int a = e / W::kUC, b = e - a * W::kUC, i = i0 - VH + a, j = j0 - VH + b;
-    const bool in = inside(g, i, j);
-    const int m = in ? at(g, i, j) : 0, solid = g.solid[m];
-    const float ux = g.u[m], uy = g.u[N + m];
-    const bool fluid = in && !wall_at(g, i, j) && solid == 0;
-    t.kind[a][b] = fluid ? 0 : in && solid == 1 ? 1 : 2;
-    t.u[0][a][b] = fluid ? ux : 0.0f;
-    t.u[1][a][b] = fluid ? uy : 0.0f;
+#pragma unroll
+  for (int f = 0; f < kVelocities; ++f) {
+    if (f * threads >= velocities) continue;
+    const int e = (int)threadIdx.x + f * threads, a = e / W::kUC, b = e - a * W::kUC, i = i0 - VH + a, j = j0 - VH + b;
+    in[f] = inside(g, i, j);
+    const int m = in[f] ? at(g, i, j) : 0;
+    solid[f] = g.solid[m];
+    vx[f] = g.u[m];
+    vy[f] = g.u[N + m];
+    open[f] = in[f] && !wall_at(g, i, j);
+  }
+#pragma unroll
+  for (int f = 0; f < kPhases; ++f) {
+    const int e = (int)threadIdx.x + f * threads, a = e / W::kPC, b = e - a * W::kPC;
+    if (e >= phases) continue;
+    const bool fluid = free[f] && label[f] == 0;  // a wall's or ice cell's phase is dropped
+    t.fluid[a][b] = fluid;
+    t.phi[a][b] = fluid ? phase[f] : 0.0f;
+  }
+#pragma unroll
+  for (int f = 0; f < kVelocities; ++f) {
+    const int e = (int)threadIdx.x + f * threads, a = e / W::kUC, b = e - a * W::kUC;
+    if (e >= velocities) continue;
+    const bool fluid = open[f] && solid[f] == 0;
+    t.kind[a][b] = fluid ? 0 : in[f] && solid[f] == 1 ? 1 : 2;
+    t.u[0][a][b] = fluid ? vx[f] : 0.0f;
+    t.u[1][a][b] = fluid ? vy[f] : 0.0f;
   }
 }
 
 // What a cell's collision reads of its own, loaded before the block waits for
 // the window: the populations as stored, velocity, pressure and water.
 struct OwnCell {
-  float f[9], h[9], u[2], p;
+  uint32_t f[9], h[9];
+  float u[2], p;
   double water_v, water_e;
 };
 __device__ __forceinline__ void load_own(const icy2d_grid& g, int n, int with_momentum, OwnCell& o) {
   const int N = cells(g);
 #pragma unroll
   for (int q = 0; q < 9; ++q) {
-    o.h[q] = pop_get<kPhase>(g.h, g, q * N + n);
-    if (with_momentum) o.f[q] = pop_get<kMomentum>(g.f, g, q * N + n);
+    o.h[q] = pop_raw<kPhase>(g.h, g, q * N + n);
+    if (with_momentum) o.f[q] = pop_raw<kMomentum>(g.f, g, q * N + n);
   }
   o.u[0] = g.u[n];
   o.u[1] = g.u[N + n];
@@ -830,14 +876,18 @@ __device__ __forceinline__ void load_own(const icy2d_grid& g, int n, int with_mo
 // its velocity arrays.  The post-collision populations go to pf and ph, the
 // force density to (ax, ay) (read from g.a when with_momentum is 0) and the
 // cut links' momentum exchange is added to load.
+// Populations are moved by kernels compiled for their storage (one_case):
+// with a branch around each access an FP16 load was converted, and so waited
+// for, before the next was issued (over the 64-case ensemble 1052 us, 628).
 // The reference forms the equilibria's and forces' moments as sums over the
 // nine directions; they are polynomials in u (momentum: raw moments of the
 // Liang equilibrium and its source; phase: central moments of the quadratic
 // equilibrium and of w_q c.n), so they are written down here, and the
 // populations come back from the moments one axis at a time.  The body's
 // pose (FP64 sine and cosine) is needed beside the ice only: near.  The sums
-// and a pose in every lane took 247 us at 1024x2048, this 180, and 157 with
-// the cell's own values loaded before the block waits for its window.
+// and a pose in every lane took 247 us at 1024x2048, this 180, 157 with the
+// cell's own values loaded before the block waits for its window, and 132 with
+// the window's loads in one go.
 template <class W>
 __device__ __forceinline__ void collide_cell(const icy2d_grid& g, const OwnCell& own, bool near, const Pose& pose,
                                              const W& tile, int a0, int b0, int av, int bv, int i, int j, int n,
@@ -888,7 +938,9 @@ __device__ __forceinline__ void collide_cell(const icy2d_grid& g, const OwnCell&
     const float Fx = rho * ax, Fy = rho * ay, drho = g.rho_w - g.rho_a;
     const float gsx = st.source[0], gsy = st.source[1];
     // Raw moments m = {00, 10, 01, 20, 02, 11, 21, 12, 22}.
-    const float(&f)[9] = own.f;
+    float f[9];
+#pragma unroll
+    for (int q = 0; q < 9; ++q) f[q] = pop_value<kMomentum>(g, own.f[q]);
     const float east = f[1] + f[5] + f[8], west = f[3] + f[6] + f[7];
     const float north = f[2] + f[5] + f[6], south = f[4] + f[7] + f[8];
     const float raw0 = f[0] + f[2] + f[4] + east + west, raw1 = east - west, raw2 = north - south;
@@ -939,7 +991,10 @@ __device__ __forceinline__ void collide_cell(const icy2d_grid& g, const OwnCell&
   const float A = third * compression * (st.g[0] / norm), B = third * compression * (st.g[1] / norm);
   float h[9];
 #pragma unroll
-  for (int q = 0; q < 9; ++q) h[q] = phase_relative(g) ? own.h[q] + wq(q) * phi : own.h[q];  // as phase_get
+  for (int q = 0; q < 9; ++q) {  // as phase_get
+    const float value = pop_value<kPhase>(g, own.h[q]);
+    h[q] = phase_relative(g) ? value + wq(q) * phi : value;
+  }
   const float east = h[1] + h[5] + h[8], west = h[3] + h[6] + h[7];
   const float north = h[2] + h[5] + h[6], south = h[4] + h[7] + h[8];
   const float total = h[0] + h[2] + h[4] + east + west;
@@ -1063,7 +1118,11 @@ __device__ __forceinline__ void pull(const icy2d_grid& g, const Pose& pose, int 
 // population sum) from the cell's populations, as the reference's separate
 // macroscopic kernel does after streaming.  The step runs both in one pass.
 constexpr int kStreamPull = 1, kStreamUpdate = 2;
-__device__ __forceinline__ void k2_stream(const icy2d_grid& g, const int blk, int phase_only, int mode) {
+// A kernel for each mode: the pulls' registers (cut links) would leave the
+// update alone, which moves most bytes, five waves a SIMD instead of eight, and its
+// loads wait for the label (269 us over the 64-case ensemble, 146).
+template <int mode>
+__device__ __forceinline__ void k2_stream(const icy2d_grid& g, const int blk, int phase_only) {
   const int n = cell_index(blk), N = cells(g);
   if (n >= N) return;
   const int i = n / g.ny, j = n - i * g.ny;
@@ -1071,9 +1130,18 @@ __device__ __forceinline__ void k2_stream(const icy2d_grid& g, const int blk, in
   const bool posed = (mode & kStreamPull) || g.solid[n] == 1;
   Pose pose = {};
   if (posed) pose = load_pose(g);
-  const bool po = phase_only != 0, pulling = mode & kStreamPull, update = mode & kStreamUpdate;
+  const bool po = phase_only != 0;
+  constexpr bool pulling = mode & kStreamPull, update = mode & kStreamUpdate;
+  const float phi_old = g.phi[n];
+  uint32_t own_f[9] = {}, own_h[9] = {};  // loaded before the label is waited for
+  if (!pulling) {
+#pragma unroll
+    for (int q = 0; q < 9; ++q) {
+      own_h[q] = pop_raw<kPhase>(g.h, g, q * N + n);
+      if (!po) own_f[q] = pop_raw<kMomentum>(g.f, g, q * N + n);
+    }
+  }
   if (fluid_at(g, i, j)) {
-    const float phi_old = g.phi[n];
     float f[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0}, h[9];
     if (pulling) {
       pull<0>(g, pose, i, j, n, phi_old, po, f[0], h[0]);
@@ -1088,8 +1156,9 @@ __device__ __forceinline__ void k2_stream(const icy2d_grid& g, const int blk, in
     } else {
 #pragma unroll
       for (int q = 0; q < 9; ++q) {
-        h[q] = phase_get(g.h, g, q, n, phi_old);
-        if (!po) f[q] = pop_get<kMomentum>(g.f, g, q * N + n);
+        const float value = pop_value<kPhase>(g, own_h[q]);
+        h[q] = phase_relative(g) ? value + wq(q) * phi_old : value;  // as phase_get
+        if (!po) f[q] = pop_value<kMomentum>(g, own_f[q]);
       }
     }
     float phi = phi_old;
@@ -1148,7 +1217,7 @@ __device__ __forceinline__ void pop_copy(float* dst, const float* src, const icy
 // what another writes: f and h are read, fbuf and hbuf written.  A
 // non-fluid cell's stored populations are carried over to fbuf and hbuf.
 // The caller swaps f/fbuf and h/hbuf and then runs the macroscopic update
-// (k2_stream mode 2), which reads only the cell's own populations.  A phase
+// (k2_stream<2>), which reads only the cell's own populations.  A phase
 // population stored relative to the phase (bit 3) is stored against its
 // destination's phase, which the update decodes it with.
 __device__ __forceinline__ void k2_collide_push(const icy2d_grid& g, const int blk) {
@@ -1290,20 +1359,38 @@ __device__ __forceinline__ void k2_outflow_partials(const icy2d_grid& g, const i
   double best = 0.0;
   if (n < N) {
     const int i = n / g.ny, j = n - i * g.ny;
-    if (fluid_at(g, i, j) && g.phi[n] > g.cutoff) {
-      const float vx = g.u[n] + 0.5f * g.a[n], vy = g.u[N + n] + 0.5f * g.a[N + n];
-      float outflow = 0.0f;
-      const int off[4][2] = {{1, 0}, {-1, 0}, {0, 1}, {0, -1}};
+    // Labels and phases of the cell and its neighbours in one go (nested in
+    // the tests they cost a memory latency each: 145 us over the 64-case
+    // ensemble, 84).
+    const int off[5][2] = {{0, 0}, {1, 0}, {-1, 0}, {0, 1}, {0, -1}};
+    int m[5];
+    float phase[5];
+    bool open[5];
+    int label[5];
 #pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        const int ni = i + off[k][0], nj = j + off[k][1];
-        if (!inside(g, ni, nj)) continue;
-        const int m = at(g, ni, nj);
-        if (fluid_at(g, ni, nj) && g.phi[m] > g.cutoff) {
-          const float wx = g.u[m] + 0.5f * g.a[m], wy = g.u[N + m] + 0.5f * g.a[N + m];
-          outflow += fmaxf(0.0f, (float)off[k][0] * (0.5f * (vx + wx)) + (float)off[k][1] * (0.5f * (vy + wy)));
-        }
+    for (int k = 0; k < 5; ++k) {
+      const int ni = i + off[k][0], nj = j + off[k][1];
+      open[k] = inside(g, ni, nj) && !wall_at(g, ni, nj);
+      m[k] = open[k] ? at(g, ni, nj) : n;
+      label[k] = g.solid[m[k]];
+      phase[k] = g.phi[m[k]];
+    }
+    bool wet[5];
+#pragma unroll
+    for (int k = 0; k < 5; ++k) wet[k] = open[k] && label[k] == 0 && phase[k] > g.cutoff;
+    if (wet[0]) {
+      const float vx = g.u[n] + 0.5f * g.a[n], vy = g.u[N + n] + 0.5f * g.a[N + n];
+      float outflow = 0.0f, wx[5], wy[5];
+#pragma unroll
+      for (int k = 1; k < 5; ++k) {
+        const int w = wet[k] ? m[k] : n;
+        wx[k] = g.u[w] + 0.5f * g.a[w];
+        wy[k] = g.u[N + w] + 0.5f * g.a[N + w];
       }
+#pragma unroll
+      for (int k = 1; k < 5; ++k)
+        if (wet[k])
+          outflow += fmaxf(0.0f, (float)off[k][0] * (0.5f * (vx + wx[k])) + (float)off[k][1] * (0.5f * (vy + wy[k])));
       if (!isfinite(vx) || !isfinite(vy)) outflow = INFINITY;
       best = outflow;
     }
@@ -1348,13 +1435,16 @@ __device__ __forceinline__ void k2_clip_phase(const icy2d_grid& g, const int blk
   double v[1] = {0.0};
   if (n < N) {
     const int i = n / g.ny, j = n - i * g.ny;
+    const float old_phase = g.phi[n];
+    uint32_t own[9];  // loaded before the label is waited for
+#pragma unroll
+    for (int q = 0; q < 9; ++q) own[q] = pop_raw<kPhase>(g.h, g, q * N + n);
     if (fluid_at(g, i, j)) {
-      const float old_phase = g.phi[n];
       float bounded = clamp01(old_phase);
       if (bounded <= g.cutoff) bounded = 0.0f;
       else if (bounded >= 1.0f - g.cutoff) bounded = 1.0f;
-      const float ux = g.u[n], uy = g.u[N + n];
       if (bounded != old_phase) {
+        const float ux = g.u[n], uy = g.u[N + n];
         const float pdyn = g.p[n] - g.p_ref[j];
         const float ro = mixture(g, old_phase), rn = mixture(g, bounded);
 #pragma unroll
@@ -1364,12 +1454,14 @@ __device__ __forceinline__ void k2_clip_phase(const icy2d_grid& g, const int blk
       float h[9], l1 = 0.0f;
 #pragma unroll
       for (int q = 0; q < 9; ++q) {
-        h[q] = phase_get(g.h, g, q, n, old_phase);
+        const float value = pop_value<kPhase>(g, own[q]);
+        h[q] = phase_relative(g) ? value + wq(q) * old_phase : value;  // as phase_get
         l1 += fabsf(h[q]);
       }
       const bool regularize = (bounded == 0.0f || bounded == 1.0f) && (double)l1 > max_bulk_l1;
       if (regularize || bounded != old_phase) {
-        const float px = g.u[n] + 0.5f * g.a[n], py = g.u[N + n] + 0.5f * g.a[N + n];
+        const float ux = g.u[n], uy = g.u[N + n];
+        const float px = ux + 0.5f * g.a[n], py = uy + 0.5f * g.a[N + n];
         float sum = 0.0f;
 #pragma unroll
         for (int q = 0; q < 9; ++q) {
@@ -1505,7 +1597,6 @@ __device__ __forceinline__ void k2_copy_band(const icy2d_grid& g, const int blk)
 }
 // simulator.py:4291-4351
 __device__ __forceinline__ void k2_evaluate_projection(const icy2d_grid& g, const int blk, double lambda) {
-  const double e = exp(lambda);
   const int n = cell_index(blk);
   double v[2] = {0.0, 0.0};
   if (n < cells(g)) {
@@ -1514,7 +1605,10 @@ __device__ __forceinline__ void k2_evaluate_projection(const icy2d_grid& g, cons
       const double phase = g.phi[n];
       double mapped = phase;
       const bool adjustable = pop_get<kPhase>(g.hbuf, g, n) == 1.0f;
-      if (adjustable) mapped = phase * e / (1.0 - phase + phase * e);
+      if (adjustable) {
+        const double e = exp(lambda);
+        mapped = phase * e / (1.0 - phase + phase * e);
+      }
       float m32 = (float)mapped;
       if (m32 <= g.cutoff) m32 = 0.0f;
       else if (m32 >= 1.0f - g.cutoff) m32 = 1.0f;
@@ -2388,8 +2482,15 @@ __device__ __forceinline__ T resolve(T a, int) {
   return a;
 }
 
-template <int T, auto F, class... A>
+// Storage >= 0: every case stores its populations that way, so a kernel body
+// has no branch around each of a cell's 18 loads and stores (an FP16 load that
+// is converted in its own branch is waited for there, one after the other).
+// Compiled for FP32 and the two stochastic FP16 forms; any other runs with
+// the branches.
+constexpr int kAnyStorage = -1, kHalfMomentum = 5, kHalfRelative = 15;
+template <int T, auto F, int Storage = kAnyStorage, class... A>
 __global__ void __launch_bounds__(T) one_case(icy2d_grid g, A... a) {
+  if (Storage != kAnyStorage) g.half_populations = Storage;
   F(g, (int)blockIdx.x, a...);
 }
 // Largest c with first[c] <= x (first is non-decreasing, first[0] = 0).
@@ -2402,12 +2503,34 @@ __device__ __forceinline__ int owner(const int32_t* first, int ncases, int x) {
   }
   return lo;
 }
-template <int T, auto F, class... A>
+// A case's grid, its pointers known to the compiler as global memory: read
+// from memory they could be LDS too, and each access would be a flat one, which
+// counts as an LDS access as well and is waited for as such.
+template <class T>
+__device__ __forceinline__ void as_global(T*& p) {
+  p = (T*)(__attribute__((address_space(1))) T*)(uintptr_t)p;
+}
+__device__ __forceinline__ icy2d_grid case_grid(const icy2d_batch& b, int c) {
+  icy2d_grid g = b.grids[c];
+  as_global(g.f), as_global(g.fbuf), as_global(g.h), as_global(g.hbuf);
+  as_global(g.phi), as_global(g.u), as_global(g.a), as_global(g.p), as_global(g.moving);
+  as_global(g.p_ref), as_global(g.rho_ref);
+  as_global(g.solid), as_global(g.prev_solid), as_global(g.eligible);
+  as_global(g.coverage), as_global(g.phase_ref);
+  as_global(g.body_mass), as_global(g.body_energy), as_global(g.body_heat);
+  as_global(g.melt_mass), as_global(g.melt_sensible), as_global(g.melt_target);
+  as_global(g.water_v), as_global(g.water_e), as_global(g.target_e);
+  as_global(g.flux_ex), as_global(g.flux_vx), as_global(g.flux_ey), as_global(g.flux_vy);
+  as_global(g.inject_acc), as_global(g.partials), as_global(g.control);
+  return g;
+}
+template <int T, auto F, int Storage = kAnyStorage, class... A>
 __global__ void __launch_bounds__(T) many_cases(icy2d_batch b, int shape, A... a) {
   const int32_t* first = b.first_block + shape * (b.ncases + 1);
   const int c = owner(first, b.ncases, (int)blockIdx.x);
   if (b.active && !b.active[c]) return;
-  const icy2d_grid g = b.grids[c];
+  icy2d_grid g = case_grid(b, c);
+  if (Storage != kAnyStorage) g.half_populations = Storage;
   F(g, (int)blockIdx.x - first[c], resolve(a, c)...);
 }
 // Destination of a finished reduction: a byte offset into the control block,
@@ -2427,7 +2550,7 @@ __global__ void __launch_bounds__(kFinishThreads) k2_finish_many(icy2d_batch b, 
                                                                  unsigned add_mask) {
   const int c = (int)blockIdx.x / K, k = (int)blockIdx.x - c * K;
   if (b.active && !b.active[c]) return;
-  const icy2d_grid g = b.grids[c];
+  const icy2d_grid g = case_grid(b, c);
   const int32_t* first = b.first_block + shape * (b.ncases + 1);
   finish_fold(g.partials, first[c + 1] - first[c], K, k, dest_ptr(g, d), min_mask, max_mask, add_mask);
 }
@@ -2463,7 +2586,7 @@ __global__ void __launch_bounds__(kFinishThreads) k2_finish_many_tail(icy2d_batc
                                                                       unsigned add_mask, A... a) {
   const int c = (int)blockIdx.x / K, k = (int)blockIdx.x - c * K;
   if (b.active && !b.active[c]) return;
-  const icy2d_grid g = b.grids[c];
+  const icy2d_grid g = case_grid(b, c);
   const int32_t* first = b.first_block + shape * (b.ncases + 1);
   finish_fold(g.partials, first[c + 1] - first[c], K, k, dest_ptr(g, d), min_mask, max_mask, add_mask);
   if (last_finisher(g.control, K) && threadIdx.x == 0) Tail(g, 0, resolve(a, c)...);
@@ -2486,9 +2609,21 @@ struct One {
     one_case<kBlock, F><<<shape_blocks(g, shape), shape_threads(shape), 0, s>>>(g, a...);
     return launch_status();
   }
+  // A kernel that moves populations, compiled for the grid's storage.
+  template <auto F, class... A>
+  int launch_stored(int shape, A... a) const {
+    const unsigned blocks = shape_blocks(g, shape);
+    const int threads = shape_threads(shape);
+    auto kernel = one_case<kBlock, F, kAnyStorage, A...>;
+    if (g.half_populations == 0) kernel = one_case<kBlock, F, 0, A...>;
+    if (g.half_populations == kHalfMomentum) kernel = one_case<kBlock, F, kHalfMomentum, A...>;
+    if (g.half_populations == kHalfRelative) kernel = one_case<kBlock, F, kHalfRelative, A...>;
+    kernel<<<blocks, threads, 0, s>>>(g, a...);
+    return launch_status();
+  }
   template <auto F, class... A>
   int launch_tuned(int shape, A... a) const {
-    return launch<F>(shape, a...);
+    return launch_stored<F>(shape, a...);
   }
   int finish(int shape, int K, Dest d, unsigned mn, unsigned mx, unsigned add) const {
     k2_finish<<<K, kFinishThreads, 0, s>>>(g.partials, (int)shape_blocks(g, shape), K, dest_ptr(g, d), mn, mx, add);
@@ -2514,12 +2649,22 @@ struct Many {
     many_cases<kBlock, F><<<b.total_blocks[shape], shape_threads(shape), 0, s>>>(b, shape, a...);
     return launch_status();
   }
+  // A kernel that moves populations, compiled for the cases' common storage.
+  template <auto F, class... A>
+  int launch_stored(int shape, A... a) const {
+    auto kernel = many_cases<kBlock, F, kAnyStorage, A...>;
+    if (b.storage == 1) kernel = many_cases<kBlock, F, 0, A...>;
+    if (b.storage == 1 + kHalfMomentum) kernel = many_cases<kBlock, F, kHalfMomentum, A...>;
+    if (b.storage == 1 + kHalfRelative) kernel = many_cases<kBlock, F, kHalfRelative, A...>;
+    kernel<<<b.total_blocks[shape], kBlock, 0, s>>>(b, shape, a...);
+    return launch_status();
+  }
   template <auto F, class... A>
   int launch_tuned(int shape, A... a) const {
     const unsigned blocks = b.total_blocks[shape];
     if (shape_threads(shape) == 128) many_cases<128, F><<<blocks, 128, 0, s>>>(b, shape, a...);
     else if (shape_threads(shape) == 512) many_cases<512, F><<<blocks, 512, 0, s>>>(b, shape, a...);
-    else many_cases<kBlock, F><<<blocks, kBlock, 0, s>>>(b, shape, a...);
+    else return launch_stored<F>(shape, a...);
     return launch_status();
   }
   int finish(int shape, int K, Dest d, unsigned mn, unsigned mx, unsigned add) const {
@@ -2589,7 +2734,10 @@ template <class D> int op_prepare_cut_links(const D& d) {
 }
 template <class D> int op_stream(const D& d, int phase_only, int mode) {
   if (mode < 1 || mode > 3) return ICY2D_ERR_ARGUMENT;
-  return d.template launch_tuned<k2_stream>(d.tuned_shape(1), phase_only, mode);
+  const int shape = d.tuned_shape(1);
+  if (mode == kStreamPull) return d.template launch_tuned<k2_stream<kStreamPull>>(shape, phase_only);
+  if (mode == kStreamUpdate) return d.template launch_tuned<k2_stream<kStreamUpdate>>(shape, phase_only);
+  return d.template launch_tuned<k2_stream<kStreamPull | kStreamUpdate>>(shape, phase_only);
 }
 template <class D> int op_update_pressure(const D& d) { return d.template launch<k2_update_pressure>(kCells); }
 template <class D> int op_refill(const D& d) { return d.template launch<k2_refill>(kCells); }
@@ -2600,7 +2748,7 @@ template <class D> int op_measure_outflow(const D& d) {
 }
 template <class D> int op_clip_phase(const D& d, double max_bulk_l1) {
   NEED(d, kCells, 1);
-  TRY(d.template launch<k2_clip_phase>(kCells, max_bulk_l1));
+  TRY(d.template launch_stored<k2_clip_phase>(kCells, max_bulk_l1));
   return d.finish(kCells, 1, CTL(water, 1), 0u, 0u, 0u);
 }
 template <class D> int op_seed_projection(const D& d) { return d.template launch<k2_seed_projection>(kCells); }
@@ -2620,7 +2768,7 @@ template <class D> int op_evaluate_projection(const D& d, typename D::Real lambd
 }
 template <class D> int op_apply_projection(const D& d, typename D::Real lambda) {
   NEED(d, kCells, 1);
-  TRY(d.template launch<k2_apply_projection>(kCells, lambda));
+  TRY(d.template launch_stored<k2_apply_projection>(kCells, lambda));
   return d.finish(kCells, 1, CTL(water, 1), 0u, 0u, 0u);
 }
 template <class D> int op_projection_residual_weight(const D& d, typename D::Real residual) {
@@ -2655,7 +2803,7 @@ template <class D> int op_melt_weight_geometry(const D& d) {
   return d.template finish_tail<k2_melt_status>(kCells, 3, CTL(wet, 1), 0u, 0u, 0u);
 }
 template <class D> int op_apply_melt_correction(const D& d) {
-  return d.template launch<k2_apply_melt_correction>(kCells);
+  return d.template launch_stored<k2_apply_melt_correction>(kCells);
 }
 template <class D> int op_reduce_final_momentum(const D& d) { return fluid_momentum(d, CTL(after, 0)); }
 template <class D> int op_local_melt_correction(const D& d) {

@@ -87,6 +87,7 @@ class IceFlowEnsemble2D:
         b = self._batch
         b.ncases = n
         b.collide_threads = b.stream_threads = 256
+        b.storage = 1 + self.cases[0]._g.half_populations  # one population_storage for every case
         self._flow_parity = 0  # swaps of the fused pass's buffer pairs in the device grids, mod 2
         b.grids = self._grids.data_ptr()
         b.active = None

@@ -1,7 +1,8 @@
 """2D kernels that leave out what cannot matter: cells beyond the body's
 reach take no pose, and the aperture transfer forms its totals from what it
 writes.  Against the FP64 oracle's coverage and masks at angles where the
-corners reach furthest, and against the two separate entry points."""
+corners reach furthest, and against the two separate entry points.  Kernels
+compiled for one population storage against the general ones."""
 
 import math
 
@@ -42,3 +43,26 @@ def test_transfer_equals_apply_then_finish():
                         np.array(control.transfer[:])))
     for a, b in zip(*results):  # the same cells' values, summed in the same blocks
         np.testing.assert_array_equal(a, b)
+
+
+@pytest.mark.parametrize("storage,step", [("fp32", 2.0 ** -24), ("fp16-momentum-sr", 2.0 ** -24),
+                                          ("fp16-rel-sr", 2.0 ** -11)])
+def test_kernels_compiled_for_a_storage(storage, step):
+    """A batch that states its cases' common storage runs kernels compiled
+    for it, one that does not the general ones; the two may contract
+    differently.  The bound: in each of three steps a phase is the sum of nine
+    populations below 1, each off by some roundings (32 allowed) of its
+    storage's step."""
+    from projecticy_amd.iceflow2d.ensemble import IceFlowEnsemble2D
+
+    phases = []
+    for stated in (True, False):
+        batch = IceFlowEnsemble2D([submerged_config(), submerged_config()], population_storage=storage,
+                                  use_graph=False)
+        assert batch._batch.storage == 1 + batch.cases[0]._g.half_populations
+        if not stated:
+            batch._batch.storage = 0
+        batch.step(3)
+        phases.append([case.water_phase.to_numpy() for case in batch.cases])
+    for a, b in zip(*phases):
+        np.testing.assert_allclose(a, b, rtol=0.0, atol=3 * 9 * 32 * step)
