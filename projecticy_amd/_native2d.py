@@ -79,7 +79,7 @@ CALLS = {
     "apply_fallback": [_i], "reduce_totals": [],
 }
 
-SHAPES = 12  # ICY2D_SHAPES
+SHAPES = 13  # ICY2D_SHAPES
 
 
 class Batch2D(ctypes.Structure):

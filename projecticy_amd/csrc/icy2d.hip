@@ -48,6 +48,24 @@ __device__ __forceinline__ bool wall_at(const icy2d_grid& g, int i, int j) {
 }
 // simulator.py:2300-2301
 __device__ __forceinline__ bool fluid_at(const icy2d_grid& g, int i, int j) { return !wall_at(g, i, j) && g.solid[at(g, i, j)] == 0; }
+// Row and column of cell n, one of the cells first .. first + 255: on long
+// rows the division is that of the first cell, the same for all lanes (a
+// lane's own takes some 30 vector instructions).  For the reductions that run
+// over several such blocks of cells; the kernels of one cell a thread gained
+// nothing by it.
+__device__ __forceinline__ void row_col(const icy2d_grid& g, int first, int n, int& i, int& j) {
+  if (g.ny >= 512) {
+    i = first / g.ny;
+    j = n - i * g.ny;
+    if (j >= g.ny) {
+      j -= g.ny;
+      ++i;
+    }
+  } else {
+    i = n / g.ny;
+    j = n - i * g.ny;
+  }
+}
 __device__ __forceinline__ float clamp01(float v) { return fminf(1.0f, fmaxf(0.0f, v)); }
 __device__ __forceinline__ double clamp01d(double v) { return fmin(1.0, fmax(0.0, v)); }
 
@@ -416,6 +434,12 @@ __global__ void __launch_bounds__(kFinishThreads) k2_finish(const double* __rest
   finish_fold(partials, blocks, K, (int)blockIdx.x, out, min_mask, max_mask, add_mask);
 }
 
+// Reductions over all cells take kRun cells a thread (kRuns): the FP64 wave
+// sums, the quotients that are the same for all cells and the block sums' fold
+// were a light kernel's largest part (over the 64-case ensemble: evaluation 47
+// to 25 us, support 46 to 22, aperture 74 to 54, its targets 76 to 58, the
+// transfer 81 to 72).
+constexpr int kRun = 4;
 __device__ __forceinline__ int cell_index(int blk) { return blk * (int)blockDim.x + (int)threadIdx.x; }
 
 // ---------------------------------------------------- geometry kernels
@@ -445,21 +469,32 @@ __device__ __forceinline__ void k2_commit_raster(const icy2d_grid& g, const int 
 // simulator.py:3940-3965: per-block extrema (min x, max x, min y, max y) as partials
 __device__ __forceinline__ void k2_support_partials(const icy2d_grid& g, const int blk, int only_if_projected) {
   if (only_if_projected && g.control->projected == 0) return;
-  const int n = cell_index(blk);
   double v[4] = {1.0e30, -1.0e30, 1.0e30, -1.0e30};
-  const bool covered = n < cells(g) && g.coverage[n] >= g.threshold;
-  if (!__syncthreads_or(covered ? 1 : 0)) {  // a block without ice: the identities
+  bool covered[kRun], any = false;
+#pragma unroll
+  for (int r = 0; r < kRun; ++r) {
+    const int n = (blk * kRun + r) * kBlock + (int)threadIdx.x;
+    covered[r] = n < cells(g) && g.coverage[n] >= g.threshold;
+    any = any || covered[r];
+  }
+  if (!__syncthreads_or(any ? 1 : 0)) {  // a block without ice: the identities
     if (threadIdx.x < 4) g.partials[blk * 4 + threadIdx.x] = v[threadIdx.x & 1];
     return;
   }
-  if (covered) {
-    const int i = n / g.ny, j = n - i * g.ny;
+  if (any) {
     const Pose p = load_pose(g);
-    if (signed_distance(g, p, i, j) <= 0.0f) {
-      v[0] = (float)(i - p.ox);
-      v[1] = (float)(i + 1 - p.ox);
-      v[2] = (float)(j - p.oy);
-      v[3] = (float)(j + 1 - p.oy);
+#pragma unroll
+    for (int r = 0; r < kRun; ++r) {
+      if (!covered[r]) continue;
+      const int first = (blk * kRun + r) * kBlock;
+      int i, j;
+      row_col(g, first, first + (int)threadIdx.x, i, j);
+      if (signed_distance(g, p, i, j) <= 0.0f) {
+        v[0] = fmin(v[0], (double)(float)(i - p.ox));
+        v[1] = fmax(v[1], (double)(float)(i + 1 - p.ox));
+        v[2] = fmin(v[2], (double)(float)(j - p.oy));
+        v[3] = fmax(v[3], (double)(float)(j + 1 - p.oy));
+      }
     }
   }
   // Minima (even k) and maxima (odd k) over the block: per wave by
@@ -1370,7 +1405,7 @@ __device__ __forceinline__ void k2_outflow_partials(const icy2d_grid& g, const i
 #pragma unroll
     for (int k = 0; k < 5; ++k) {
       const int ni = i + off[k][0], nj = j + off[k][1];
-      open[k] = inside(g, ni, nj) && !wall_at(g, ni, nj);
+      open[k] = !wall_at(g, ni, nj);  // and so inside
       m[k] = open[k] ? at(g, ni, nj) : n;
       label[k] = g.solid[m[k]];
       phase[k] = g.phi[m[k]];
@@ -1597,14 +1632,18 @@ __device__ __forceinline__ void k2_copy_band(const icy2d_grid& g, const int blk)
 }
 // simulator.py:4291-4351
 __device__ __forceinline__ void k2_evaluate_projection(const icy2d_grid& g, const int blk, double lambda) {
-  const int n = cell_index(blk);
   double v[2] = {0.0, 0.0};
-  if (n < cells(g)) {
-    const int i = n / g.ny, j = n - i * g.ny;
+#pragma unroll
+  for (int r = 0; r < kRun; ++r) {
+    const int first = (blk * kRun + r) * kBlock, n = first + (int)threadIdx.x;
+    if (n >= cells(g)) continue;
+    int i, j;
+    row_col(g, first, n, i, j);
+    const double phase = g.phi[n];
+    const bool flagged = pop_get<kPhase>(g.hbuf, g, n) == 1.0f;
     if (fluid_at(g, i, j)) {
-      const double phase = g.phi[n];
       double mapped = phase;
-      const bool adjustable = pop_get<kPhase>(g.hbuf, g, n) == 1.0f;
+      const bool adjustable = flagged;
       if (adjustable) {
         const double e = exp(lambda);
         mapped = phase * e / (1.0 - phase + phase * e);
@@ -1612,8 +1651,8 @@ __device__ __forceinline__ void k2_evaluate_projection(const icy2d_grid& g, cons
       float m32 = (float)mapped;
       if (m32 <= g.cutoff) m32 = 0.0f;
       else if (m32 >= 1.0f - g.cutoff) m32 = 1.0f;
-      v[0] = (double)m32;
-      if (adjustable && g.cutoff < m32 && m32 < 1.0f - g.cutoff) v[1] = (double)m32 * (1.0 - (double)m32);
+      v[0] += (double)m32;
+      if (adjustable && g.cutoff < m32 && m32 < 1.0f - g.cutoff) v[1] += (double)m32 * (1.0 - (double)m32);
     }
   }
   block_partials<2>(v, g.partials, blk);
@@ -1961,18 +2000,25 @@ __device__ __forceinline__ void k2_reset_thermal_diagnostics(const icy2d_grid& g
 // simulator.py:633-714 in control order: volume, energy, base and full
 // capacity (sums), specific energy min, max.
 __device__ __forceinline__ void k2_aperture_partials(const icy2d_grid& g, const int blk) {
-  const int n = cell_index(blk);
   double v[6] = {0.0, 0.0, 0.0, 0.0, 1.0e30, -1.0e30};
-  if (n < cells(g)) {
-    const int i = n / g.ny, j = n - i * g.ny;
+#pragma unroll
+  for (int r = 0; r < kRun; ++r) {
+    const int first = (blk * kRun + r) * kBlock, n = first + (int)threadIdx.x;
+    if (n >= cells(g)) continue;
+    int i, j;
+    row_col(g, first, n, i, j);
     const double vol = g.water_v[n];
-    v[0] = vol;
-    v[1] = g.water_e[n];
-    if (vol > 1.0e-30) v[4] = v[5] = g.water_e[n] / vol;
+    const double energy = g.water_e[n];
+    v[0] += vol;
+    v[1] += energy;
+    if (vol > 1.0e-30) {
+      v[4] = fmin(v[4], energy / vol);
+      v[5] = fmax(v[5], energy / vol);
+    }
     const float phase = clamp01(g.phi[n]);
     if (!wall_at(g, i, j) && g.solid[n] == 0 && phase > g.cutoff) {
-      v[2] = g.area * (double)phase;
-      v[3] = g.area;
+      v[2] += g.area * (double)phase;
+      v[3] += g.area;
     }
   }
   __shared__ double part[6][kBlock / 64];
@@ -2028,14 +2074,16 @@ __device__ __forceinline__ double aperture_target(const icy2d_grid& g, int i, in
 }
 // simulator.py:716-827 (control aperture = {volume, energy, base, full, min, max})
 __device__ __forceinline__ void k2_build_aperture_targets(const icy2d_grid& g, const int blk) {
-  const int n = cell_index(blk);
   const icy2d_control* ctl = g.control;
-  double v[3] = {0.0, 0.0, 0.0};
-  if (n < cells(g)) {
-    const int i = n / g.ny, j = n - i * g.ny;
-    double bs, ss;
-    aperture_scales(ctl, bs, ss);
-    const double low = ctl->aperture[4], high = ctl->aperture[5], total = fmax(0.0, ctl->aperture[0]);
+  double v[3] = {0.0, 0.0, 0.0}, bs, ss;
+  aperture_scales(ctl, bs, ss);
+  const double low = ctl->aperture[4], high = ctl->aperture[5], total = fmax(0.0, ctl->aperture[0]);
+#pragma unroll
+  for (int run = 0; run < kRun; ++run) {
+    const int first = (blk * kRun + run) * kBlock, n = first + (int)threadIdx.x;
+    if (n >= cells(g)) continue;
+    int i, j;
+    row_col(g, first, n, i, j);
     const double target = aperture_target(g, i, j, bs, ss), vol = g.water_v[n];
     double energy = 0.0;
     if (target > 0.0) {
@@ -2062,42 +2110,49 @@ __device__ __forceinline__ void k2_build_aperture_targets(const icy2d_grid& g, c
       }
       sp = fmin(high, fmax(low, sp));
       energy = target * sp;
-      v[1] = target * (sp - low);
-      v[2] = target * (high - sp);
+      v[1] += target * (sp - low);
+      v[2] += target * (high - sp);
     }
     g.target_e[n] = energy;
-    v[0] = energy;
+    v[0] += energy;
   }
   block_partials<3>(v, g.partials, blk);
 }
 // simulator.py:829-859
 // with the new water in v (zeros past the grid) for the totals of its block.
-__device__ __forceinline__ void aperture_transfer_cell(const icy2d_grid& g, int n, double v[2]) {
+__device__ __forceinline__ void aperture_transfer_cell(const icy2d_grid& g, int first, int n, double bs, double ss, double v[2]) {
   if (n >= cells(g)) return;
   const icy2d_control* ctl = g.control;
-  const int i = n / g.ny, j = n - i * g.ny;
+  int i, j;
+  row_col(g, first, n, i, j);
   const double correction = ctl->aperture[1] - ctl->targets[0];
   const double low = ctl->aperture[4], high = ctl->aperture[5], cool = ctl->targets[1], heat = ctl->targets[2];
-  double bs, ss;
-  aperture_scales(ctl, bs, ss);
   const double target = aperture_target(g, i, j, bs, ss);
   double energy = g.target_e[n];
   if (target > 0.0) {
     if (correction < 0.0 && cool > 1.0e-30) energy += fmax(-1.0, correction / cool) * fmax(0.0, energy - low * target);
     else if (correction > 0.0 && heat > 1.0e-30) energy += fmin(1.0, correction / heat) * fmax(0.0, high * target - energy);
   }
-  g.water_v[n] = v[0] = target;
-  g.water_e[n] = v[1] = energy;
+  g.water_v[n] = target;
+  g.water_e[n] = energy;
+  v[0] += target;
+  v[1] += energy;
 }
 __device__ __forceinline__ void k2_apply_aperture_transfer(const icy2d_grid& g, const int blk) {
-  double v[2] = {0.0, 0.0};
-  aperture_transfer_cell(g, cell_index(blk), v);
+  double v[2] = {0.0, 0.0}, bs, ss;
+  aperture_scales(g.control, bs, ss);
+  aperture_transfer_cell(g, blk * (int)blockDim.x, cell_index(blk), bs, ss, v);
 }
 // The transfer and the block sums of what it wrote (k2_water_totals_partials),
 // without reading the water planes again: 14 us at 1024x2048 instead of 12 + 11.
 __device__ __forceinline__ void k2_transfer_partials(const icy2d_grid& g, const int blk) {
-  double v[2] = {0.0, 0.0};
-  aperture_transfer_cell(g, cell_index(blk), v);
+  double v[2] = {0.0, 0.0}, bs, ss;
+  aperture_scales(g.control, bs, ss);
+#pragma unroll
+  for (int r = 0; r < kRun; ++r) {
+    const int first = (blk * kRun + r) * kBlock;
+    aperture_transfer_cell(g, first, first + (int)threadIdx.x, bs, ss, v);
+  }
   block_partials<2>(v, g.partials, blk);
 }
 __device__ __forceinline__ void k2_add_correction_abs(const icy2d_grid& g, const int blk) {
@@ -2106,11 +2161,13 @@ __device__ __forceinline__ void k2_add_correction_abs(const icy2d_grid& g, const
 }
 // simulator.py:861-877
 __device__ __forceinline__ void k2_water_totals_partials(const icy2d_grid& g, const int blk) {
-  const int n = cell_index(blk);
   double v[2] = {0.0, 0.0};
-  if (n < cells(g)) {
-    v[0] = g.water_v[n];
-    v[1] = g.water_e[n];
+#pragma unroll
+  for (int r = 0; r < kRun; ++r) {
+    const int n = (blk * kRun + r) * kBlock + (int)threadIdx.x;
+    if (n >= cells(g)) continue;
+    v[0] += g.water_v[n];
+    v[1] += g.water_e[n];
   }
   block_partials<2>(v, g.partials, blk);
 }
@@ -2437,7 +2494,7 @@ __device__ __forceinline__ void k2_totals_partials(const icy2d_grid& g, const in
 // the block in a batch's prefix table.
 enum Shape : int {
   kCells = 0, kBody, kFaceX, kFaceY, kOne, kTotals, kCells128, kCells512, kBandTiles,
-  kTiles128, kTiles256, kTiles512, kShapes
+  kTiles128, kTiles256, kTiles512, kRuns, kShapes
 };
 static_assert(kShapes == ICY2D_SHAPES, "shape count");
 
@@ -2449,6 +2506,7 @@ long shape_count(const icy2d_grid& g, int shape) {
     case kFaceY: return (long)g.nx * (g.ny + 1);
     case kOne: return 1;
     case kTotals: return cells > body ? cells : body;
+    case kRuns: return (cells + kRun - 1) / kRun;
     case kBandTiles:  // one block of kBlock threads per 16 x 64 band tile
       return (long)((g.nx + kBandI - 1) / kBandI) * ((g.ny + kBandJ - 1) / kBandJ) * kBlock;
     case kTiles128:  // one block per (threads / 64) x 64 collision tile
@@ -2693,11 +2751,11 @@ template <class D> int op_body_fraction(const D& d, int only_if_projected) {
 }
 template <class D> int op_commit_raster(const D& d) { return d.template launch<k2_commit_raster>(kCells); }
 template <class D> int op_contact_support(const D& d, int reduce, int only_if_projected) {
-  NEED(d, kCells, 4);
+  NEED(d, kRuns, 4);
   if (reduce) {
-    TRY(d.template launch<k2_support_partials>(kCells, only_if_projected));
+    TRY(d.template launch<k2_support_partials>(kRuns, only_if_projected));
     // min x, max x, min y, max y into the last four partials slots
-    return d.template finish_tail<k2_support_store>(kCells, 4, TAIL(4), 0x5u, 0xAu, 0u, reduce, only_if_projected);
+    return d.template finish_tail<k2_support_store>(kRuns, 4, TAIL(4), 0x5u, 0xAu, 0u, reduce, only_if_projected);
   }
   return d.template launch<k2_support_store>(kOne, reduce, only_if_projected);
 }
@@ -2762,9 +2820,9 @@ template <class D> int op_dilate_band(const D& d, int radius) {
   return d.template launch<k2_copy_band>(kCells);
 }
 template <class D> int op_evaluate_projection(const D& d, typename D::Real lambda) {
-  NEED(d, kCells, 2);
-  TRY(d.template launch<k2_evaluate_projection>(kCells, lambda));
-  return d.finish(kCells, 2, CTL(water, 1), 0u, 0u, 0u);
+  NEED(d, kRuns, 2);
+  TRY(d.template launch<k2_evaluate_projection>(kRuns, lambda));
+  return d.finish(kRuns, 2, CTL(water, 1), 0u, 0u, 0u);
 }
 template <class D> int op_apply_projection(const D& d, typename D::Real lambda) {
   NEED(d, kCells, 1);
@@ -2813,29 +2871,29 @@ template <class D> int op_finish_melt_momentum(const D& d) {
   return d.template launch<k2_finish_melt_momentum>(kOne);
 }
 template <class D> int op_measure_aperture(const D& d) {
-  NEED(d, kCells, 6);
-  TRY(d.template launch<k2_aperture_partials>(kCells));
-  return d.template finish_tail<k2_check_aperture>(kCells, 6, CTL(aperture, 0), 0x10u, 0x20u, 0u);
+  NEED(d, kRuns, 6);
+  TRY(d.template launch<k2_aperture_partials>(kRuns));
+  return d.template finish_tail<k2_check_aperture>(kRuns, 6, CTL(aperture, 0), 0x10u, 0x20u, 0u);
 }
 template <class D> int op_build_aperture_targets(const D& d) {
-  NEED(d, kCells, 3);
-  TRY(d.template launch<k2_build_aperture_targets>(kCells));
+  NEED(d, kRuns, 3);
+  TRY(d.template launch<k2_build_aperture_targets>(kRuns));
   // the transfer's |energy correction| (simulator.py:829-859) is added as
   // soon as the targets are folded
-  return d.template finish_tail<k2_add_correction_abs>(kCells, 3, CTL(targets, 0), 0u, 0u, 0u);
+  return d.template finish_tail<k2_add_correction_abs>(kRuns, 3, CTL(targets, 0), 0u, 0u, 0u);
 }
 template <class D> int op_apply_aperture_transfer(const D& d) {
   return d.template launch<k2_apply_aperture_transfer>(kCells);
 }
 template <class D> int op_finish_aperture_transfer(const D& d) {
-  NEED(d, kCells, 2);
-  TRY(d.template launch<k2_water_totals_partials>(kCells));
-  return d.finish(kCells, 2, CTL(transfer, 0), 0u, 0u, 0u);
+  NEED(d, kRuns, 2);
+  TRY(d.template launch<k2_water_totals_partials>(kRuns));
+  return d.finish(kRuns, 2, CTL(transfer, 0), 0u, 0u, 0u);
 }
 template <class D> int op_transfer_aperture(const D& d) {
-  NEED(d, kCells, 2);
-  TRY(d.template launch<k2_transfer_partials>(kCells));
-  return d.finish(kCells, 2, CTL(transfer, 0), 0u, 0u, 0u);
+  NEED(d, kRuns, 2);
+  TRY(d.template launch<k2_transfer_partials>(kRuns));
+  return d.finish(kRuns, 2, CTL(transfer, 0), 0u, 0u, 0u);
 }
 template <class D> int op_body_conduction(const D& d, typename D::Real dt) {
   return d.template launch<k2_body_conduction>(kBody, dt);

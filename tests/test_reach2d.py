@@ -8,6 +8,7 @@ import math
 
 import numpy as np
 import pytest
+import torch
 
 from cases2d import submerged_config
 
@@ -66,3 +67,41 @@ def test_kernels_compiled_for_a_storage(storage, step):
         phases.append([case.water_phase.to_numpy() for case in batch.cases])
     for a, b in zip(*phases):
         np.testing.assert_allclose(a, b, rtol=0.0, atol=3 * 9 * 32 * step)
+
+
+@pytest.mark.parametrize("shape", [(12, 520), (21, 512), (24, 43), (33, 31)])
+def test_reductions_over_runs_of_cells(shape):
+    """The sums, minimum and maximum over blocks of four times 256 cells, on
+    rows of more and less than 512 cells and with a remainder of every kind:
+    against NumPy on the same fields (FP64; the order of n terms changes a
+    sum by at most n ulps of the sum of magnitudes)."""
+    from projecticy_amd.iceflow2d import IceFlow2D
+
+    nx, ny = shape
+    config = submerged_config(resolution=shape, water_width_fraction=(nx - 2) / nx, water_height_fraction=24.0 / ny,
+                              ice_width_fraction=4.0 / nx, ice_height_fraction=4.0 / ny, phase_warmup_steps=0)
+    sim = IceFlow2D(config)
+    rng = np.random.default_rng(nx)
+    volume, energy = sim.thermal.water_volume_m2.t, sim.thermal.water_sensible_energy.t
+    g = sim._g
+    scale = torch.from_numpy(rng.uniform(0.5, 1.0, size=shape)).cuda()
+    volume.copy_((volume * scale.reshape(volume.shape)))
+    energy.copy_((energy * scale.reshape(energy.shape) ** 2))
+    sim._call("measure_aperture")
+    control = sim._read_control()
+    v, e = volume.cpu().numpy().reshape(shape), energy.cpu().numpy().reshape(shape)
+    phase = np.clip(sim.water_phase.to_numpy().astype(np.float64), 0.0, 1.0)
+    free = (sim.solid_mask.to_numpy() == 0) & (phase > g.cutoff)
+    b = g.boundary
+    inner = np.zeros(shape, bool)
+    inner[b:nx - b, b:ny - b] = True
+    free &= inner
+    wet = v > 1.0e-30
+    expected = [v.sum(), e.sum(), g.area * phase[free].sum(), g.area * free.sum(), (e[wet] / v[wet]).min(),
+                (e[wet] / v[wet]).max()]
+    np.testing.assert_allclose(np.array(control.aperture[:]), expected, rtol=nx * ny * 2.0 ** -52)
+    sim._call("build_aperture_targets")
+    sim._call("transfer_aperture")
+    control = sim._read_control()
+    np.testing.assert_allclose(np.array(control.transfer[:]), [volume.sum().item(), energy.sum().item()],
+                               rtol=nx * ny * 2.0 ** -52)
