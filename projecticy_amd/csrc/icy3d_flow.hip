@@ -337,7 +337,7 @@ __device__ void general_gradient(const icy3d_grid& g, const Cell& c) {
 // their mirrored neighbours) is staged once in LDS, every thread forms
 // P = S_y S_z, Qy = D_y S_z and Qz = S_y D_z for its column, and the x
 // combination runs in registers over three consecutive slabs.
-constexpr int kGradJ = 4, kGradK = 64, kGradX = 16;
+constexpr int kGradJ = 4, kGradK = 64;
 constexpr int kGradHJ = kGradJ + 2, kGradHK = kGradK + 2, kGradSlab = kGradHJ * kGradHK;
 constexpr int kGradRounds = (kGradSlab + kGradJ * kGradK - 1) / (kGradJ * kGradK);
 
@@ -356,13 +356,13 @@ constexpr unsigned kGradientListBlocks = 2048, kForceListBlocks = 1280;
 // gradients.py:15-20: every phase and coverage dependency of a gradient lies
 // within this many cells.
 constexpr int kGradientRadius = 6;
-// Tiles of box m: ceil(ez / kGradK) x ceil(ey / kGradJ) x ceil(ex / kGradX),
+// Tiles of box m: ceil(ez / kGradK) x ceil(ey / kGradJ) x ceil(ex / slabs),
 // k fastest; the boxes' tiles share one launch.
-__host__ __device__ inline int grad_tiles(const int lo[3], const int hi[3]) {
+__host__ __device__ inline int grad_tiles(const int lo[3], const int hi[3], int slabs) {
   return ((hi[2] - lo[2] + kGradK - 1) / kGradK) * ((hi[1] - lo[1] + kGradJ - 1) / kGradJ) *
-         ((hi[0] - lo[0] + kGradX - 1) / kGradX);
+         ((hi[0] - lo[0] + slabs - 1) / slabs);
 }
-__global__ void __launch_bounds__(kGradJ* kGradK) k_gradients_tiled(icy3d_grid g, BoxList tiles) {
+__global__ void __launch_bounds__(kGradJ* kGradK) k_gradients_tiled(icy3d_grid g, BoxList tiles, int slabs) {
   __shared__ float sp[kGradSlab];
   int m = 0;
   while (m + 1 < tiles.count && (int)blockIdx.x >= tiles.first[m + 1]) ++m;
@@ -376,9 +376,10 @@ __global__ void __launch_bounds__(kGradJ* kGradK) k_gradients_tiled(icy3d_grid g
   const int nk = (box.hi[2] - box.lo[2] + kGradK - 1) / kGradK, nj = (box.hi[1] - box.lo[1] + kGradJ - 1) / kGradJ;
   const int tk = threadIdx.x % kGradK, tj = threadIdx.x / kGradK;
   const int k0 = box.lo[2] + (tile % nk) * kGradK, j0 = box.lo[1] + (tile / nk % nj) * kGradJ;
-  const int x0 = box.lo[0] + tile / nk / nj * kGradX, x_end = min(x0 + kGradX, box.hi[0]);
+  const int x0 = box.lo[0] + tile / nk / nj * slabs, x_end = min(x0 + slabs, box.hi[0]);
   const int j = j0 + tj, k = k0 + tk;
   const bool mine = j < box.hi[1] && k < box.hi[2];
+  int label = 0;  // of the cell that the next slab completes, loaded a slab ahead
   float fetched[kGradRounds];
 #pragma unroll
   for (int r = 0; r < kGradRounds; ++r) {
@@ -401,6 +402,8 @@ __global__ void __launch_bounds__(kGradJ* kGradK) k_gradients_tiled(icy3d_grid g
         fetched[r] = t < kGradSlab ? staged_phi(g, s + 1, j0 - 1 + t / kGradHK, k0 - 1 + t % kGradHK) : 0.0f;
       }
     }
+    const int flag = label;
+    if (s >= x0 && s < x_end && mine) label = g.flag[lin(g, s, j, k)];
     __syncthreads();
     float sz[3], dz[3];
 #pragma unroll
@@ -416,7 +419,6 @@ __global__ void __launch_bounds__(kGradJ* kGradK) k_gradients_tiled(icy3d_grid g
     const int x = s - 1;
     if (x >= x0 && mine) {
       const int n = lin(g, x, j, k);
-      const int flag = g.flag[n];
       if (flag == 0 || flag == 1) {
         store_gradient(g, n, 3.0f * (p - p_m2) * sixth, 3.0f * (qy_m2 + 4.0f * qy_m1 + qy) * sixth,
                        3.0f * (qz_m2 + 4.0f * qz_m1 + qz) * sixth);
@@ -2052,9 +2054,17 @@ int launch_classify_all(const icy3d_grid& g, hipStream_t s) {
 // boxes.  Overlapping boxes write the same values twice.
 int launch_gradients_list(const icy3d_grid& g, const BoxList& L, hipStream_t s) {
   if (!L.count) return 0;
+  // Slabs a block sweeps: 16 where that gives every CU its eight blocks, else
+  // 8 or 4 (a slab is a serial step; two more are read for the halo): with 16
+  // everywhere, and each label loaded at its use, 26 us at 256x128x128 and 15
+  // at 24x20x16, this way 21 and 6.
   BoxList tiles = L;
-  for (int m = 0; m < L.count; ++m) tiles.first[m + 1] = tiles.first[m] + grad_tiles(L.lo[m], L.hi[m]);
-  k_gradients_tiled<<<(unsigned)tiles.first[L.count], kGradJ * kGradK, 0, s>>>(g, tiles);
+  int slabs = 32;
+  do {
+    slabs /= 2;
+    for (int m = 0; m < L.count; ++m) tiles.first[m + 1] = tiles.first[m] + grad_tiles(L.lo[m], L.hi[m], slabs);
+  } while (slabs > 4 && tiles.first[L.count] < 2048);
+  k_gradients_tiled<<<(unsigned)tiles.first[L.count], kGradJ * kGradK, 0, s>>>(g, tiles, slabs);
   k_gradients_general_list<<<kGradientListBlocks, kBlock, 0, s>>>(g, L);
   ICY_LAUNCH_CHECK();
   return 0;
