@@ -162,6 +162,28 @@ __device__ __forceinline__ float phase_get(const float* base, const icy2d_grid& 
 __device__ __forceinline__ void phase_set(float* base, const icy2d_grid& g, int q, int n, float ref, float v) {
   pop_set<kPhase>(base, g, q * cells(g) + n, phase_relative(g) ? v - wq(q) * ref : v);
 }
+// The same for the kernels that are compiled for a storage too.  Whether
+// w_q * ref is fused with the sum or rounded before it is written out there: a
+// stochastic rounding draws another sample for another last bit, and the
+// compiler's choice changes with what else a kernel does with the product.
+template <bool Fused>
+__device__ __forceinline__ float phase_decoded(const icy2d_grid& g, int q, float stored, float ref) {
+#pragma clang fp contract(off)
+  if (!phase_relative(g)) return stored;
+  return Fused ? fmaf(wq(q), ref, stored) : stored + wq(q) * ref;
+}
+template <bool Fused>
+__device__ __forceinline__ float phase_encoded(const icy2d_grid& g, int q, float v, float ref) {
+#pragma clang fp contract(off)
+  if (!phase_relative(g)) return v;
+  return Fused ? fmaf(-wq(q), ref, v) : v - wq(q) * ref;
+}
+// Bit q of Fused: as above for direction q.
+template <unsigned Fused>
+__device__ __forceinline__ void phase_store(float* base, const icy2d_grid& g, int q, int n, float ref, float v) {
+  const float x = (Fused >> q) & 1u ? phase_encoded<true>(g, q, v, ref) : phase_encoded<false>(g, q, v, ref);
+  pop_set<kPhase>(base, g, q * cells(g) + n, x);
+}
 // The saved phase of a cell whose hbuf is read (0 when unused).
 __device__ __forceinline__ float hbuf_ref(const icy2d_grid& g, int n) { return phase_relative(g) ? g.phase_ref[n] : 0.0f; }
 
@@ -172,6 +194,26 @@ __device__ __forceinline__ float momentum_eq(float p, float rho, float ux, float
   float value = 3.0f * wq(Q) * p + wq(Q) * rho * (3.0f * cu + 4.5f * cu * cu - 1.5f * uu);
   if (Q == 0) value -= 3.0f * p;
   return value;
+}
+// c_q . (x, y) without the products by zero (which a compiler has to keep).
+__device__ __forceinline__ float along(int q, float x, float y) {
+  const float cx = (float)cxq(q), cy = (float)cyq(q);
+  return cxq(q) && cyq(q) ? cx * x + cy * y : cxq(q) ? cx * x : cyq(q) ? cy * y : 0.0f;
+}
+// The velocity's part of the momentum equilibrium and the whole from it, for the
+// kernels that are compiled for a storage.  Which operations are fused is
+// written out there (Square: -1.5 u.u): left to the compiler it depends on
+// what else of a kernel shares a product, and a stochastic rounding draws
+// another sample for another last bit.
+template <bool Square>
+__device__ __forceinline__ float momentum_poly(int q, float uu, float ux, float uy) {
+#pragma clang fp contract(off)
+  const float cu = along(q, ux, uy), linear = fmaf(3.0f, cu, 4.5f * cu * cu);
+  return Square ? fmaf(-1.5f, uu, linear) : linear - 1.5f * uu;
+}
+__device__ __forceinline__ float momentum_eq_of(int q, float p, float rho, float poly) {
+  const float value = fmaf(wq(q) * rho, poly, 3.0f * wq(q) * p);
+  return q == 0 ? fmaf(-3.0f, p, value) : value;
 }
 __device__ __forceinline__ float momentum_eq_rt(int q, float p, float rho, float ux, float uy) {
   const float cu = (float)cxq(q) * ux + (float)cyq(q) * uy, uu = ux * ux + uy * uy;
@@ -187,6 +229,14 @@ __device__ __forceinline__ float phase_eq(float phi, float ux, float uy) {
 __device__ __forceinline__ float phase_eq_rt(int q, float phi, float ux, float uy) {
   const float cu = (float)cxq(q) * ux + (float)cyq(q) * uy, uu = ux * ux + uy * uy;
   return wq(q) * phi * (1.0f + 3.0f * cu + 4.5f * cu * cu - 1.5f * uu);
+}
+// The velocity's part of phase_eq, as momentum_poly (Products: 3 c.u + 4.5 (c.u)^2).
+template <bool Products, bool Square>
+__device__ __forceinline__ float phase_poly(int q, float uu, float ux, float uy) {
+#pragma clang fp contract(off)
+  const float cu = along(q, ux, uy);
+  const float linear = Products ? fmaf(4.5f * cu, cu, fmaf(3.0f, cu, 1.0f)) : 1.0f + 3.0f * cu + 4.5f * cu * cu;
+  return Square ? fmaf(-1.5f, uu, linear) : linear - 1.5f * uu;
 }
 // lattice.py:112-115
 __device__ __forceinline__ float mixture(const icy2d_grid& g, float phi) {
@@ -210,6 +260,27 @@ __device__ __forceinline__ void basis(float u, float b[3]) {
     b[2] = 0.5f;
   }
 }
+template <int Q>
+__device__ __forceinline__ float reconstruct_cm(float ux, float uy, const float m[9]) {
+  float bx[3], by[3];
+  basis<cxq(Q)>(ux, bx);
+  basis<cyq(Q)>(uy, by);
+  return bx[0] * by[0] * m[0] + bx[1] * by[0] * m[1] + bx[0] * by[1] * m[2] + bx[2] * by[0] * m[3] +
+         bx[0] * by[2] * m[4] + bx[1] * by[1] * m[5] + bx[2] * by[1] * m[6] + bx[1] * by[2] * m[7] +
+         bx[2] * by[2] * m[8];
+}
+// sums[m] += c_q's raw moment m times v, without the moments that vanish.
+template <int M>
+__device__ __forceinline__ void add_raw(float (&sums)[M], int q, float v) {
+  const int cx = cxq(q), cy = cyq(q);
+  const int k[9] = {1, cx, cy, cx * cx, cy * cy, cx * cy, cx * cx * cy, cx * cy * cy, cx * cx * cy * cy};
+#pragma unroll
+  for (int m = 0; m < M; ++m) {
+    if (k[m] > 0) sums[m] += v;
+    if (k[m] < 0) sums[m] -= v;
+  }
+}
+
 // --------------------------------------------------------------- body
 // The pose transform, the bilinear coverage sample and the signed distance
 // are evaluated in FP64: the cut-link fraction sdf_f / (sdf_f - sdf_s)
@@ -337,40 +408,60 @@ __device__ __forceinline__ float cut_fraction(const icy2d_grid& g, const Pose& p
 }
 
 // ------------------------------------------------------- reductions
-// Wave-wide, the result in every lane: four steps within a row of 16 lanes
-// (pairs, quads, mirrored halves) and two swaps of rows, all between
-// registers.  ds_bpermute shuffles, two a step for FP64, took most of the
-// block sums' time: the aperture's six 31 us at 1024x2048, 17 this way.
+// Wave-wide, the result in every lane: lane l takes in lanes l ^ 32, 16, 8, 4,
+// 2 and 1 in turn, as two swaps of rows and four moves within a row of 16
+// lanes (rotations by 8 and 4, which are l ^ 8 and l ^ 4 on values of that
+// period, then quads and pairs), all between registers.  ds_bpermute shuffles,
+// two a step for FP64, took most of the block sums' time: the aperture's six
+// 31 us at 1024x2048, 17 with a cell a thread.  The order of the adds is part of the
+// results: a stochastically rounded FP16 population hashes its value's bits,
+// so that a sum off by its last bit leads to another sample everywhere.
 template <int Ctrl>
 __device__ __forceinline__ double row_move(double v) {
   const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), Ctrl, 0xf, 0xf, true);
   const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), Ctrl, 0xf, 0xf, true);
   return __hiloint2double(hi, lo);
 }
-// The two values that a swap of 16-lane rows (32-lane halves) leaves in each lane.
+// What a swap of 16-lane rows (32-lane halves) leaves in each lane: of v and w
+// the even rows (lower halves), and the odd rows (upper halves).
 struct Pair {
   double a, b;
 };
-__device__ __forceinline__ Pair swap_rows(double v) {
-  const auto lo = __builtin_amdgcn_permlane16_swap(__double2loint(v), __double2loint(v), false, false);
-  const auto hi = __builtin_amdgcn_permlane16_swap(__double2hiint(v), __double2hiint(v), false, false);
+__device__ __forceinline__ Pair swap_rows(double v, double w) {
+  const auto lo = __builtin_amdgcn_permlane16_swap(__double2loint(v), __double2loint(w), false, false);
+  const auto hi = __builtin_amdgcn_permlane16_swap(__double2hiint(v), __double2hiint(w), false, false);
   return {__hiloint2double((int)hi[0], (int)lo[0]), __hiloint2double((int)hi[1], (int)lo[1])};
 }
-__device__ __forceinline__ Pair swap_halves(double v) {
-  const auto lo = __builtin_amdgcn_permlane32_swap(__double2loint(v), __double2loint(v), false, false);
-  const auto hi = __builtin_amdgcn_permlane32_swap(__double2hiint(v), __double2hiint(v), false, false);
+__device__ __forceinline__ Pair swap_halves(double v, double w) {
+  const auto lo = __builtin_amdgcn_permlane32_swap(__double2loint(v), __double2loint(w), false, false);
+  const auto hi = __builtin_amdgcn_permlane32_swap(__double2hiint(v), __double2hiint(w), false, false);
   return {__hiloint2double((int)hi[0], (int)lo[0]), __hiloint2double((int)hi[1], (int)lo[1])};
+}
+// The last four steps: over the lanes of each row.
+template <class Op>
+__device__ __forceinline__ double row_fold(double v, Op op) {
+  v = op(v, row_move<0x128>(v));   // rotated by 8
+  v = op(v, row_move<0x124>(v));   // rotated by 4
+  v = op(v, row_move<0x4e>(v));    // lanes 2 3 0 1
+  return op(v, row_move<0xb1>(v)); // lanes 1 0 3 2
 }
 template <class Op>
 __device__ __forceinline__ double wave_fold(double v, Op op) {
-  v = op(v, row_move<0xb1>(v));   // lanes 1 0 3 2
-  v = op(v, row_move<0x4e>(v));   // lanes 2 3 0 1
-  v = op(v, row_move<0x141>(v));  // mirrored within 8
-  v = op(v, row_move<0x140>(v));  // mirrored within 16
-  Pair p = swap_rows(v);
+  Pair p = swap_halves(v, v);
   v = op(p.a, p.b);
-  p = swap_halves(v);
-  return op(p.a, p.b);
+  p = swap_rows(v, v);
+  return row_fold(op(p.a, p.b), op);
+}
+// Four values at once, each in wave_fold's order: on return row 0 of the wave
+// (lanes 0 to 15) holds the first's result, rows 1, 2 and 3 the third's, the
+// second's and the fourth's.  A swap of two values leaves the halves of one in
+// the lower lanes and those of the other in the upper, so one fold of 64 lanes
+// and three adds do for four.
+template <class Op>
+__device__ __forceinline__ double wave_fold4(double v0, double v1, double v2, double v3, Op op) {
+  const Pair p = swap_halves(v0, v1), q = swap_halves(v2, v3);
+  const Pair r = swap_rows(op(p.a, p.b), op(q.a, q.b));
+  return row_fold(op(r.a, r.b), op);
 }
 __device__ __forceinline__ double wave_sum(double v) {
   return wave_fold(v, [](double a, double b) { return a + b; });
@@ -397,6 +488,41 @@ __device__ __forceinline__ void block_partials(double (&v)[K], double* partials,
     double total = 0.0;
     for (int w = 0; w < (int)(blockDim.x >> 6); ++w) total += part[threadIdx.x][w];
     partials[blk * K + threadIdx.x] = total;
+  }
+}
+// Reductions over all cells take kRun cells a thread (kRuns): the FP64 wave
+// sums, the quotients that are the same for all cells and the block sums' fold
+// were a light kernel's largest part.  Each run of kBlock cells keeps its own
+// partials, those of a block of its own, so the sums' order is the one of the
+// kernels with a cell a thread; the four runs' wave sums share their steps.
+// Over the 64-case ensemble, with a cell a thread and this way: evaluation 47
+// and 26 us, aperture 74 and 57, targets 76 and 60, transfer 81 and 74, and
+// support (minima and maxima only) 46 and 22.
+constexpr int kRun = 4;
+__device__ __forceinline__ int run_blocks(const icy2d_grid& g) { return (cells(g) + kBlock - 1) / kBlock; }
+// Writes the sums (minima, maxima: bit k of the masks) of v[r][0..K) over run r
+// of the block to partials[(blk * kRun + r) * K + k].
+template <int K, unsigned kMins = 0u, unsigned kMaxs = 0u>
+__device__ __forceinline__ void run_partials(const icy2d_grid& g, double (&v)[kRun][K], int blk) {
+  static_assert(kRun == 4, "a run for each row of 16 lanes");
+  __shared__ double part[kRun][K][kBlock / 64];
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int row = lane >> 4, run = (row & 1) * 2 + (row >> 1);  // the run whose result wave_fold4 leaves in the row
+  auto combine = [](int k, double a, double b) {
+    return (kMins >> k) & 1u ? fmin(a, b) : (kMaxs >> k) & 1u ? fmax(a, b) : a + b;
+  };
+#pragma unroll
+  for (int k = 0; k < K; ++k) {
+    const double s = wave_fold4(v[0][k], v[1][k], v[2][k], v[3][k], [&](double a, double b) { return combine(k, a, b); });
+    if ((lane & 15) == 0) part[run][k][wave] = s;
+  }
+  __syncthreads();
+  if ((int)threadIdx.x < kRun * K) {
+    const int r = (int)threadIdx.x / K, k = (int)threadIdx.x - r * K;
+    double total = part[r][k][0];
+#pragma unroll
+    for (int w = 1; w < kBlock / 64; ++w) total = combine(k, total, part[r][k][w]);
+    if (blk * kRun + r < run_blocks(g)) g.partials[(blk * kRun + r) * K + k] = total;
   }
 }
 // Folds partials[b * K + k] over b in a fixed order: one block per k,
@@ -434,12 +560,6 @@ __global__ void __launch_bounds__(kFinishThreads) k2_finish(const double* __rest
   finish_fold(partials, blocks, K, (int)blockIdx.x, out, min_mask, max_mask, add_mask);
 }
 
-// Reductions over all cells take kRun cells a thread (kRuns): the FP64 wave
-// sums, the quotients that are the same for all cells and the block sums' fold
-// were a light kernel's largest part (over the 64-case ensemble: evaluation 47
-// to 25 us, support 46 to 22, aperture 74 to 54, its targets 76 to 58, the
-// transfer 81 to 72).
-constexpr int kRun = 4;
 __device__ __forceinline__ int cell_index(int blk) { return blk * (int)blockDim.x + (int)threadIdx.x; }
 
 // ---------------------------------------------------- geometry kernels
@@ -743,13 +863,12 @@ __device__ __forceinline__ PhaseStencil phase_stencil(const icy2d_grid& g, int i
 
 // Tao single-node reflection into the cut link's outgoing slot and its
 // momentum exchange (simulator.py:4798-4866).  Returns true when a link was cut.
-// (ax, ay): the cell's force density, as the collision has just computed it.
-__device__ __forceinline__ bool prepare_cut_links(const icy2d_grid& g, const Pose& p, int i, int j, float ax, float ay,
-                                                  float raw[9], double load[3]) {
+// pdyn and poly: the cell's dynamic pressure and momentum_poly of its velocity
+// with half its force density, as the collision has just computed them.
+__device__ __forceinline__ bool prepare_cut_links(const icy2d_grid& g, const Pose& p, int i, int j, float pdyn,
+                                                  const float poly[9], float raw[9], double load[3]) {
   const int N = cells(g), n = at(g, i, j);
   const float rho = mixture(g, g.phi[n]);
-  const float pdyn = g.p[n] - g.p_ref[j];
-  const float ux = g.u[n] + 0.5f * ax, uy = g.u[N + n] + 0.5f * ay;
   float prepared[9];
 #pragma unroll
   for (int q = 0; q < 9; ++q) prepared[q] = raw[q];
@@ -763,13 +882,15 @@ __device__ __forceinline__ bool prepare_cut_links(const icy2d_grid& g, const Pos
     float ub[2];
     body_velocity(p, bx, by, ub);
     const int o = oppq(q);
-    const float noneq = pop_get<kMomentum>(g.f, g, q * N + n) - momentum_eq_rt(q, pdyn, rho, ux, uy);
+    const float noneq = pop_get<kMomentum>(g.f, g, q * N + n) - momentum_eq_of(q, pdyn, rho, poly[q]);
     const float wall = momentum_eq_rt(o, pdyn, rho, ub[0], ub[1]);
     const float reflected = (wall + noneq + eta * raw[o]) / (1.0f + eta);
     prepared[q] = reflected;
     float ix = ((float)cxq(q) - ub[0]) * raw[q] - ((float)-cxq(q) - ub[0]) * reflected;
     float iy = ((float)cyq(q) - ub[1]) * raw[q] - ((float)-cyq(q) - ub[1]) * reflected;
-    const float pref = (1.0f - eta) * g.p_ref[j] + eta * g.p_ref[nj];
+    // (1 - eta) p_ref[j] + eta p_ref[nj]; written out as either product could be the fused one
+    const float keep = 1.0f - eta, own_ref = g.p_ref[j];
+    const float pref = cyq(q) ? fmaf(keep, own_ref, eta * g.p_ref[nj]) : fmaf(eta, own_ref, keep * own_ref);
     ix += 6.0f * wq(q) * pref * (float)cxq(q);
     iy += 6.0f * wq(q) * pref * (float)cyq(q);
     const double rx = (double)(bx - p.cx), ry = (double)(by - p.cy);
@@ -913,24 +1034,24 @@ __device__ __forceinline__ void load_own(const icy2d_grid& g, int n, int with_mo
 // cut links' momentum exchange is added to load.
 // Populations are moved by kernels compiled for their storage (one_case):
 // with a branch around each access an FP16 load was converted, and so waited
-// for, before the next was issued (over the 64-case ensemble 1052 us, 628).
-// The reference forms the equilibria's and forces' moments as sums over the
-// nine directions; they are polynomials in u (momentum: raw moments of the
-// Liang equilibrium and its source; phase: central moments of the quadratic
-// equilibrium and of w_q c.n), so they are written down here, and the
-// populations come back from the moments one axis at a time.  The body's
-// pose (FP64 sine and cosine) is needed beside the ice only: near.  The sums
-// and a pose in every lane took 247 us at 1024x2048, this 180, 157 with the
-// cell's own values loaded before the block waits for its window, and 132 with
-// the window's loads in one go.
-template <class W>
+// for, before the next was issued.
+// The moments of the populations, equilibria and forces are sums over the nine
+// directions in the reference's order, which is part of the results: the
+// momentum populations are small differences of terms of order one (the same
+// moments as polynomials in u moved them by 2e-4 in eight steps), and a
+// stochastically rounded FP16 one draws another sample for another last bit.
+// What costs nothing is left out: the products by a direction's zeros and the
+// vanishing moments (a compiler has to keep 0 * x), and the body's pose (FP64
+// sine and cosine) where no neighbour is ice.  Bound by the vector ALUs: 149 us
+// at 1024x2048 (its bytes take 85) and 699 over the 64-case ensemble; 247 and
+// 1503 with all products, a pose in every lane and branches around the loads.
+template <bool Push, class W>
 __device__ __forceinline__ void collide_cell(const icy2d_grid& g, const OwnCell& own, bool near, const Pose& pose,
                                              const W& tile, int a0, int b0, int av, int bv, int i, int j, int n,
                                              int with_momentum, float pf[9], float ph[9], float& ax, float& ay, double load[3]) {
   const int N = cells(g);
   const float phi = tile.phi[a0][b0];
   const PhaseStencil st = phase_stencil_tile(tile, a0, b0, phi);
-  const float third = 1.0f / 3.0f;
   if (with_momentum) {
     // _fluid_force_viscosity_and_gradient (simulator.py:3241-3368)
     const float bounded = clamp01(phi), rho_b = g.rho_w * bounded + g.rho_a * (1.0f - bounded);
@@ -940,9 +1061,14 @@ __device__ __forceinline__ void collide_cell(const icy2d_grid& g, const OwnCell&
     const float temperature = (float)(v > 1.0e-30 ? g.t_melt + own.water_e / (g.rho_w_si * g.cp_w * v) : g.t_air);
     const float ratio = -g.expansion * (temperature - g.t_ref);
     const float ww = clamp01(2.0f * bounded - 1.0f);
-    const float weight = anomaly_rho + ww * g.rho_w * ratio;
+    float fx = anomaly_rho * g.gx, fy = anomaly_rho * g.gy;
+    fx += ww * g.rho_w * ratio * g.gx;
+    fy += ww * g.rho_w * ratio * g.gy;
+    fx /= rho_b;
+    fy /= rho_b;
     const float chemical = 4.0f * beta * bounded * (bounded - 1.0f) * (bounded - 0.5f) - kappa * st.laplacian;
-    const float fx = (weight * g.gx + chemical * st.g[0]) / rho_b, fy = (weight * g.gy + chemical * st.g[1]) / rho_b;
+    fx += chemical * st.g[0] / rho_b;
+    fy += chemical * st.g[1] / rho_b;
     const float ux0 = own.u[0], uy0 = own.u[1];
     float gxx = 0.0f, gxy = 0.0f, gyx = 0.0f, gyy = 0.0f;
 #pragma unroll
@@ -973,46 +1099,38 @@ __device__ __forceinline__ void collide_cell(const icy2d_grid& g, const OwnCell&
     const float Fx = rho * ax, Fy = rho * ay, drho = g.rho_w - g.rho_a;
     const float gsx = st.source[0], gsy = st.source[1];
     // Raw moments m = {00, 10, 01, 20, 02, 11, 21, 12, 22}.
-    float f[9];
+    float raw[6] = {0, 0, 0, 0, 0, 0}, eq[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0}, src[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0}, poly[9];
 #pragma unroll
-    for (int q = 0; q < 9; ++q) f[q] = pop_value<kMomentum>(g, own.f[q]);
-    const float east = f[1] + f[5] + f[8], west = f[3] + f[6] + f[7];
-    const float north = f[2] + f[5] + f[6], south = f[4] + f[7] + f[8];
-    const float raw0 = f[0] + f[2] + f[4] + east + west, raw1 = east - west, raw2 = north - south;
-    const float raw_diff = (f[1] + f[3]) - (f[2] + f[4]);                 // 20 - 02
-    const float raw5 = (f[5] + f[7]) - (f[6] + f[8]);
-    const float uu = ux * ux + uy * uy, ugx = drho * ux * gsx, ugy = drho * uy * gsy;
-    const float eq5 = rho * ux * uy;
-    const float src0 = ugx + ugy, src5 = drho * (ux * gsy + uy * gsx) * third;
+    for (int q = 0; q < 9; ++q) {
+      add_raw(raw, q, pop_value<kMomentum>(g, own.f[q]));
+      poly[q] = momentum_poly<true>(q, ux * ux + uy * uy, ux, uy);
+      add_raw(eq, q, momentum_eq_of(q, pdyn, rho, poly[q]));
+      if (q > 0) add_raw(src, q, wq(q) * 3.0f * (along(q, Fx, Fy) + drho * along(q, ux, uy) * along(q, gsx, gsy)));
+    }
     const float w_phys = 1.0f / tau, w_shear = 1.0f / shear_tau;
     const float sp = 1.0f - 0.5f * w_phys, ss = 1.0f - 0.5f * w_shear;
     float post[9];
-    post[0] = raw0 - w_phys * raw0 + sp * src0;
-    post[1] = raw1 - w_phys * (raw1 - rho * ux) + sp * Fx;
-    post[2] = raw2 - w_phys * (raw2 - rho * uy) + sp * Fy;
-    // 20 + 02 relaxes fully: 2 p + rho u.u + (2/3) drho (u.g); 20 - 02 with the shear rate.
-    const float trace = 2.0f * pdyn + rho * uu + 2.0f * third * src0;
-    const float eq_diff = rho * (ux * ux - uy * uy), src_diff = 2.0f * third * (ugx - ugy);
-    const float post_diff = raw_diff - w_shear * (raw_diff - eq_diff) + ss * src_diff;
+#pragma unroll
+    for (int m = 0; m < 3; ++m) post[m] = raw[m] - w_phys * (raw[m] - eq[m]) + sp * src[m];
+    const float trace = eq[3] + eq[4] + 0.5f * (src[3] + src[4]);
+    const float diff = raw[3] - raw[4];
+    const float post_diff = diff - w_shear * (diff - (eq[3] - eq[4])) + ss * (src[3] - src[4]);
     post[3] = 0.5f * (trace + post_diff);
     post[4] = 0.5f * (trace - post_diff);
-    post[5] = raw5 - w_shear * (raw5 - eq5) + ss * src5;
-    post[6] = third * (rho * uy + 0.5f * Fy);
-    post[7] = third * (rho * ux + 0.5f * Fx);
-    post[8] = third * (pdyn + rho * uu + 0.5f * src0);
-    // The inverse at u = 0.
+    post[5] = raw[5] - w_shear * (raw[5] - eq[5]) + ss * src[5];
+#pragma unroll
+    for (int m = 6; m < 9; ++m) post[m] = eq[m] + 0.5f * src[m];
+    // reconstruct_cm at u = 0: factors 1, 1/2 and 1/4, so every product is exact.
     pf[0] = post[0] - post[3] - post[4] + post[8];
-    const float h20 = post[3] - post[8], h10 = post[1] - post[7], h02 = post[4] - post[8], h01 = post[2] - post[6];
-    pf[1] = 0.5f * (h20 + h10);
-    pf[3] = 0.5f * (h20 - h10);
-    pf[2] = 0.5f * (h02 + h01);
-    pf[4] = 0.5f * (h02 - h01);
-    const float d_same = post[8] + post[5], d_other = post[8] - post[5], e_same = post[6] + post[7], e_other = post[6] - post[7];
-    pf[5] = 0.25f * (d_same + e_same);
-    pf[7] = 0.25f * (d_same - e_same);
-    pf[6] = 0.25f * (d_other + e_other);
-    pf[8] = 0.25f * (d_other - e_other);
-    if (near) prepare_cut_links(g, pose, i, j, ax, ay, pf, load);
+    pf[1] = 0.5f * (post[1] + post[3] - post[7] - post[8]);
+    pf[2] = 0.5f * (post[2] + post[4] - post[6] - post[8]);
+    pf[3] = 0.5f * (post[3] - post[1] + post[7] - post[8]);
+    pf[4] = 0.5f * (post[4] - post[2] + post[6] - post[8]);
+    pf[5] = 0.25f * (post[5] + post[6] + post[7] + post[8]);
+    pf[6] = 0.25f * (post[6] - post[5] - post[7] + post[8]);
+    pf[7] = 0.25f * (post[5] - post[6] - post[7] + post[8]);
+    pf[8] = 0.25f * (post[7] - (post[5] + post[6]) + post[8]);
+    if (near) prepare_cut_links(g, pose, i, j, pdyn, poly, pf, load);
   } else {
     ax = g.a[n];
     ay = g.a[N + n];
@@ -1022,47 +1140,40 @@ __device__ __forceinline__ void collide_cell(const icy2d_grid& g, const OwnCell&
   const float rate = 1.0f / (3.0f * g.mobility + 0.5f);
   const float norm = sqrtf(st.g[0] * st.g[0] + st.g[1] * st.g[1]) + 1.0e-14f;
   const float compression = 4.0f * phi * (1.0f - phi) / g.width;
-  // First moments of w_q compression (c.n), which vanish at even order.
-  const float A = third * compression * (st.g[0] / norm), B = third * compression * (st.g[1] / norm);
-  float h[9];
-#pragma unroll
-  for (int q = 0; q < 9; ++q) {  // as phase_get
-    const float value = pop_value<kPhase>(g, own.h[q]);
-    h[q] = phase_relative(g) ? value + wq(q) * phi : value;
-  }
-  const float east = h[1] + h[5] + h[8], west = h[3] + h[6] + h[7];
-  const float north = h[2] + h[5] + h[6], south = h[4] + h[7] + h[8];
-  const float total = h[0] + h[2] + h[4] + east + west;
-  const float r10 = (east - west) - ux * total, r01 = (north - south) - uy * total;
-  const float uxuy = ux * uy;
-  // Central moments K[a][b] of x power a and y power b.
-  float K[3][3];
-  K[0][0] = phi;
-  K[1][0] = r10 - rate * r10 + (1.0f - 0.5f * rate) * A;
-  K[0][1] = r01 - rate * r01 + (1.0f - 0.5f * rate) * B;
-  K[2][0] = third * phi - ux * A;
-  K[0][2] = third * phi - uy * B;
-  K[1][1] = -0.5f * (uy * A + ux * B);
-  K[2][1] = -phi * ux * uxuy + 0.5f * (third * B + 2.0f * uxuy * A + ux * ux * B);
-  K[1][2] = -phi * uy * uxuy + 0.5f * (third * A + 2.0f * uxuy * B + uy * uy * A);
-  K[2][2] = phi * (third * third + 3.0f * uxuy * uxuy) - third * (uy * B + ux * A) - uxuy * (uy * A + ux * B);
-  float bx[3][3], by[3][3];  // of c = 0, +1, -1
-  basis<0>(ux, bx[0]);
-  basis<1>(ux, bx[1]);
-  basis<-1>(ux, bx[2]);
-  basis<0>(uy, by[0]);
-  basis<1>(uy, by[1]);
-  basis<-1>(uy, by[2]);
-  float row[3][3];  // [c_x][power of y]
-#pragma unroll
-  for (int c = 0; c < 3; ++c)
-#pragma unroll
-    for (int b = 0; b < 3; ++b) row[c][b] = bx[c][0] * K[0][b] + bx[c][1] * K[1][b] + bx[c][2] * K[2][b];
+  const float nx_ = st.g[0] / norm, ny_ = st.g[1] / norm;
+  // Central moments, m = {00, 10, 01, 20, 02, 11, 21, 12, 22}.
+  const float uu = ux * ux + uy * uy;
+  float r10 = 0.0f, r01 = 0.0f, eq[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0}, src[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
 #pragma unroll
   for (int q = 0; q < 9; ++q) {
-    const int cx = cxq(q) == 0 ? 0 : cxq(q) > 0 ? 1 : 2, cy = cyq(q) == 0 ? 0 : cyq(q) > 0 ? 1 : 2;
-    ph[q] = by[cy][0] * row[cx][0] + by[cy][1] * row[cx][1] + by[cy][2] * row[cx][2];
+    const float rx = (float)cxq(q) - ux, ry = (float)cyq(q) - uy;
+    const float hv = phase_decoded<true>(g, q, pop_value<kPhase>(g, own.h[q]), phi);
+    const float he = wq(q) * phi * phase_poly<!Push, !Push>(q, uu, ux, uy);
+    const float force = wq(q) * compression * along(q, nx_, ny_);
+    const float rx2 = rx * rx, ry2 = ry * ry;
+    const float k[9] = {1.0f, rx, ry, rx2, ry2, rx * ry, rx2 * ry, rx * ry2, rx2 * ry2};
+    r10 += hv * rx;
+    r01 += hv * ry;
+#pragma unroll
+    for (int m = 0; m < 9; ++m) {
+      eq[m] += he * k[m];
+      if (q > 0) src[m] += force * k[m];
+    }
   }
+  float post[9];
+#pragma unroll
+  for (int m = 0; m < 9; ++m) post[m] = eq[m] + 0.5f * src[m];
+  post[1] = r10 - rate * (r10 - eq[1]) + (1.0f - 0.5f * rate) * src[1];
+  post[2] = r01 - rate * (r01 - eq[2]) + (1.0f - 0.5f * rate) * src[2];
+  ph[0] = reconstruct_cm<0>(ux, uy, post);
+  ph[1] = reconstruct_cm<1>(ux, uy, post);
+  ph[2] = reconstruct_cm<2>(ux, uy, post);
+  ph[3] = reconstruct_cm<3>(ux, uy, post);
+  ph[4] = reconstruct_cm<4>(ux, uy, post);
+  ph[5] = reconstruct_cm<5>(ux, uy, post);
+  ph[6] = reconstruct_cm<6>(ux, uy, post);
+  ph[7] = reconstruct_cm<7>(ux, uy, post);
+  ph[8] = reconstruct_cm<8>(ux, uy, post);
 }
 // Whether one of the cell's eight neighbours is ice (the window's kinds).
 template <class W>
@@ -1094,7 +1205,8 @@ __device__ __forceinline__ void k2_collide(const icy2d_grid& g, const int blk, i
     const bool near = beside_ice(tile, li + 1, lj + 1);
     Pose pose = {};
     if (near) pose = load_pose(g);
-    collide_cell(g, own, near, pose, tile, li + 2, lj + 2, li + 1, lj + 1, i, j, n, with_momentum, pf, ph, ax, ay, load);
+    collide_cell<false>(g, own, near, pose, tile, li + 2, lj + 2, li + 1, lj + 1, i, j, n, with_momentum, pf, ph, ax, ay,
+                        load);
     if (with_momentum) {
       g.a[n] = ax;
       g.a[N + n] = ay;
@@ -1102,7 +1214,7 @@ __device__ __forceinline__ void k2_collide(const icy2d_grid& g, const int blk, i
       for (int q = 0; q < 9; ++q) pop_set<kMomentum>(g.fbuf, g, q * N + n, pf[q]);
     }
 #pragma unroll
-    for (int q = 0; q < 9; ++q) phase_set(g.hbuf, g, q, n, phi, ph[q]);
+    for (int q = 0; q < 9; ++q) phase_store<0x1u>(g.hbuf, g, q, n, phi, ph[q]);
     if (phase_relative(g)) g.phase_ref[n] = phi;
   }
   if (with_momentum) block_partials<3>(load, g.partials, blk);
@@ -1118,7 +1230,11 @@ __device__ __forceinline__ void k2_prepare_cut_links(const icy2d_grid& g, const 
       float raw[9];
 #pragma unroll
       for (int q = 0; q < 9; ++q) raw[q] = pop_get<kMomentum>(g.fbuf, g, q * N + n);
-      prepare_cut_links(g, load_pose(g), i, j, g.a[n], g.a[N + n], raw, load);
+      const float ux = g.u[n] + 0.5f * g.a[n], uy = g.u[N + n] + 0.5f * g.a[N + n];
+      float poly[9];
+#pragma unroll
+      for (int q = 0; q < 9; ++q) poly[q] = momentum_poly<true>(q, ux * ux + uy * uy, ux, uy);
+      prepare_cut_links(g, load_pose(g), i, j, g.p[n] - g.p_ref[j], poly, raw, load);
 #pragma unroll
       for (int q = 0; q < 9; ++q) pop_set<kMomentum>(g.fbuf, g, q * N + n, raw[q]);
     }
@@ -1135,11 +1251,11 @@ __device__ __forceinline__ void pull(const icy2d_grid& g, const Pose& pose, int 
   if (Q == 0 || (inside(g, si, sj) && fluid_at(g, si, sj))) {
     const int m = Q == 0 ? n : at(g, si, sj);
     if (!phase_only) fq = pop_get<kMomentum>(g.fbuf, g, Q * N + m);
-    hq = phase_get(g.hbuf, g, Q, m, hbuf_ref(g, m));
+    hq = phase_decoded<false>(g, Q, pop_get<kPhase>(g.hbuf, g, Q * N + m), hbuf_ref(g, m));
   } else {
     constexpr int out = oppq(Q);  // own population sent towards (si, sj)
     if (!phase_only) fq = pop_get<kMomentum>(g.fbuf, g, out * N + n);
-    float ho = phase_get(g.hbuf, g, out, n, hbuf_ref(g, n));
+    float ho = phase_decoded<false>(g, out, pop_get<kPhase>(g.hbuf, g, out * N + n), hbuf_ref(g, n));
     if (inside(g, si, sj) && g.solid[at(g, si, sj)] == 1) {
       const float eta = cut_fraction(g, pose, i, j, si, sj);
       float ub[2];
@@ -1191,8 +1307,7 @@ __device__ __forceinline__ void k2_stream(const icy2d_grid& g, const int blk, in
     } else {
 #pragma unroll
       for (int q = 0; q < 9; ++q) {
-        const float value = pop_value<kPhase>(g, own_h[q]);
-        h[q] = phase_relative(g) ? value + wq(q) * phi_old : value;  // as phase_get
+        h[q] = phase_decoded<true>(g, q, pop_value<kPhase>(g, own_h[q]), phi_old);
         if (!po) f[q] = pop_value<kMomentum>(g, own_f[q]);
       }
     }
@@ -1206,7 +1321,7 @@ __device__ __forceinline__ void k2_stream(const icy2d_grid& g, const int blk, in
     if (pulling || (update && phase_relative(g))) {
 #pragma unroll
       for (int q = 0; q < 9; ++q) {
-        phase_set(g.h, g, q, n, phi, h[q]);
+        phase_store<0x23u>(g.h, g, q, n, phi, h[q]);
         if (pulling && !po) pop_set<kMomentum>(g.f, g, q * N + n, f[q]);
       }
     }
@@ -1275,18 +1390,18 @@ __device__ __forceinline__ void k2_collide_push(const icy2d_grid& g, const int b
       if (near) pose = load_pose(g);
       const float phi = tile.phi[li + 2][lj + 2];
       float pf[9], ph[9], ax, ay;
-      collide_cell(g, own, near, pose, tile, li + 2, lj + 2, li + 1, lj + 1, i, j, n, 1, pf, ph, ax, ay, load);
+      collide_cell<true>(g, own, near, pose, tile, li + 2, lj + 2, li + 1, lj + 1, i, j, n, 1, pf, ph, ax, ay, load);
       g.a[n] = ax;
       g.a[N + n] = ay;
       pop_set<kMomentum>(g.fbuf, g, n, pf[0]);
-      phase_set(g.hbuf, g, 0, n, phi, ph[0]);
+      phase_store<0x1u>(g.hbuf, g, 0, n, phi, ph[0]);
 #pragma unroll
       for (int q = 1; q < 9; ++q) {
         const int di = cxq(q), dj = cyq(q);
         if (tile.fluid[li + 2 + di][lj + 2 + dj]) {
           const int m = at(g, i + di, j + dj);
           pop_set<kMomentum>(g.fbuf, g, q * N + m, pf[q]);
-          phase_set(g.hbuf, g, q, m, phase_relative(g) ? tile.phi[li + 2 + di][lj + 2 + dj] : 0.0f, ph[q]);
+          phase_store<0u>(g.hbuf, g, q, m, phase_relative(g) ? tile.phi[li + 2 + di][lj + 2 + dj] : 0.0f, ph[q]);
         } else {
           float ho = ph[q];
           if (tile.kind[li + 1 + di][lj + 1 + dj] == 1) {
@@ -1297,7 +1412,7 @@ __device__ __forceinline__ void k2_collide_push(const icy2d_grid& g, const int b
           }
           const int o = oppq(q);
           pop_set<kMomentum>(g.fbuf, g, o * N + n, pf[q]);
-          phase_set(g.hbuf, g, o, n, phi, ho);
+          phase_store<0u>(g.hbuf, g, o, n, phi, ho);
         }
       }
     } else {
@@ -1448,20 +1563,24 @@ __device__ __forceinline__ void k2_store_outflow(const icy2d_grid& g, const int 
 __device__ __forceinline__ void lift_phase(const icy2d_grid& g, int n, int j, float old_phase, float new_phase) {
   const int N = cells(g);
   const float ux = g.u[n], uy = g.u[N + n], pdyn = g.p[n] - g.p_ref[j];
-  const float ro = mixture(g, old_phase), rn = mixture(g, new_phase);
+  const float ro = mixture(g, old_phase), rn = mixture(g, new_phase), uu = ux * ux + uy * uy;
 #pragma unroll
-  for (int q = 0; q < 9; ++q)
-    pop_add<kMomentum>(g.f, g, q * N + n, momentum_eq_rt(q, pdyn, rn, ux, uy) - momentum_eq_rt(q, pdyn, ro, ux, uy));
+  for (int q = 0; q < 9; ++q) {
+    const float poly = momentum_poly<false>(q, uu, ux, uy);
+    pop_add<kMomentum>(g.f, g, q * N + n, momentum_eq_of(q, pdyn, rn, poly) - momentum_eq_of(q, pdyn, ro, poly));
+  }
   const float stored = g.phi[n];
   float lifted[9], sum = 0.0f;
 #pragma unroll
   for (int q = 0; q < 9; ++q) {
-    lifted[q] = phase_get(g.h, g, q, n, stored) + phase_eq_rt(q, new_phase, ux, uy) - phase_eq_rt(q, old_phase, ux, uy);
+    const float poly = phase_poly<false, false>(q, uu, ux, uy);
+    lifted[q] = fmaf(wq(q) * new_phase, poly, phase_decoded<true>(g, q, pop_get<kPhase>(g.h, g, q * N + n), stored));
+    lifted[q] = fmaf(-(wq(q) * old_phase), poly, lifted[q]);
     sum += lifted[q];
   }
   lifted[0] += new_phase - sum;
 #pragma unroll
-  for (int q = 0; q < 9; ++q) phase_set(g.h, g, q, n, new_phase, lifted[q]);
+  for (int q = 0; q < 9; ++q) phase_store<0x1u>(g.h, g, q, n, new_phase, lifted[q]);
   g.phi[n] = new_phase;
 }
 // simulator.py:4150-4229
@@ -1483,30 +1602,37 @@ __device__ __forceinline__ void k2_clip_phase(const icy2d_grid& g, const int blk
         const float pdyn = g.p[n] - g.p_ref[j];
         const float ro = mixture(g, old_phase), rn = mixture(g, bounded);
 #pragma unroll
-        for (int q = 0; q < 9; ++q)
-          pop_add<kMomentum>(g.f, g, q * N + n, momentum_eq_rt(q, pdyn, rn, ux, uy) - momentum_eq_rt(q, pdyn, ro, ux, uy));
+        for (int q = 0; q < 9; ++q) {
+          const float poly = momentum_poly<false>(q, ux * ux + uy * uy, ux, uy);
+          pop_add<kMomentum>(g.f, g, q * N + n, momentum_eq_of(q, pdyn, rn, poly) - momentum_eq_of(q, pdyn, ro, poly));
+        }
       }
       float h[9], l1 = 0.0f;
 #pragma unroll
       for (int q = 0; q < 9; ++q) {
-        const float value = pop_value<kPhase>(g, own[q]);
-        h[q] = phase_relative(g) ? value + wq(q) * old_phase : value;  // as phase_get
+        h[q] = phase_decoded<true>(g, q, pop_value<kPhase>(g, own[q]), old_phase);
         l1 += fabsf(h[q]);
       }
       const bool regularize = (bounded == 0.0f || bounded == 1.0f) && (double)l1 > max_bulk_l1;
       if (regularize || bounded != old_phase) {
         const float ux = g.u[n], uy = g.u[N + n];
         const float px = ux + 0.5f * g.a[n], py = uy + 0.5f * g.a[N + n];
+        if (regularize) {
+#pragma unroll
+          for (int q = 0; q < 9; ++q) h[q] = wq(q) * bounded * phase_poly<true, false>(q, px * px + py * py, px, py);
+        } else {
+#pragma unroll
+          for (int q = 0; q < 9; ++q) {
+            const float poly = phase_poly<true, false>(q, ux * ux + uy * uy, ux, uy);
+            h[q] = fmaf(-(wq(q) * old_phase), poly, fmaf(wq(q) * bounded, poly, h[q]));
+          }
+        }
         float sum = 0.0f;
 #pragma unroll
-        for (int q = 0; q < 9; ++q) {
-          h[q] = regularize ? phase_eq_rt(q, bounded, px, py)
-                            : h[q] + phase_eq_rt(q, bounded, ux, uy) - phase_eq_rt(q, old_phase, ux, uy);
-          sum += h[q];
-        }
+        for (int q = 0; q < 9; ++q) sum += h[q];
         h[0] += bounded - sum;
 #pragma unroll
-        for (int q = 0; q < 9; ++q) phase_set(g.h, g, q, n, bounded, h[q]);
+        for (int q = 0; q < 9; ++q) phase_store<0u>(g.h, g, q, n, bounded, h[q]);
       }
       g.phi[n] = bounded;
       v[0] = (double)bounded;
@@ -1632,7 +1758,7 @@ __device__ __forceinline__ void k2_copy_band(const icy2d_grid& g, const int blk)
 }
 // simulator.py:4291-4351
 __device__ __forceinline__ void k2_evaluate_projection(const icy2d_grid& g, const int blk, double lambda) {
-  double v[2] = {0.0, 0.0};
+  double v[kRun][2] = {};
 #pragma unroll
   for (int r = 0; r < kRun; ++r) {
     const int first = (blk * kRun + r) * kBlock, n = first + (int)threadIdx.x;
@@ -1651,11 +1777,11 @@ __device__ __forceinline__ void k2_evaluate_projection(const icy2d_grid& g, cons
       float m32 = (float)mapped;
       if (m32 <= g.cutoff) m32 = 0.0f;
       else if (m32 >= 1.0f - g.cutoff) m32 = 1.0f;
-      v[0] += (double)m32;
-      if (adjustable && g.cutoff < m32 && m32 < 1.0f - g.cutoff) v[1] += (double)m32 * (1.0 - (double)m32);
+      v[r][0] = (double)m32;
+      if (adjustable && g.cutoff < m32 && m32 < 1.0f - g.cutoff) v[r][1] = (double)m32 * (1.0 - (double)m32);
     }
   }
-  block_partials<2>(v, g.partials, blk);
+  run_partials<2>(g, v, blk);
 }
 // simulator.py:4353-4406
 __device__ __forceinline__ void k2_apply_projection(const icy2d_grid& g, const int blk, double lambda) {
@@ -1927,7 +2053,10 @@ __device__ __forceinline__ void add_momentum(const icy2d_grid& g, int n, double 
   g.u[n] += mx / rho;
   g.u[N + n] += my / rho;
 #pragma unroll
-  for (int q = 0; q < 9; ++q) pop_add<kMomentum>(g.f, g, q * N + n, 3.0f * wq(q) * ((float)cxq(q) * mx + (float)cyq(q) * my));
+  for (int q = 0; q < 9; ++q) {
+    const float c_m = (float)cxq(q) * mx + (float)cyq(q) * my;
+    pop_set<kMomentum>(g.f, g, q * N + n, fmaf(3.0f * wq(q), c_m, pop_get<kMomentum>(g.f, g, q * N + n)));
+  }
 }
 // simulator.py:2842-2884
 __device__ __forceinline__ void k2_apply_melt_correction(const icy2d_grid& g, const int blk) {
@@ -2000,42 +2129,28 @@ __device__ __forceinline__ void k2_reset_thermal_diagnostics(const icy2d_grid& g
 // simulator.py:633-714 in control order: volume, energy, base and full
 // capacity (sums), specific energy min, max.
 __device__ __forceinline__ void k2_aperture_partials(const icy2d_grid& g, const int blk) {
-  double v[6] = {0.0, 0.0, 0.0, 0.0, 1.0e30, -1.0e30};
+  double v[kRun][6];
 #pragma unroll
   for (int r = 0; r < kRun; ++r) {
     const int first = (blk * kRun + r) * kBlock, n = first + (int)threadIdx.x;
+    v[r][0] = v[r][1] = v[r][2] = v[r][3] = 0.0;
+    v[r][4] = 1.0e30;
+    v[r][5] = -1.0e30;
     if (n >= cells(g)) continue;
     int i, j;
     row_col(g, first, n, i, j);
     const double vol = g.water_v[n];
     const double energy = g.water_e[n];
-    v[0] += vol;
-    v[1] += energy;
-    if (vol > 1.0e-30) {
-      v[4] = fmin(v[4], energy / vol);
-      v[5] = fmax(v[5], energy / vol);
-    }
+    v[r][0] = vol;
+    v[r][1] = energy;
+    if (vol > 1.0e-30) v[r][4] = v[r][5] = energy / vol;
     const float phase = clamp01(g.phi[n]);
     if (!wall_at(g, i, j) && g.solid[n] == 0 && phase > g.cutoff) {
-      v[2] += g.area * (double)phase;
-      v[3] += g.area;
+      v[r][2] = g.area * (double)phase;
+      v[r][3] = g.area;
     }
   }
-  __shared__ double part[6][kBlock / 64];
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-#pragma unroll
-  for (int k = 0; k < 6; ++k) {
-    const double x = k == 4 ? wave_min(v[k]) : k == 5 ? wave_max(v[k]) : wave_sum(v[k]);
-    if (lane == 0) part[k][wave] = x;
-  }
-  __syncthreads();
-  if (threadIdx.x < 6) {
-    const int k = threadIdx.x;
-    double r = part[k][0];
-    for (int w = 1; w < (int)(blockDim.x >> 6); ++w)
-      r = k == 4 ? fmin(r, part[k][w]) : k == 5 ? fmax(r, part[k][w]) : r + part[k][w];
-    g.partials[blk * 6 + k] = r;
-  }
+  run_partials<6, 0x10u, 0x20u>(g, v, blk);
 }
 // simulator.py:522-540: the thermal volume must stay within [0, capacity].
 __device__ __forceinline__ void k2_check_aperture(const icy2d_grid& g, const int blk) {
@@ -2075,7 +2190,7 @@ __device__ __forceinline__ double aperture_target(const icy2d_grid& g, int i, in
 // simulator.py:716-827 (control aperture = {volume, energy, base, full, min, max})
 __device__ __forceinline__ void k2_build_aperture_targets(const icy2d_grid& g, const int blk) {
   const icy2d_control* ctl = g.control;
-  double v[3] = {0.0, 0.0, 0.0}, bs, ss;
+  double v[kRun][3] = {}, bs, ss;
   aperture_scales(ctl, bs, ss);
   const double low = ctl->aperture[4], high = ctl->aperture[5], total = fmax(0.0, ctl->aperture[0]);
 #pragma unroll
@@ -2110,17 +2225,18 @@ __device__ __forceinline__ void k2_build_aperture_targets(const icy2d_grid& g, c
       }
       sp = fmin(high, fmax(low, sp));
       energy = target * sp;
-      v[1] += target * (sp - low);
-      v[2] += target * (high - sp);
+      v[run][1] = target * (sp - low);
+      v[run][2] = target * (high - sp);
     }
     g.target_e[n] = energy;
-    v[0] += energy;
+    v[run][0] = energy;
   }
-  block_partials<3>(v, g.partials, blk);
+  run_partials<3>(g, v, blk);
 }
 // simulator.py:829-859
-// with the new water in v (zeros past the grid) for the totals of its block.
-__device__ __forceinline__ void aperture_transfer_cell(const icy2d_grid& g, int first, int n, double bs, double ss, double v[2]) {
+// with the new water in v (left alone past the grid) for the totals of its block.
+__device__ __forceinline__ void aperture_transfer_cell(const icy2d_grid& g, int first, int n, double bs, double ss,
+                                                       double (&v)[2]) {
   if (n >= cells(g)) return;
   const icy2d_control* ctl = g.control;
   int i, j;
@@ -2135,8 +2251,8 @@ __device__ __forceinline__ void aperture_transfer_cell(const icy2d_grid& g, int 
   }
   g.water_v[n] = target;
   g.water_e[n] = energy;
-  v[0] += target;
-  v[1] += energy;
+  v[0] = target;
+  v[1] = energy;
 }
 __device__ __forceinline__ void k2_apply_aperture_transfer(const icy2d_grid& g, const int blk) {
   double v[2] = {0.0, 0.0}, bs, ss;
@@ -2144,16 +2260,16 @@ __device__ __forceinline__ void k2_apply_aperture_transfer(const icy2d_grid& g, 
   aperture_transfer_cell(g, blk * (int)blockDim.x, cell_index(blk), bs, ss, v);
 }
 // The transfer and the block sums of what it wrote (k2_water_totals_partials),
-// without reading the water planes again: 14 us at 1024x2048 instead of 12 + 11.
+// without reading the water planes again: 13 us at 1024x2048 instead of 12 + 11.
 __device__ __forceinline__ void k2_transfer_partials(const icy2d_grid& g, const int blk) {
-  double v[2] = {0.0, 0.0}, bs, ss;
+  double v[kRun][2] = {}, bs, ss;
   aperture_scales(g.control, bs, ss);
 #pragma unroll
   for (int r = 0; r < kRun; ++r) {
     const int first = (blk * kRun + r) * kBlock;
-    aperture_transfer_cell(g, first, first + (int)threadIdx.x, bs, ss, v);
+    aperture_transfer_cell(g, first, first + (int)threadIdx.x, bs, ss, v[r]);
   }
-  block_partials<2>(v, g.partials, blk);
+  run_partials<2>(g, v, blk);
 }
 __device__ __forceinline__ void k2_add_correction_abs(const icy2d_grid& g, const int blk) {
   icy2d_control* ctl = g.control;
@@ -2161,15 +2277,15 @@ __device__ __forceinline__ void k2_add_correction_abs(const icy2d_grid& g, const
 }
 // simulator.py:861-877
 __device__ __forceinline__ void k2_water_totals_partials(const icy2d_grid& g, const int blk) {
-  double v[2] = {0.0, 0.0};
+  double v[kRun][2] = {};
 #pragma unroll
   for (int r = 0; r < kRun; ++r) {
     const int n = (blk * kRun + r) * kBlock + (int)threadIdx.x;
     if (n >= cells(g)) continue;
-    v[0] += g.water_v[n];
-    v[1] += g.water_e[n];
+    v[r][0] = g.water_v[n];
+    v[r][1] = g.water_e[n];
   }
-  block_partials<2>(v, g.partials, blk);
+  run_partials<2>(g, v, blk);
 }
 // simulator.py:879-907
 __device__ __forceinline__ void k2_body_conduction(const icy2d_grid& g, const int blk, double dt) {
@@ -2546,8 +2662,14 @@ __device__ __forceinline__ T resolve(T a, int) {
 // Compiled for FP32 and the two stochastic FP16 forms; any other runs with
 // the branches.
 constexpr int kAnyStorage = -1, kHalfMomentum = 5, kHalfRelative = 15;
+// Waves a SIMD that a kernel's registers have to leave room for: the collision
+// needs 126 to 129 of them, and a fourth wave fits up to 128.
+template <auto F>
+constexpr int kWaves = 1;
+template <>
+constexpr int kWaves<k2_collide_push> = 4;
 template <int T, auto F, int Storage = kAnyStorage, class... A>
-__global__ void __launch_bounds__(T) one_case(icy2d_grid g, A... a) {
+__global__ void __launch_bounds__(T, kWaves<F>) one_case(icy2d_grid g, A... a) {
   if (Storage != kAnyStorage) g.half_populations = Storage;
   F(g, (int)blockIdx.x, a...);
 }
@@ -2583,7 +2705,7 @@ __device__ __forceinline__ icy2d_grid case_grid(const icy2d_batch& b, int c) {
   return g;
 }
 template <int T, auto F, int Storage = kAnyStorage, class... A>
-__global__ void __launch_bounds__(T) many_cases(icy2d_batch b, int shape, A... a) {
+__global__ void __launch_bounds__(T, kWaves<F>) many_cases(icy2d_batch b, int shape, A... a) {
   const int32_t* first = b.first_block + shape * (b.ncases + 1);
   const int c = owner(first, b.ncases, (int)blockIdx.x);
   if (b.active && !b.active[c]) return;
@@ -2751,7 +2873,7 @@ template <class D> int op_body_fraction(const D& d, int only_if_projected) {
 }
 template <class D> int op_commit_raster(const D& d) { return d.template launch<k2_commit_raster>(kCells); }
 template <class D> int op_contact_support(const D& d, int reduce, int only_if_projected) {
-  NEED(d, kRuns, 4);
+  NEED(d, kCells, 4);
   if (reduce) {
     TRY(d.template launch<k2_support_partials>(kRuns, only_if_projected));
     // min x, max x, min y, max y into the last four partials slots
@@ -2820,9 +2942,9 @@ template <class D> int op_dilate_band(const D& d, int radius) {
   return d.template launch<k2_copy_band>(kCells);
 }
 template <class D> int op_evaluate_projection(const D& d, typename D::Real lambda) {
-  NEED(d, kRuns, 2);
+  NEED(d, kCells, 2);
   TRY(d.template launch<k2_evaluate_projection>(kRuns, lambda));
-  return d.finish(kRuns, 2, CTL(water, 1), 0u, 0u, 0u);
+  return d.finish(kCells, 2, CTL(water, 1), 0u, 0u, 0u);
 }
 template <class D> int op_apply_projection(const D& d, typename D::Real lambda) {
   NEED(d, kCells, 1);
@@ -2871,29 +2993,29 @@ template <class D> int op_finish_melt_momentum(const D& d) {
   return d.template launch<k2_finish_melt_momentum>(kOne);
 }
 template <class D> int op_measure_aperture(const D& d) {
-  NEED(d, kRuns, 6);
+  NEED(d, kCells, 6);
   TRY(d.template launch<k2_aperture_partials>(kRuns));
-  return d.template finish_tail<k2_check_aperture>(kRuns, 6, CTL(aperture, 0), 0x10u, 0x20u, 0u);
+  return d.template finish_tail<k2_check_aperture>(kCells, 6, CTL(aperture, 0), 0x10u, 0x20u, 0u);
 }
 template <class D> int op_build_aperture_targets(const D& d) {
-  NEED(d, kRuns, 3);
+  NEED(d, kCells, 3);
   TRY(d.template launch<k2_build_aperture_targets>(kRuns));
   // the transfer's |energy correction| (simulator.py:829-859) is added as
   // soon as the targets are folded
-  return d.template finish_tail<k2_add_correction_abs>(kRuns, 3, CTL(targets, 0), 0u, 0u, 0u);
+  return d.template finish_tail<k2_add_correction_abs>(kCells, 3, CTL(targets, 0), 0u, 0u, 0u);
 }
 template <class D> int op_apply_aperture_transfer(const D& d) {
   return d.template launch<k2_apply_aperture_transfer>(kCells);
 }
 template <class D> int op_finish_aperture_transfer(const D& d) {
-  NEED(d, kRuns, 2);
+  NEED(d, kCells, 2);
   TRY(d.template launch<k2_water_totals_partials>(kRuns));
-  return d.finish(kRuns, 2, CTL(transfer, 0), 0u, 0u, 0u);
+  return d.finish(kCells, 2, CTL(transfer, 0), 0u, 0u, 0u);
 }
 template <class D> int op_transfer_aperture(const D& d) {
-  NEED(d, kRuns, 2);
+  NEED(d, kCells, 2);
   TRY(d.template launch<k2_transfer_partials>(kRuns));
-  return d.finish(kRuns, 2, CTL(transfer, 0), 0u, 0u, 0u);
+  return d.finish(kCells, 2, CTL(transfer, 0), 0u, 0u, 0u);
 }
 // measure, build, transfer: the whole of simulator.py:511-548.
 template <class D> int op_synchronize_aperture(const D& d) {
