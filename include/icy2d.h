@@ -42,7 +42,8 @@ typedef struct icy2d_control {
   float max_outflow;
   int32_t error_flags;        /* bit 0: negative water volume, bit 1: volume above the aperture capacity,
                                * bit 2: a heat or melt term outside the fixed-point range of the
-                               * thermal scatters (body_heat, inject_acc) */
+                               * thermal scatters (body_heat, inject_acc), bit 3: a batch stated a
+                               * population storage that is not this case's */
   double mass, inertia, local_com[2];
   double impulse[3];          /* hydrodynamic impulse x, y and torque */
   double melted[3];           /* cumulative melted body momentum */
@@ -240,7 +241,9 @@ typedef struct icy2d_batch {
   int32_t ncases;
   int32_t collide_threads;      /* 128, 256 or 512 (chosen by the autotuner) */
   int32_t stream_threads;       /* 128, 256 or 512 */
-  int32_t storage;              /* 1 + the half_populations that all cases share, 0: not stated (any mix) */
+  int32_t storage;              /* 1 + the half_populations that all cases share, 0: not stated (any mix); a case
+                                 * with another storage sets bit 3 of its error_flags, and its populations are
+                                 * left alone */
   const icy2d_grid* grids;      /* device array of ncases grids */
   const int32_t* active;        /* device, ncases flags, or NULL for all */
   const int32_t* first_block;   /* device, ICY2D_SHAPES * (ncases + 1) prefix sums */

@@ -2710,7 +2710,15 @@ __global__ void __launch_bounds__(T, kWaves<F>) many_cases(icy2d_batch b, int sh
   const int c = owner(first, b.ncases, (int)blockIdx.x);
   if (b.active && !b.active[c]) return;
   icy2d_grid g = case_grid(b, c);
-  if (Storage != kAnyStorage) g.half_populations = Storage;
+  if (Storage != kAnyStorage) {
+    // The batch's word is not taken for it: at the wrong width the accesses
+    // would leave the case's buffers.
+    if (g.half_populations != Storage) {
+      if (threadIdx.x == 0) atomicOr(&g.control->error_flags, 8);
+      return;
+    }
+    g.half_populations = Storage;
+  }
   F(g, (int)blockIdx.x - first[c], resolve(a, c)...);
 }
 // Destination of a finished reduction: a byte offset into the control block,

@@ -371,6 +371,8 @@ class IceFlow2D:
         flags = control.error_flags
         control.error_flags = 0
         self._write_control(control)
+        if flags & 8:
+            raise RuntimeError("a batch stated a population storage that is not this case's")
         if flags & 4:
             raise RuntimeError("a body heat or melt injection term left the fixed-point range of the thermal "
                                "scatters (over a quarter of a cell's latent heat in one step)")

@@ -69,6 +69,26 @@ def test_kernels_compiled_for_a_storage(storage, step):
         np.testing.assert_allclose(a, b, rtol=0.0, atol=3 * 9 * 32 * step)
 
 
+@pytest.mark.parametrize("storage,stated", [("fp16-momentum-sr", 0), ("fp32", 15), ("fp16-rel-sr", 5)])
+def test_stated_storage_that_is_not_the_cases(storage, stated):
+    """The kernels compiled for a storage leave a case of another alone and say
+    so: at the wrong width they would leave its buffers."""
+    from projecticy_amd.iceflow2d.ensemble import IceFlowEnsemble2D
+
+    batch = IceFlowEnsemble2D([submerged_config(), submerged_config()], population_storage=storage, use_graph=False)
+    batch._batch.storage = 1 + stated
+    names = ("f", "fbuf", "h", "hbuf", "phi", "u", "a")
+    before = [[case._t[name].clone() for name in names] for case in batch.cases]
+    for call in (("collide_stream",), ("stream", 0, 2), ("collide", 1), ("clip_phase", 2.0)):
+        batch._call(*call)
+        with pytest.raises(RuntimeError, match="ensemble case 0: .*storage"):
+            batch._read_controls()
+    batch._stream.synchronize()
+    for case, values in zip(batch.cases, before):
+        for name, value in zip(names, values):
+            assert torch.equal(case._t[name], value), name
+
+
 @pytest.mark.parametrize("shape", [(12, 520), (21, 512), (24, 43), (33, 31)])
 def test_reductions_over_runs_of_cells(shape):
     """The sums, minimum and maximum over blocks of four times 256 cells, on
