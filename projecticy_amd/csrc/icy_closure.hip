@@ -560,7 +560,9 @@ __global__ void __launch_bounds__(kSpreadThreads)
 //     registers).  Nine pairs over four waves: two each, and the ninth pair's
 //     16-cell chunks spread over the waves.
 //   - At the end the two halves add up through LDS, so 256 blocks write one
-//     partial each (28 MB at 128x64x64, half of one a column group).
+//     partial each (28 MB at 128x64x64, half of one a column group).  A block
+//     takes several (columns, slabs) items where a grid has more than
+//     kMaxGradBlocks of them, as wide ones do.
 // A block that staged each column's nine neighbours transposed, element by
 // element, took 109 us a layer at 128x64x64; 40 us now, and the fold of half as
 // many partials 7 us instead of 12.
@@ -584,8 +586,8 @@ static_assert(2 * kGradBuffer <= kGradShared && 8 * 3 * kC * kC * 4 <= kGradShar
 
 template <int T>
 __global__ void __launch_bounds__(kGradThreads, 2)
-    k_conv3d_wgrad(int nx, int ny, int per, const uint16_t* __restrict__ in, const uint16_t* __restrict__ dout,
-                   float* __restrict__ partials) {
+    k_conv3d_wgrad(int nx, int ny, int per, int items, const uint16_t* __restrict__ in,
+                   const uint16_t* __restrict__ dout, float* __restrict__ partials) {
   constexpr int nz = 16 * T;
   constexpr int kIn = (kGradCols + 2) * nz * 4, kOut = kGradCols * nz * 4;  // 16-byte pieces of a slab and of a row
   constexpr int kFetch = (kIn + kGradThreads - 1) / kGradThreads;
@@ -594,28 +596,28 @@ __global__ void __launch_bounds__(kGradThreads, 2)
   __shared__ float bias_part[kGradThreads / 64][kC];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, half = wave >> 2, part = wave & 3;
   const int tiles_j = (ny + kGradCols - 1) / kGradCols;
-  const int j0 = (int)(blockIdx.x % tiles_j) * kGradCols, x0 = (int)(blockIdx.x / tiles_j) * per;
-  const int x1 = min(nx, x0 + per);
-  for (int e = tid; e < 2 * kGradBuffer / 16; e += kGradThreads)
-    reinterpret_cast<u32x4*>(shared)[e] = u32x4{0u, 0u, 0u, 0u};
+  int j0, x0, x1;  // of the item in hand: its first column and its slabs
   // Staging: pieces as in the sweep (a thread without one reads the first
   // piece of the slab and stores none).
-  int src[kFetch], dst[kFetch];
+  int src[kFetch], dst[kFetch], out_src, out_dst;
+  auto begin = [&](int item) __attribute__((always_inline)) {
+    j0 = item % tiles_j * kGradCols;
+    x0 = item / tiles_j * per;
+    x1 = min(nx, x0 + per);
+    for (int e = tid; e < 2 * kGradBuffer / 16; e += kGradThreads)
+      reinterpret_cast<u32x4*>(shared)[e] = u32x4{0u, 0u, 0u, 0u};
 #pragma unroll
-  for (int f = 0; f < kFetch; ++f) {
-    const int e = tid + f * kGradThreads, col = e / (nz * 4), k = e / 4 % nz, c = e % 4, j = j0 - 1 + col;
-    const bool mine = e < kIn && j >= 0 && j < ny;
-    src[f] = mine ? (j * nz + k) * 4 + c : 0;
-    dst[f] = mine ? col * kGradColumn + (k + 1) * kGradRow + c * 16 : -1;
-  }
-  int out_src = 0, out_dst = -1;
-  {
-    const int col = tid / (nz * 4), k = tid / 4 % nz, c = tid % 4, j = j0 + col;
-    if (tid < kOut && j < ny) {
-      out_src = (j * nz + k) * 4 + c;
-      out_dst = (kGradCols + 2 + col) * kGradColumn + (k + 1) * kGradRow + c * 16;
+    for (int f = 0; f < kFetch; ++f) {
+      const int e = tid + f * kGradThreads, col = e / (nz * 4), k = e / 4 % nz, c = e % 4, j = j0 - 1 + col;
+      const bool mine = e < kIn && j >= 0 && j < ny;
+      src[f] = mine ? (j * nz + k) * 4 + c : 0;
+      dst[f] = mine ? col * kGradColumn + (k + 1) * kGradRow + c * 16 : -1;
     }
-  }
+    const int col = tid / (nz * 4), k = tid / 4 % nz, c = tid % 4, j = j0 + col;
+    const bool mine = tid < kOut && j < ny;
+    out_src = mine ? (j * nz + k) * 4 + c : 0;
+    out_dst = mine ? (kGradCols + 2 + col) * kGradColumn + (k + 1) * kGradRow + c * 16 : -1;
+  };
   u32x4 fetched[kFetch], fetched_out;
   // Slab s of the input and row s + 1 of the output gradient.
   auto fetch = [&](int s) __attribute__((always_inline)) {
@@ -654,9 +656,6 @@ __global__ void __launch_bounds__(kGradThreads, 2)
     for (int d = 0; d < 3; ++d)
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[q][d][r] = 0.0f;
-  __syncthreads();
-  fetch(x0 - 1);
-  stage(x0 - 1, shared);
   int current = 0;
   bf16x8 rows[3][T];
   // Input slab s with the gradient's rows s - 1 (A), s (B) and s + 1 (C, read here).
@@ -664,12 +663,12 @@ __global__ void __launch_bounds__(kGradThreads, 2)
     __syncthreads();
     const char* buffer = shared + current * kGradBuffer;
     if (s < x1) fetch(s + 1);
-    const bool has_a = s - 1 >= x0, has_b = s >= x0 && s < x1, has_c = s + 1 < x1;
+    const bool has_a = s - 1 >= x0 && s <= x1, has_b = s >= x0 && s < x1, has_c = s + 1 < x1;
     if (has_c) {
 #pragma unroll
       for (int c = 0; c < T; ++c) C[c] = column_operand(buffer + out_column + c * 16 * kGradRow, lane_offset);
     }
-    if (s >= 0 && s < nx) {
+    if (s >= 0 && s < nx && s <= x1) {
 #pragma unroll
       for (int c = 0; c < T; ++c)
 #pragma unroll
@@ -684,13 +683,18 @@ __global__ void __launch_bounds__(kGradThreads, 2)
     current ^= 1;
     if (s < x1) stage(s + 1, shared + current * kGradBuffer);
   };
-  for (int s = x0 - 1;;) {
-    step(s, rows[0], rows[1], rows[2]);
-    if (++s > x1) break;
-    step(s, rows[1], rows[2], rows[0]);
-    if (++s > x1) break;
-    step(s, rows[2], rows[0], rows[1]);
-    if (++s > x1) break;
+  for (int item = (int)blockIdx.x; item < items; item += (int)gridDim.x) {
+    if (item != (int)blockIdx.x) __syncthreads();  // the last item's slabs have been read
+    begin(item);
+    __syncthreads();
+    fetch(x0 - 1);
+    stage(x0 - 1, shared);
+    current = 0;
+    for (int s = x0 - 1; s <= x1; s += 3) {  // beyond x1 a step does nothing
+      step(s, rows[0], rows[1], rows[2]);
+      step(s + 1, rows[1], rows[2], rows[0]);
+      step(s + 2, rows[2], rows[0], rows[1]);
+    }
   }
   float* result = partials + (long)blockIdx.x * kLayer;
   float* red = reinterpret_cast<float*>(shared);
@@ -748,8 +752,8 @@ __global__ void __launch_bounds__(kGradThreads, 2)
 constexpr int kScalarGradCols = 4, kScalarGradRow = kTaps * kC + 8, kScalarGradSlab = (kScalarGradCols + 2) * kTapColumn;
 template <int T>
 __global__ void __launch_bounds__(kGradThreads)
-    k_scalar_wgrad(int nx, int ny, int per, const uint16_t* __restrict__ in, const uint16_t* __restrict__ g,
-                   float* __restrict__ partials) {
+    k_scalar_wgrad(int nx, int ny, int per, int items, const uint16_t* __restrict__ in,
+                   const uint16_t* __restrict__ g, float* __restrict__ partials) {
   constexpr int nz = 16 * T, kPieces = kScalarGradCols * nz * 4, kFetch = (kPieces + kGradThreads - 1) / kGradThreads;
   __shared__ __attribute__((aligned(16))) char xs[2][kScalarGradCols * kMaxColumn * kGradRow];
   __shared__ uint16_t gs[2][3 * kScalarGradSlab];
@@ -757,17 +761,21 @@ __global__ void __launch_bounds__(kGradThreads)
   __shared__ float bias_part[kGradThreads / 64];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, half = lane >> 5;
   const int tiles_j = (ny + kScalarGradCols - 1) / kScalarGradCols;
-  const int j0 = (int)(blockIdx.x % tiles_j) * kScalarGradCols, x0 = (int)(blockIdx.x / tiles_j) * per;
-  const int x1 = min(nx, x0 + per);
+  int j0, x0, x1;  // of the item in hand: its first column and its slabs
   u32x4 fetched[kFetch];
   bool mine[kFetch];
   int src[kFetch];
+  auto begin = [&](int item) __attribute__((always_inline)) {
+    j0 = item % tiles_j * kScalarGradCols;
+    x0 = item / tiles_j * per;
+    x1 = min(nx, x0 + per);
 #pragma unroll
-  for (int f = 0; f < kFetch; ++f) {
-    const int e = tid + f * kGradThreads, col = e / (nz * 4), j = j0 + col;
-    mine[f] = e < kPieces && j < ny;
-    src[f] = mine[f] ? j * nz * 4 + e % (nz * 4) : 0;
-  }
+    for (int f = 0; f < kFetch; ++f) {
+      const int e = tid + f * kGradThreads, col = e / (nz * 4), j = j0 + col;
+      mine[f] = e < kPieces && j < ny;
+      src[f] = mine[f] ? j * nz * 4 + e % (nz * 4) : 0;
+    }
+  };
   float bias_acc = 0.0f;
   constexpr int kGather = (3 * kScalarGradSlab + kGradThreads - 1) / kGradThreads;
   uint16_t gathered[kGather];
@@ -807,23 +815,27 @@ __global__ void __launch_bounds__(kGradThreads)
   floatx16 acc;
 #pragma unroll
   for (int r = 0; r < 16; ++r) acc[r] = 0.0f;
-  fetch(x0);
-  stage(0);
-  for (int s = x0; s < x1; ++s) {
-    const int buffer = (s - x0) & 1;
-    __syncthreads();
-    if (s + 1 < x1) fetch(s + 1);
-    for (int unit = wave; unit < kScalarGradCols * T; unit += kGradThreads / 64) {
-      const int col = unit / T, k0 = unit % T * 16;
-      typedef uint16_t u16x8 __attribute__((ext_vector_type(8)));
-      u16x8 v;
-      const uint16_t* cell_g = gs[buffer] + col * kTapColumn + k0 + tap_at;
+  for (int item = (int)blockIdx.x; item < items; item += (int)gridDim.x) {
+    if (item != (int)blockIdx.x) __syncthreads();  // the last item's slabs have been read
+    begin(item);
+    fetch(x0);
+    stage(0);
+    for (int s = x0; s < x1; ++s) {
+      const int buffer = (s - x0) & 1;
+      __syncthreads();
+      if (s + 1 < x1) fetch(s + 1);
+      for (int unit = wave; unit < kScalarGradCols * T; unit += kGradThreads / 64) {
+        const int col = unit / T, k0 = unit % T * 16;
+        typedef uint16_t u16x8 __attribute__((ext_vector_type(8)));
+        u16x8 v;
+        const uint16_t* cell_g = gs[buffer] + col * kTapColumn + k0 + tap_at;
 #pragma unroll
-      for (int e = 0; e < 8; ++e) v[e] = tap ? cell_g[e] : (uint16_t)0;
-      const bf16x8 x = column_operand(xs[buffer] + (col * kMaxColumn + k0) * kGradRow, lane_offset);
-      acc = mfma32(__builtin_bit_cast(bf16x8, v), x, acc);
+        for (int e = 0; e < 8; ++e) v[e] = tap ? cell_g[e] : (uint16_t)0;
+        const bf16x8 x = column_operand(xs[buffer] + (col * kMaxColumn + k0) * kGradRow, lane_offset);
+        acc = mfma32(__builtin_bit_cast(bf16x8, v), x, acc);
+      }
+      if (s + 1 < x1) stage(buffer ^ 1);
     }
-    if (s + 1 < x1) stage(buffer ^ 1);
   }
 #pragma unroll
   for (int r = 0; r < 16; ++r) red[wave][(8 * (r / 4) + 4 * half + r % 4) * kC + t] = acc[r];
@@ -1042,16 +1054,24 @@ void launch_taps(int nx, int ny, int nz, const uint16_t* in, const uint16_t* w, 
   auto kernel = nz == 16 ? k_conv3d_taps<1> : nz == 32 ? k_conv3d_taps<2> : nz == 48 ? k_conv3d_taps<3> : k_conv3d_taps<4>;
   kernel<<<blocks, kTapThreads, 0, s>>>(nx, ny, per, in, w, bias, out);
 }
-// Weight-gradient blocks: pairs of columns times chunks of slabs, one block
-// for each of the 256 CUs where the grid has as many, but four slabs a chunk
-// at least: a chunk reads two slabs more than it owns and writes 110 KB of
-// sums that the fold reads again.
+// Weight-gradient items: groups of `cols` columns times chunks of slabs, one
+// for each of the 256 CUs where the grid has as many, but four slabs a chunk at
+// least: a chunk reads two slabs more than it owns, and each block writes 110
+// KB of sums that the fold reads again.  With at least 1, 2, 4 and 8 slabs the
+// gradient and its fold take 27, 20, 20 and 22 us at 24x17x16, 28, 22, 24 and
+// 28 at 24x17x64, 28, 28, 27 and 30 at 40x33x48 and 12, 15, 14 and 15 at
+// 8x8x16 (the scalar layer's 18, 18, 13 and 11, 19, 19, 14 and 14, 20, 20, 14
+// and 21, 8, 7, 7 and 8); larger grids have four slabs or more by themselves.
+// At most kMaxGradBlocks blocks share the items: the 32768 of 1x65536x16, a
+// block each, would leave 3.6 GB of sums and take 1961 us; 251 this way.
+constexpr int kMaxGradBlocks = 512;
 struct GradPlan {
-  int per, blocks;
+  int per, items, blocks;
 };
-GradPlan wgrad_plan(int nx, int ny) {
-  const int tiles_j = (ny + kGradCols - 1) / kGradCols, slabs = sweep_slabs(nx, tiles_j), per = slabs < 4 ? 4 : slabs;
-  return {per, tiles_j * ((nx + per - 1) / per)};
+GradPlan wgrad_plan(int nx, int ny, int cols) {
+  const int tiles_j = (ny + cols - 1) / cols, slabs = sweep_slabs(nx, tiles_j), per = slabs < 4 ? 4 : slabs;
+  const int items = tiles_j * ((nx + per - 1) / per);
+  return {per, items, items < kMaxGradBlocks ? items : kMaxGradBlocks};
 }
 
 }  // namespace icyc
@@ -1133,7 +1153,7 @@ int icyc_conv3d_k8(int32_t nx, int32_t ny, int32_t nz, const uint16_t* in, const
 
 int64_t icyc_wgrad_partials_size(int32_t nx, int32_t ny, int32_t nz) {
   if (!valid_grid(nx, ny, nz)) return 0;
-  return (int64_t)wgrad_plan(nx, ny).blocks * kLayer;
+  return (int64_t)wgrad_plan(nx, ny, kGradCols).blocks * kLayer;
 }
 
 int icyc_conv3d_wgrad(int32_t nx, int32_t ny, int32_t nz, const uint16_t* in, const uint16_t* dout,
@@ -1141,12 +1161,12 @@ int icyc_conv3d_wgrad(int32_t nx, int32_t ny, int32_t nz, const uint16_t* in, co
   if (!valid_grid(nx, ny, nz) || nz % 16 != 0 || nz > kMaxColumn || !in || !dout || !partials || !grad)
     return ICYC_ERR_ARGUMENT;
   hipStream_t s = (hipStream_t)stream;
-  const GradPlan plan = wgrad_plan(nx, ny);
+  const GradPlan plan = wgrad_plan(nx, ny, kGradCols);
   auto kernel = nz == 16   ? k_conv3d_wgrad<1>
                 : nz == 32 ? k_conv3d_wgrad<2>
                 : nz == 48 ? k_conv3d_wgrad<3>
                            : k_conv3d_wgrad<4>;
-  kernel<<<plan.blocks, kGradThreads, 0, s>>>(nx, ny, plan.per, in, dout, partials);
+  kernel<<<plan.blocks, kGradThreads, 0, s>>>(nx, ny, plan.per, plan.items, in, dout, partials);
   if (int rc = status()) return rc;
   k_fold<<<blocks_of(kLayer, kFoldThreads), kFoldThreads, 0, s>>>(partials, plan.blocks, kLayer, grad);
   return status();
@@ -1170,15 +1190,14 @@ int icyc_conv3d_scalar_wgrad(int32_t nx, int32_t ny, int32_t nz, const uint16_t*
   if (!valid_grid(nx, ny, nz) || nz % 16 != 0 || nz > kMaxColumn || !in || !dout || !partials || !grad)
     return ICYC_ERR_ARGUMENT;
   hipStream_t s = (hipStream_t)stream;
-  const int tiles_j = (ny + kScalarGradCols - 1) / kScalarGradCols, slabs = sweep_slabs(nx, tiles_j);
-  const int per = slabs < 4 ? 4 : slabs, blocks = tiles_j * ((nx + per - 1) / per);
+  const GradPlan plan = wgrad_plan(nx, ny, kScalarGradCols);
   auto kernel = nz == 16   ? k_scalar_wgrad<1>
                 : nz == 32 ? k_scalar_wgrad<2>
                 : nz == 48 ? k_scalar_wgrad<3>
                            : k_scalar_wgrad<4>;
-  kernel<<<(unsigned)blocks, kGradThreads, 0, s>>>(nx, ny, per, in, dout, partials);
+  kernel<<<plan.blocks, kGradThreads, 0, s>>>(nx, ny, plan.per, plan.items, in, dout, partials);
   if (int rc = status()) return rc;
-  k_fold_scalar<<<blocks_of(kLayer, 64), 64, 0, s>>>(partials, blocks, grad);
+  k_fold_scalar<<<blocks_of(kLayer, 64), 64, 0, s>>>(partials, plan.blocks, grad);
   return status();
 }
 

@@ -303,6 +303,14 @@ def test_weight_gradient_edges(shape):
     test_weight_gradient(shape)
 
 
+# More (columns, slabs) items than weight-gradient blocks: a block takes two or
+# three of them; an odd number of columns in the last.
+@pytest.mark.parametrize("shape", [(2, 1101, 16), (5, 2399, 16)])
+def test_gradients_of_wide_grids(shape):
+    test_weight_gradient(shape)
+    test_scalar_layer_gradients(shape)
+
+
 @pytest.mark.parametrize("shape", SWEEP_SHAPES)
 def test_first_layer_edges(shape):
     test_conv_forward_with_eight_input_channels(shape)
