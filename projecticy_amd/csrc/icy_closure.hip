@@ -166,12 +166,13 @@ __global__ void __launch_bounds__(kSweepThreads, 2)
   for (int r = 0; r < 4; ++r) bias_r[r] = Epi == ICYC_RELU_BF16 ? bias[channels + 4 * group + r] : 0.0f;
   // Staging: piece e % 4 of cell e / 4 of the slab's columns; a thread
   // without a piece reads the slab's first and stores none.
-  int src[kFetch], dst[kFetch];
+  long src[kFetch];
+  int dst[kFetch];
 #pragma unroll
   for (int f = 0; f < kFetch; ++f) {
     const int e = threadIdx.x + f * kSweepThreads, col = e / (nz * 4), k = e / 4 % nz, c = e % 4, j = j0 - 1 + col;
     const bool mine = e < kPieces && j >= 0 && j < ny;
-    src[f] = mine ? (j * nz + k) * 4 + c : 0;
+    src[f] = mine ? (long)(j * nz + k) * 4 + c : 0;
     dst[f] = mine ? col * kSweepColumn + (k + 1) * 4 + (c ^ (((k + 1) >> 2) & 3)) : -1;
   }
   u32x4 fetched[kFetch];
@@ -309,12 +310,13 @@ __global__ void __launch_bounds__(kSweepThreads)
     di[m] = t / 9;
     at[m] = t / 3 % 3 * kColumn + t % 3;
   }
-  int src[kFetch], dst[kFetch];
+  long src[kFetch];
+  int dst[kFetch];
 #pragma unroll
   for (int f = 0; f < kFetch; ++f) {
     const int e = threadIdx.x + f * kSweepThreads, col = e / nz, k = e % nz, j = j0 - 1 + col;
     const bool mine = e < kCells && j >= 0 && j < ny;
-    src[f] = mine ? (j * nz + k) * 4 : 0;
+    src[f] = mine ? (long)(j * nz + k) * 4 : 0;
     dst[f] = mine ? col * kColumn + k + 1 : -1;
   }
   u32x4 fetched[kFetch];
@@ -405,12 +407,13 @@ __global__ void __launch_bounds__(kTapThreads)
       wr[h] = *reinterpret_cast<const bf16x8*>(w + (long)(lane & 31) * kC * kC + 16 * h + 8 * half);
   }
   // This lane's cell of the wave's tiles (none: -1) and its place in a row of y.
-  int src[kPerWave], dst[kPerWave];
+  long src[kPerWave];
+  int dst[kPerWave];
 #pragma unroll
   for (int p = 0; p < kPerWave; ++p) {
     const int f = (wave + p * (kTapThreads / 64)) * 32 + (lane & 31), col = f / nz, k = f % nz, j = j0 - 1 + col;
     const bool mine = f < (kScalarCols + 2) * nz && j >= 0 && j < ny;
-    src[p] = mine ? (j * nz + k) * 4 + half : -1;
+    src[p] = mine ? (long)(j * nz + k) * 4 + half : -1;
     dst[p] = col * kTapColumn + k + 1;
   }
   u32x4 fetched[kPerWave][2];
@@ -419,7 +422,7 @@ __global__ void __launch_bounds__(kTapThreads)
 #pragma unroll
     for (int p = 0; p < kPerWave; ++p)
 #pragma unroll
-      for (int h = 0; h < 2; ++h) fetched[p][h] = slab[max(src[p], 0) + 2 * h];
+      for (int h = 0; h < 2; ++h) fetched[p][h] = slab[max(src[p], 0L) + 2 * h];
   };
   const int own_j = threadIdx.x / nz, own_k = threadIdx.x % nz;
   const bool owned = (int)threadIdx.x < kScalarCols * nz && j0 + own_j < ny;
@@ -599,7 +602,8 @@ __global__ void __launch_bounds__(kGradThreads, 2)
   int j0, x0, x1;  // of the item in hand: its first column and its slabs
   // Staging: pieces as in the sweep (a thread without one reads the first
   // piece of the slab and stores none).
-  int src[kFetch], dst[kFetch], out_src, out_dst;
+  long src[kFetch], out_src;
+  int dst[kFetch], out_dst;
   auto begin = [&](int item) __attribute__((always_inline)) {
     j0 = item % tiles_j * kGradCols;
     x0 = item / tiles_j * per;
@@ -610,12 +614,12 @@ __global__ void __launch_bounds__(kGradThreads, 2)
     for (int f = 0; f < kFetch; ++f) {
       const int e = tid + f * kGradThreads, col = e / (nz * 4), k = e / 4 % nz, c = e % 4, j = j0 - 1 + col;
       const bool mine = e < kIn && j >= 0 && j < ny;
-      src[f] = mine ? (j * nz + k) * 4 + c : 0;
+      src[f] = mine ? (long)(j * nz + k) * 4 + c : 0;
       dst[f] = mine ? col * kGradColumn + (k + 1) * kGradRow + c * 16 : -1;
     }
     const int col = tid / (nz * 4), k = tid / 4 % nz, c = tid % 4, j = j0 + col;
     const bool mine = tid < kOut && j < ny;
-    out_src = mine ? (j * nz + k) * 4 + c : 0;
+    out_src = mine ? (long)(j * nz + k) * 4 + c : 0;
     out_dst = mine ? (kGradCols + 2 + col) * kGradColumn + (k + 1) * kGradRow + c * 16 : -1;
   };
   u32x4 fetched[kFetch], fetched_out;
@@ -764,7 +768,7 @@ __global__ void __launch_bounds__(kGradThreads)
   int j0, x0, x1;  // of the item in hand: its first column and its slabs
   u32x4 fetched[kFetch];
   bool mine[kFetch];
-  int src[kFetch];
+  long src[kFetch];
   auto begin = [&](int item) __attribute__((always_inline)) {
     j0 = item % tiles_j * kScalarGradCols;
     x0 = item / tiles_j * per;
@@ -773,7 +777,7 @@ __global__ void __launch_bounds__(kGradThreads)
     for (int f = 0; f < kFetch; ++f) {
       const int e = tid + f * kGradThreads, col = e / (nz * 4), j = j0 + col;
       mine[f] = e < kPieces && j < ny;
-      src[f] = mine[f] ? j * nz * 4 + e % (nz * 4) : 0;
+      src[f] = mine[f] ? (long)j * nz * 4 + e % (nz * 4) : 0;
     }
   };
   float bias_acc = 0.0f;

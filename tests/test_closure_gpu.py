@@ -358,3 +358,55 @@ def test_scalar_layer_gradients(shape):
     weights = co.TAPS * co.C * co.C
     assert np.abs(got[:weights] - dw.ravel()).max() <= 2e-6 * np.abs(dw).max() * max(1.0, cells / 64)
     assert np.abs(got[weights:] - db).max() <= 1e-5 * max(np.abs(db).max(), 1.0)
+
+
+def test_slabs_of_more_than_2_to_the_29_cells():
+    """A slab whose 16-byte pieces pass 2^31: the last eight columns alone are
+    nonzero, so every layer's outputs there, and the gradients, are those of a
+    grid of twelve columns (the forward passes and the data gradient sum a cell
+    in the same order: bit for bit)."""
+    from projecticy_amd import _native_closure as nc
+
+    if torch.cuda.mem_get_info()[0] < 200 << 30:
+        pytest.skip("needs 200 GB of GPU memory")
+    lib, s = nc.lib(), stream()
+    nz, small, live = 64, 12, 8
+    ny = (1 << 23) + 37
+    rng = np.random.default_rng(29)
+    values = [co.bf16_round(rng.normal(size=(live * nz, co.C))) for _ in range(2)]
+    plane = co.bf16_round(rng.normal(size=(live * nz,)))
+    w = co.bf16_round(rng.normal(scale=0.1, size=(co.TAPS, co.C, co.C)))
+    wt, bias = bits_tensor(w), torch.zeros(co.C, device="cuda")
+    results = []
+    for width in (small, ny):
+        cells = width * nz
+        first = cells - live * nz
+        x, dout = (torch.zeros(cells * co.C, dtype=torch.int16, device="cuda") for _ in range(2))
+        g = torch.zeros(cells, dtype=torch.int16, device="cuda")
+        for t, v in ((x, values[0]), (dout, values[1]), (g, plane)):
+            t[t.numel() - v.size:] = bits_tensor(v).view(-1)
+        out = torch.zeros(cells * co.C, dtype=torch.int16, device="cuda")
+        pred = torch.zeros(cells, device="cuda")
+        partials = torch.zeros(int(lib.icyc_wgrad_partials_size(1, width, nz)), device="cuda")
+        grad = torch.zeros(co.LAYER_PARAMS, device="cuda")
+        tail = slice((cells - small * nz) * co.C, None)
+        got = []
+        nc.check(lib.icyc_conv3d(1, width, nz, ptr(x), ptr(wt), ptr(bias), nc.RELU_BF16, None, ptr(out), None, s), "fwd")
+        got.append(out[tail].clone())
+        nc.check(lib.icyc_conv3d_k8(1, width, nz, ptr(x), ptr(wt), ptr(bias), nc.RELU_BF16, ptr(out), None, s), "first")
+        got.append(out[tail].clone())
+        nc.check(lib.icyc_conv3d(1, width, nz, ptr(x), ptr(wt), ptr(bias), nc.LINEAR_F32, None, None, ptr(pred), s),
+                 "last")
+        got.append(pred[-small * nz:].clone())
+        nc.check(lib.icyc_conv3d_scalar_data(1, width, nz, ptr(g), ptr(wt), ptr(x), ptr(out), s), "scalar data")
+        got.append(out[tail].clone())
+        nc.check(lib.icyc_conv3d_wgrad(1, width, nz, ptr(x), ptr(dout), ptr(partials), ptr(grad), s), "wgrad")
+        got.append(grad.clone())
+        nc.check(lib.icyc_conv3d_scalar_wgrad(1, width, nz, ptr(x), ptr(g), ptr(partials), ptr(grad), s), "scalar wgrad")
+        got.append(grad.clone())
+        results.append(got)
+        del x, dout, g, out, pred, partials
+    for a, b in zip(*[r[:4] for r in results]):
+        assert torch.equal(a, b)
+    for a, b in zip(*[r[4:] for r in results]):  # 512 cells' products in another grouping
+        assert (a - b).abs().max().item() <= live * nz * 2.0 ** -23 * a.abs().max().item()
