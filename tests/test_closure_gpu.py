@@ -288,9 +288,12 @@ def test_weight_gradient_at_closure_grid():
 
 
 # Column depths and widths where the x sweep's tiles and chunks end unevenly:
-# every depth, y extents that are no multiple of its 4 columns, one slab, and
-# more slabs than one a block (with a shorter last chunk).
-SWEEP_SHAPES = [(1, 1, 16), (1, 5, 48), (4, 7, 48), (3, 9, 64), (70, 17, 16), (37, 30, 32)]
+# every depth, y extents that are no multiple of its columns, one slab, and two
+# slabs a block.  Then several slabs a block of every kernel (four of the
+# 8-column ones, five of the 4-column ones, which reuses their rings' slots and
+# hands partial sums from slab to slab) with a shorter last chunk, at every depth.
+SWEEP_SHAPES = [(1, 1, 16), (1, 5, 48), (4, 7, 48), (3, 9, 64), (70, 17, 16), (37, 30, 32),
+                (391, 9, 16), (391, 9, 32), (387, 9, 48), (387, 9, 64)]
 
 
 @pytest.mark.parametrize("shape", SWEEP_SHAPES)
