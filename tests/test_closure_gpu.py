@@ -189,6 +189,10 @@ def test_adam_matches_oracle_and_packs_weights():
 
 
 def test_training_reduces_a_smooth_regression_loss():
+    """At this rate the loss falls to 0.4% of its start (at most 1.5% over 20
+    runs from parameters changed by 1e-6 of themselves), so the bound of 20%
+    is no matter of rounding; at three times the rate it was: 12% in the
+    middle, 96% at most."""
     from projecticy_amd.closure import ClosureNet
 
     shape = (8, 8, 16)
@@ -205,7 +209,7 @@ def test_training_reduces_a_smooth_regression_loss():
     start = np.mean([net.evaluate(*s) for s in samples])
     for _ in range(60):
         for s in samples:
-            net.train_step(*s, lr=3e-3)
+            net.train_step(*s, lr=1e-3)
     end = np.mean([net.evaluate(*s) for s in samples])
     assert end < 0.2 * start, (start, end)
 
