@@ -242,8 +242,8 @@ typedef struct icy2d_batch {
   int32_t collide_threads;      /* 128, 256 or 512 (chosen by the autotuner) */
   int32_t stream_threads;       /* 128, 256 or 512 */
   int32_t storage;              /* 1 + the half_populations that all cases share, 0: not stated (any mix); a case
-                                 * with another storage sets bit 3 of its error_flags, and its populations are
-                                 * left alone */
+                                 * with another storage is left alone by the kernels that move populations,
+                                 * and the next reduction sets bit 3 of its error_flags */
   const icy2d_grid* grids;      /* device array of ncases grids */
   const int32_t* active;        /* device, ncases flags, or NULL for all */
   const int32_t* first_block;   /* device, ICY2D_SHAPES * (ncases + 1) prefix sums */

@@ -2663,7 +2663,8 @@ __device__ __forceinline__ T resolve(T a, int) {
 // the branches.
 constexpr int kAnyStorage = -1, kHalfMomentum = 5, kHalfRelative = 15;
 // Waves a SIMD that a kernel's registers have to leave room for: the collision
-// needs 126 to 129 of them, and a fourth wave fits up to 128.
+// takes 126 to 129 by itself, and four waves fit up to 128 (over the 64-case
+// ensemble with FP16 deviations 862 us at three waves, 748 at four).
 template <auto F>
 constexpr int kWaves = 1;
 template <>
@@ -2712,14 +2713,17 @@ __global__ void __launch_bounds__(T, kWaves<F>) many_cases(icy2d_batch b, int sh
   icy2d_grid g = case_grid(b, c);
   if (Storage != kAnyStorage) {
     // The batch's word is not taken for it: at the wrong width the accesses
-    // would leave the case's buffers.
-    if (g.half_populations != Storage) {
-      if (threadIdx.x == 0) atomicOr(&g.control->error_flags, 8);
-      return;
-    }
+    // would leave the case's buffers.  check_storage reports it, as a store
+    // here would keep the grid's fields from being loaded as scalars (143
+    // registers for 128, and 848 us for 702 over the 64-case ensemble).
+    if (g.half_populations != Storage) return;
     g.half_populations = Storage;
   }
   F(g, (int)blockIdx.x - first[c], resolve(a, c)...);
+}
+// Of a batch that states a storage, the cases that have another.
+__device__ __forceinline__ void check_storage(const icy2d_batch& b, const icy2d_grid& g) {
+  if (b.storage != 0 && b.storage != 1 + g.half_populations && threadIdx.x == 0) atomicOr(&g.control->error_flags, 8);
 }
 // Destination of a finished reduction: a byte offset into the control block,
 // or the last `tail` slots of the case's partials.
@@ -2739,6 +2743,7 @@ __global__ void __launch_bounds__(kFinishThreads) k2_finish_many(icy2d_batch b, 
   const int c = (int)blockIdx.x / K, k = (int)blockIdx.x - c * K;
   if (b.active && !b.active[c]) return;
   const icy2d_grid g = case_grid(b, c);
+  check_storage(b, g);
   const int32_t* first = b.first_block + shape * (b.ncases + 1);
   finish_fold(g.partials, first[c + 1] - first[c], K, k, dest_ptr(g, d), min_mask, max_mask, add_mask);
 }
@@ -2775,6 +2780,7 @@ __global__ void __launch_bounds__(kFinishThreads) k2_finish_many_tail(icy2d_batc
   const int c = (int)blockIdx.x / K, k = (int)blockIdx.x - c * K;
   if (b.active && !b.active[c]) return;
   const icy2d_grid g = case_grid(b, c);
+  check_storage(b, g);
   const int32_t* first = b.first_block + shape * (b.ncases + 1);
   finish_fold(g.partials, first[c + 1] - first[c], K, k, dest_ptr(g, d), min_mask, max_mask, add_mask);
   if (last_finisher(g.control, K) && threadIdx.x == 0) Tail(g, 0, resolve(a, c)...);

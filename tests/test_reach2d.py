@@ -81,6 +81,8 @@ def test_stated_storage_that_is_not_the_cases(storage, stated):
     before = [[case._t[name].clone() for name in names] for case in batch.cases]
     for call in (("collide_stream",), ("stream", 0, 2), ("collide", 1), ("clip_phase", 2.0)):
         batch._call(*call)
+        if call[0] == "stream":  # no reduction in it
+            continue
         with pytest.raises(RuntimeError, match="ensemble case 0: .*storage"):
             batch._read_controls()
     batch._stream.synchronize()
