@@ -505,7 +505,8 @@ __device__ __forceinline__ void plane_set(float* base, unsigned offset, float v)
 // wave, and it stages two rows and two slabs more than it owns, so the
 // cheapest cut is searched over the row tiles that fit and the slab chunks
 // that fill whole rounds of the 256 CUs (kSlabLatency, kWaveTime: microseconds
-// measured at 24x20x16 and 256x128x128).
+// measured at 24x20x16 and 256x128x128).  A block has tens of rows, however
+// many the grid has, so a launch searches tens of cuts.
 inline StreamTiles stream_tiles(const icy3d_grid& g, int threads) {
   constexpr int kCus = 256;
   constexpr double kSlabLatency = 1.6, kWaveTime = 0.24;
@@ -517,16 +518,17 @@ inline StreamTiles stream_tiles(const icy3d_grid& g, int threads) {
   tiles_k = (g.nz + K - 1) / K;
   const int most = cells_most / L - 2;
   double least = 0.0;
-  for (int tiles_j = (g.ny + most - 1) / most; tiles_j <= g.ny; ++tiles_j) {
-    const int J = (g.ny + tiles_j - 1) / tiles_j, waves = ((J + 2) * L + kWaveCells - 1) / kWaveCells;
-    const int yz = tiles_k * ((g.ny + J - 1) / J);
+  for (int J = most < g.ny ? most : g.ny; J >= 1; --J) {
+    const int tiles_j = (g.ny + J - 1) / J;
+    if ((g.ny + tiles_j - 1) / tiles_j != J) continue;  // as many tiles of fewer rows do
+    const int waves = ((J + 2) * L + kWaveCells - 1) / kWaveCells, yz = tiles_k * tiles_j;
     for (int rounds = 1; rounds <= 4; ++rounds) {
       const int chunks = yz >= kCus * rounds ? 1 : kCus * rounds / yz;
       const int X = (g.nx + chunks - 1) / chunks, blocks = yz * ((g.nx + X - 1) / X);
       const double cost = (double)((blocks + kCus - 1) / kCus) * (X + 2) * (kSlabLatency + kWaveTime * waves);
       if (best.J == 0 || cost < least) {
         least = cost;
-        best = {J, K, X, (g.ny + J - 1) / J, tiles_k};
+        best = {J, K, X, tiles_j, tiles_k};
       }
     }
   }
