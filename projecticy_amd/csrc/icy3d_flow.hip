@@ -1433,21 +1433,6 @@ __global__ void k_collide_momentum(icy3d_grid g, int zero_loads) {
 struct MomentSums {
   float p, jx, jy, jz, xx, yy, zz, xy, xz, yz;
 };
-template <int Q>
-__device__ __forceinline__ void accumulate(MomentSums& s, float v) {
-  constexpr int X = cx(Q), Y = cy(Q), Z = cz(Q);
-  s.p += v;
-  if (X) s.jx += (float)X * v;
-  if (Y) s.jy += (float)Y * v;
-  if (Z) s.jz += (float)Z * v;
-  if (X) s.xx += v;
-  if (Y) s.yy += v;
-  if (Z) s.zz += v;
-  if (X && Y) s.xy += (float)(X * Y) * v;
-  if (X && Z) s.xz += (float)(X * Z) * v;
-  if (Y && Z) s.yz += (float)(Y * Z) * v;
-}
-
 __device__ __forceinline__ void store_streamed(const icy3d_grid& g, float* __restrict__ dst, int n, const MomentSums& s) {
   const size_t N = cells(g);
   const float third = s.p * (1.0f / 3.0f);
@@ -1826,7 +1811,7 @@ __device__ float reflect_link(const icy3d_grid& g, const Cell& c, int outgoing, 
 // partials; a slot that took a non-finite or out-of-range load writes NaN.  Fused: the
 // post-collision moments of each pulled cell are computed from g.home here
 // (collide_at) and the result goes to g.home_post, as in
-// k_collide_stream_tiled; otherwise they are read from home_post and the
+// k_stream_rows<true>; otherwise they are read from home_post and the
 // result goes to g.home.
 constexpr double kLoadScale = 0x1p40;
 template <bool Fused>
