@@ -309,6 +309,9 @@ def closure_dam_break(args):
     out = dam_break_score(net, seed=args.seed, steps=args.closure_score_steps)
     out["seconds"] = round(time.perf_counter() - t0, 1)
     out["weights"] = str(CLOSURE_WEIGHTS.relative_to(ROOT))
+    # The melted masses and centre trajectories of dam_break_score are for
+    # plots; in the one line of results they were most of 9 KB.
+    del out["melted_kg"], out["centres_m"]
     print(f"[bench] closure dam break {out['coarse_steps']} coarse steps in {out['seconds']} s: final melt error "
           f"plain {out['plain']['final_melt_error']:.3f}, closure {out['closure']['final_melt_error']:.3f}; "
           f"max centroid error plain {out['plain']['max_centroid_error_m']:.2e} m, closure "
@@ -446,11 +449,14 @@ def fine_solver_gate(configs, draws, steps):
     worst = {k: max(e for e in v if e is not None) for k, v in errors.items()}
     print(f"[bench] fine-solver gate: {len(picked)} widths x {steps} steps, melted-mass error vs fine "
           + ", ".join(f"{k} max {v:.3e}" for k, v in worst.items()), file=sys.stderr, flush=True)
+    short = lambda values: [None if v is None else float(f"{v:.4g}") for v in values]  # noqa: E731
     return {
         "steps": steps, "fine_steps": 2 * steps, "widths": [c.nx for c, _ in picked],
-        "melted_kg_m_fine": fine_melt, "melted_kg_m_coarse": melted,
-        "melted_mass_relative_error": errors, "error_fraction_of_initial_ice": ice_errors,
-        "max_relative_error": worst, "within_1pct_by_width": passed, "within_1pct_of_ice_by_width": passed_ice,
+        "melted_kg_m_fine": short(fine_melt),
+        "melted_mass_relative_error": {k: short(v) for k, v in errors.items()},
+        "error_fraction_of_initial_ice": {k: short(v) for k, v in ice_errors.items()},
+        "max_relative_error": {k: float(f"{v:.4g}") for k, v in worst.items()},
+        "within_1pct_by_width": passed, "within_1pct_of_ice_by_width": passed_ice,
         "reference": "the same case on a twice finer grid, FP32 populations, over the same physical time",
     }
 
