@@ -260,14 +260,25 @@ __device__ __forceinline__ void basis(float u, float b[3]) {
     b[2] = 0.5f;
   }
 }
-template <int Q>
+// s + a b with the product fused or rounded.
+template <bool Fused>
+__device__ __forceinline__ float add_product(float s, float a, float b) {
+#pragma clang fp contract(off)
+  return Fused ? fmaf(a, b, s) : s + a * b;
+}
+// Bit m of Rounded: moment m's product is rounded before it is added.
+template <int Q, unsigned Rounded>
 __device__ __forceinline__ float reconstruct_cm(float ux, float uy, const float m[9]) {
   float bx[3], by[3];
   basis<cxq(Q)>(ux, bx);
   basis<cyq(Q)>(uy, by);
-  return bx[0] * by[0] * m[0] + bx[1] * by[0] * m[1] + bx[0] * by[1] * m[2] + bx[2] * by[0] * m[3] +
-         bx[0] * by[2] * m[4] + bx[1] * by[1] * m[5] + bx[2] * by[1] * m[6] + bx[1] * by[2] * m[7] +
-         bx[2] * by[2] * m[8];
+  float s = bx[0] * by[0] * m[0] + bx[1] * by[0] * m[1] + bx[0] * by[1] * m[2];
+  s = add_product<!(Rounded >> 3 & 1u)>(s, bx[2] * by[0], m[3]);
+  s = add_product<!(Rounded >> 4 & 1u)>(s, bx[0] * by[2], m[4]);
+  s += bx[1] * by[1] * m[5];
+  s = add_product<!(Rounded >> 6 & 1u)>(s, bx[2] * by[1], m[6]);
+  s = add_product<!(Rounded >> 7 & 1u)>(s, bx[1] * by[2], m[7]);
+  return s + bx[2] * by[2] * m[8];
 }
 // sums[m] += c_q's raw moment m times v, without the moments that vanish.
 template <int M>
@@ -1103,7 +1114,7 @@ __device__ __forceinline__ void collide_cell(const icy2d_grid& g, const OwnCell&
 #pragma unroll
     for (int q = 0; q < 9; ++q) {
       add_raw(raw, q, pop_value<kMomentum>(g, own.f[q]));
-      poly[q] = momentum_poly<true>(q, ux * ux + uy * uy, ux, uy);
+      poly[q] = momentum_poly<true>(q, fmaf(uy, uy, ux * ux), ux, uy);
       add_raw(eq, q, momentum_eq_of(q, pdyn, rho, poly[q]));
       if (q > 0) add_raw(src, q, wq(q) * 3.0f * (along(q, Fx, Fy) + drho * along(q, ux, uy) * along(q, gsx, gsy)));
     }
@@ -1142,7 +1153,7 @@ __device__ __forceinline__ void collide_cell(const icy2d_grid& g, const OwnCell&
   const float compression = 4.0f * phi * (1.0f - phi) / g.width;
   const float nx_ = st.g[0] / norm, ny_ = st.g[1] / norm;
   // Central moments, m = {00, 10, 01, 20, 02, 11, 21, 12, 22}.
-  const float uu = ux * ux + uy * uy;
+  const float uu = Push ? fmaf(uy, uy, ux * ux) : fmaf(ux, ux, uy * uy);  // as momentum_poly: written out
   float r10 = 0.0f, r01 = 0.0f, eq[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0}, src[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
 #pragma unroll
   for (int q = 0; q < 9; ++q) {
@@ -1165,15 +1176,17 @@ __device__ __forceinline__ void collide_cell(const icy2d_grid& g, const OwnCell&
   for (int m = 0; m < 9; ++m) post[m] = eq[m] + 0.5f * src[m];
   post[1] = r10 - rate * (r10 - eq[1]) + (1.0f - 0.5f * rate) * src[1];
   post[2] = r01 - rate * (r01 - eq[2]) + (1.0f - 0.5f * rate) * src[2];
-  ph[0] = reconstruct_cm<0>(ux, uy, post);
-  ph[1] = reconstruct_cm<1>(ux, uy, post);
-  ph[2] = reconstruct_cm<2>(ux, uy, post);
-  ph[3] = reconstruct_cm<3>(ux, uy, post);
-  ph[4] = reconstruct_cm<4>(ux, uy, post);
-  ph[5] = reconstruct_cm<5>(ux, uy, post);
-  ph[6] = reconstruct_cm<6>(ux, uy, post);
-  ph[7] = reconstruct_cm<7>(ux, uy, post);
-  ph[8] = reconstruct_cm<8>(ux, uy, post);
+  // Opposite directions of an axis share two products: fused where they are
+  // used first, rounded where they are used again. Written out like momentum_poly's.
+  ph[0] = reconstruct_cm<0, 0u>(ux, uy, post);
+  ph[1] = reconstruct_cm<1, 0u>(ux, uy, post);
+  ph[2] = reconstruct_cm<2, 0u>(ux, uy, post);
+  ph[3] = reconstruct_cm<3, 0x48u>(ux, uy, post);
+  ph[4] = reconstruct_cm<4, 0x90u>(ux, uy, post);
+  ph[5] = reconstruct_cm<5, 0u>(ux, uy, post);
+  ph[6] = reconstruct_cm<6, 0x48u>(ux, uy, post);
+  ph[7] = reconstruct_cm<7, 0x90u>(ux, uy, post);
+  ph[8] = reconstruct_cm<8, 0xd8u>(ux, uy, post);
 }
 // Whether one of the cell's eight neighbours is ice (the window's kinds).
 template <class W>
