@@ -2816,7 +2816,9 @@ struct One {
     one_case<kBlock, F><<<shape_blocks(g, shape), shape_threads(shape), 0, s>>>(g, a...);
     return launch_status();
   }
-  // A kernel that moves populations, compiled for the grid's storage.
+  // A kernel that moves populations, compiled for the grid's storage: for the
+  // three that the single run, the ensembles and the smallest footprint take by
+  // default (each costs its own code); the others run the general kernel.
   template <auto F, class... A>
   int launch_stored(int shape, A... a) const {
     const unsigned blocks = shape_blocks(g, shape);

@@ -958,9 +958,10 @@ __device__ void acceleration_at(const icy3d_grid& g, const Cell& c, const float 
 // cell of the fluid box, and staged as the tank formulas use it: the gradient
 // with the mirrored components negated (capillary), no pressure term, the
 // velocity -u of the mirror cell (halfway no-slip), and no donor flux.
-// Bound by memory: 77 bytes a cell and the tile's halo.  Tiles of 4 x 64
-// cells with every quantity's 3 x 3 window read from LDS took 168 us at
-// 256x128x128, 406 at 450x150x90 and 90 at 24x20x16; 110, 182 and 6 now (with
+// Bound by memory: 77 bytes a cell are needed, and 117 move at 256x128x128 (the
+// halo's rows come again) at 89% of the copy rate, the vector ALUs 53% busy.
+// Tiles of 4 x 64 cells with every quantity's 3 x 3 window read from LDS took
+// 168 us there, 406 at 450x150x90 and 90 at 24x20x16; 122, 182 and 6 now (with
 // twelve waves a block: sixteen spill 33 registers, 209 us at 256x128x128).
 struct ForceFetch {
   float grad[3], phi, p, u[3], flux[3], volume, energy;
@@ -1467,7 +1468,9 @@ __device__ __forceinline__ void store_streamed(const icy3d_grid& g, float* __res
 // 1/6; the 1/216 comes last); then the same along y and along x.  A non-fluid
 // cell sends zeros, and its links come back by the bounce below.  About 140
 // operations and 36 LDS words a cell; summing the 27 pulled populations took
-// 450 and 122.
+// 450 and 122.  Fused, the pass is bound by memory: of 118 bytes a cell that it
+// needs 188 move at 256x128x128 (the halo's rows come again), at 95% of the copy
+// rate and with the vector ALUs 39% busy: 184 us, 260 with the 27 sums.
 //
 // A block owns J rows by K cells of a (y, z) tile and sweeps X slabs of x.
 // The tile with its halo, (J + 2) rows of K + 2 cells, is laid flat over the

@@ -256,9 +256,9 @@ __global__ void k_advect_water(icy3d_grid g, float dt, float* __restrict__ volum
 // the neighbour lanes, y neighbours through LDS, x neighbours from the slab
 // before; a cell that the advection empties takes the mean of its advected
 // neighbours, formed again from the planes (such cells are rare).  Bound by
-// memory: 37 bytes a cell and the halo, where the three passes moved 60 and
-// divided seven times a cell: 115 us at 256x128x128 with their two sums'
-// folds, 63 here.
+// memory: 37 bytes a cell are needed, and 55 move at 256x128x128 at 85% of the
+// copy rate (VALUs 32% busy), where the three passes needed 60 and divided seven
+// times a cell: 115 us there with their two sums' folds, 60 here.
 struct Water {
   float volume, energy;
 };
